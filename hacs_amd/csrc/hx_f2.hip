@@ -23,13 +23,15 @@
 //    the matrix read and written once per panel).
 //  * f2_finish: the pivot rows in pivot order to the top, zero rows below (the non-pivot rows are
 //    zero after the last panel: every row is reduced against every pivot).
-//  * The product: f2_gemm_kernel runs the same tables over B's rows, 64 at a time, accumulating the
-//    output words in registers (one lookup per byte of A's word).
+//  * The product runs on the matrix cores (hx_packed_gemm.hip).  Inside a stream capture, or when that
+//    route's planes do not fit: f2_gemm_kernel, the same tables over B's rows, 64 at a time, accumulating
+//    the output words in registers (one lookup per byte of A's word).
 #include <algorithm>
 #include <cstring>
 #include <vector>
 
 #include "hx_common.h"
+#include "hx_packed_gemm.h"
 
 namespace hx {
 namespace {
@@ -361,6 +363,7 @@ HX_API int hx_f2_gemm(uint32_t m, uint32_t n, uint32_t k, const uint64_t* A, uin
         HX_CHECK(lda >= kw && ldb >= nw && ldc >= nw, "leading dimension below the row's words");
         HX_CHECK(k == 0 || (A != nullptr && B != nullptr), "A or B is NULL");
         if (m == 0 || n == 0) return;
+        if (packed_gemm<2>(m, n, k, A, lda, B, ldb, C, ldc, accumulate != 0, (hipStream_t)s)) return;
         const dim3 grid((nw + F2_WS - 1) / F2_WS, (m + F2_ROWS - 1) / F2_ROWS);
         f2_gemm_kernel<<<grid, F2_UT, 0, (hipStream_t)s>>>(A, lda, B, ldb, C, ldc, m, kw, k, nw, accumulate);
         after_launch("f2_gemm_kernel");

@@ -21,7 +21,9 @@
 //    lookups: per group of 4 slots an LDS table of the 81 combinations of those rows with coefficients
 //    in F_3 (for the workgroup's 4 words, both planes), one lookup per group.
 //  * f3_gather / f3_place: the pivot rows in pivot order to the top, zero rows below.
-//  * The product: f3_gemm_kernel runs the same tables over B's rows, 64 at a time (one word pair of A).
+//  * The product runs on the matrix cores (hx_packed_gemm.hip).  Inside a stream capture, or when that
+//    route's planes do not fit: f3_gemm_kernel, the same tables over B's rows, 64 at a time (one word pair
+//    of A).
 //
 // F_3 arithmetic on 64 entries at once (x = (x1, x2) one-hot, z = x + y): z1 is set where (x, y) is
 // (1, 0), (0, 1) or (2, 2), z2 where it is (2, 0), (0, 2) or (1, 1); -x swaps the planes.
@@ -30,6 +32,7 @@
 #include <vector>
 
 #include "hx_common.h"
+#include "hx_packed_gemm.h"
 
 namespace hx {
 namespace {
@@ -421,6 +424,7 @@ HX_API int hx_f3_gemm(uint32_t m, uint32_t n, uint32_t k, const uint64_t* A, uin
         HX_CHECK(lda >= kw && ldb >= nw && ldc >= nw, "words per plane below the row's words");
         HX_CHECK(k == 0 || (A != nullptr && B != nullptr), "A or B is NULL");
         if (m == 0 || n == 0) return;
+        if (packed_gemm<3>(m, n, k, A, lda, B, ldb, C, ldc, accumulate != 0, (hipStream_t)s)) return;
         const dim3 grid((nw + F3_WS - 1) / F3_WS, (m + F3_ROWS - 1) / F3_ROWS);
         f3_gemm_kernel<<<grid, F3_UT, 0, (hipStream_t)s>>>(A, lda, B, ldb, C, ldc, m, kw, k, nw, accumulate);
         after_launch("f3_gemm_kernel");
