@@ -25,6 +25,7 @@
 // No floating point anywhere; no atomics on results.
 #include "hx_gemm.h"
 #include "hx_limbs.h"
+#include "hx_residue.h"
 
 #include <algorithm>
 #include <numeric>
@@ -1058,12 +1059,6 @@ void limb_attrs() {
 // Imamura, "Ozaki Scheme II: a GEMM-oriented emulation of floating-point matrix multiplication using
 // an integer modular technique", 2025, here for exact residues).
 constexpr int RES_MAXN = 12;
-constexpr uint32_t RES_KMAX = 133144;            // k * 127^2 <= 2^31 - 1
-__host__ __device__ constexpr uint32_t res_modulus(int i) {
-    // pairwise coprime: 3*5*17, 2*127, 11*23, 251, 13*19, then primes
-    return i == 0 ? 255u : i == 1 ? 254u : i == 2 ? 253u : i == 3 ? 251u : i == 4 ? 247u : i == 5 ? 241u
-         : i == 6 ? 239u : i == 7 ? 233u : i == 8 ? 229u : i == 9 ? 227u : i == 10 ? 223u : 211u;
-}
 
 // Per-modulus constants of the operand split, computed on the host (the modulus loop is not unrolled,
 // so constants derived in the kernel would cost runtime divisions): q, the bytes (1, 2^8, 2^16, 2^24)
@@ -1224,20 +1219,8 @@ __global__ __launch_bounds__(256) void res_prep_cols_kernel(PrepArgs a, ResSplit
 // blocks each on 256 x 128 tiles, whose barriers are independent, 6.10 .. 6.18 ms.)
 constexpr int RES_WAVES = 8, RES_STAGES = 3;
 constexpr int RLA = 4, RLB = 2, RTM = RLA * LM, RTN = RLB * 16 * RES_WAVES;
-
-struct ResArgs {
-    const int8_t* A8;            // residue plane i of A at A8 + i * a_plane: Mp rows of Kp bytes
-    const int8_t* B8;            // residue plane i of B at B8 + i * b_plane: Np rows of Kp bytes
-    size_t a_plane, b_plane;
-    uint32_t Kp;
-    uint32_t ntm, ntn;
-    uint8_t* R;                  // product residues of modulus i at R + i * r_plane: Mp rows of ldr bytes
-    size_t r_plane;
-    uint32_t ldr;
-    uint32_t q[RES_MAXN];
-    uint32_t y[RES_MAXN];        // (M / q_i)^-1 mod q_i, the CRT factor of modulus i
-    double invq[RES_MAXN];
-};
+// the small instance: 128 x 128 tiles (2 x 1 blocks per wave)
+constexpr int RSA = 2, RSB = 1;
 
 // B blocks hold 16 * WAVES rows (WAVES / 2 waves across, 32 columns each); A blocks 64 rows (two waves down).
 template <int LA, int LB, int WAVES>
@@ -1717,6 +1700,18 @@ uint32_t residue_choice(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k
     return large && ctx.limbs > 0 && N + 4 <= ctx.limbs * ctx.limbs ? N : 0;
 }
 
+uint32_t residue_side(uint32_t m, uint32_t n, uint32_t N) {
+    const uint64_t tiles = (uint64_t)((m + RTM - 1) / RTM) * ((n + RTN - 1) / RTN) * N;
+    return tiles >= 512 ? RTM : RTM / 2;
+}
+
+void residue_product(const ResArgs& a, uint32_t N, uint32_t side, hipStream_t s) {
+    const dim3 grid(a.ntm * a.ntn, N);
+    if (side == RTM) res_gemm_kernel<RLA, RLB, RES_STAGES, RES_WAVES><<<grid, RES_WAVES * 64, 0, s>>>(a);
+    else res_gemm_kernel<RSA, RSB, RES_STAGES, RES_WAVES><<<grid, RES_WAVES * 64, 0, s>>>(a);
+    after_launch("res_gemm_kernel");
+}
+
 // C op= A B mod p by the residue route with N moduli: residue planes of A and B (res_prep_kernel),
 // one int8 product per modulus (res_gemm_kernel, grid.y = modulus), CRT into C (crt_kernel).
 // ws holds N (Mp Kp + Np Kp + Mp Np) bytes (Mp, Np: m, n rounded up to 256; Kp: k to 64).
@@ -1809,8 +1804,7 @@ void gemm_residue(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32
     }
     ca.pmm = p - (uint32_t)(M % p);
     if (ev0) HX_HIP(hipEventRecord(ev0, s));
-    res_gemm_kernel<RLA, RLB, RES_STAGES, RES_WAVES><<<dim3(ra.ntm * ra.ntn, N), RES_WAVES * 64, 0, s>>>(ra);
-    after_launch("res_gemm_kernel");
+    residue_product(ra, N, RTM, s);
     if (ev1) HX_HIP(hipEventRecord(ev1, s));
 
     ca.R = R;

@@ -1,21 +1,30 @@
 // hx_gemm64.hip -- C op= A B mod p for 64-bit residues, every modulus 2 <= p < 2^64 (the device
 // u64 GEMM of Cuda/cuda_kernels.cu:104-164; the CPU path of record is kernels::gemm<uint64_t>,
-// ModArithmetic/Kernels.h:184).
+// ModArithmetic/Kernels.h:184).  Two routes with the same bytes:
 //
-// Exact sums, one reduction per output: each 64 x 64 -> 128-bit product is formed from four 32 x 32
-// -> 64 partial products and added into a 160-bit accumulator (w0 + w1 2^64 + w2 2^128, exact for
-// K < 2^32), and the sum is reduced once: T = w0 + w1 2^64 + w2 2^128 mod p.  For odd p by Montgomery
-// (R = 2^64): REDC(w1 mod p, w0) = (w1 2^64 + w0) R^-1, multiplied by R^2 mod p and reduced again;
-// the w2 term is w2 (2^128 mod p).  For even p (no Montgomery inverse) by binary long division of
-// the 128-bit words.  No floating point; the bytes equal the oracle's exact integer arithmetic.
+//  * The residue route (gemm64_residue; k >= 40, outside a stream capture): the operands modulo up to 19
+//    pairwise coprime bytes, one int8 MFMA product per modulus (res_gemm_kernel, hx_gemm.hip), and the CRT
+//    back to 64 bits.  2048^3 mod 2^61 - 1: 17 products, 0.300 ms = 2.9e13 multiply-adds/s for the whole
+//    call, against 4.19 ms (2.05e12) on the plain kernel; 512^3 0.049 against 0.364 ms.  Bound by the int8
+//    products and the HBM passes over the residue planes (17 bytes per operand entry and per output).
 //
-// Tiling: 64 x 64 outputs per 256-thread workgroup, 4 x 4 per thread (rows ty + 16 i, columns
-// tx + 16 j), K staged by 16 through a double-buffered LDS tile (A transposed, padded rows), the
-// next stage's global loads issued before the current stage's products.  VALU-bound: ~14 integer
-// operations per mod-p multiply-add.
+//  * The plain kernel (gemm64_kernel; everything else): each 64 x 64 -> 128-bit product is formed from four
+//    32 x 32 -> 64 partial products and added into a 160-bit accumulator (w0 + w1 2^64 + w2 2^128, exact for
+//    K < 2^32), and the sum is reduced once: T = w0 + w1 2^64 + w2 2^128 mod p.  For odd p by Montgomery
+//    (R = 2^64): REDC(w1 mod p, w0) = (w1 2^64 + w0) R^-1, multiplied by R^2 mod p and reduced again;
+//    the w2 term is w2 (2^128 mod p).  For even p (no Montgomery inverse) by binary long division of
+//    the 128-bit words.  Tiling: 64 x 64 outputs per 256-thread workgroup, 4 x 4 per thread (rows ty + 16 i,
+//    columns tx + 16 j), K staged by 16 through a double-buffered LDS tile (A transposed, padded rows), the
+//    next stage's global loads issued before the current stage's products.  VALU-bound: ~14 integer
+//    operations per mod-p multiply-add.
+//
+// The bytes of both equal the oracle's exact integer arithmetic.
+#include <algorithm>
+#include <cmath>
 #include <cstring>
 
 #include "hx_common.h"
+#include "hx_residue.h"
 
 namespace hx {
 namespace {
@@ -174,6 +183,247 @@ __global__ __launch_bounds__(G64_T) void gemm64_kernel(Gemm64Args g, Mod64 M) {
 
 Mod64 mod64_of(const hx_modctx64& c) { return Mod64{c.p, c.ninv, c.r2, c.two64, (int)(c.p & 1u)}; }
 
+// ---- the residue route ------------------------------------------------------------------------
+// The product of balanced operands (|a_b| <= p / 2) modulo N pairwise coprime moduli q_i <= 255, one int8
+// MFMA product each, and the CRT back to the residue mod p: hx_gemm.hip's route with the operands and the
+// recombination on 64-bit words.  N is the least count with prod q_i > 2.05 k (p/2)^2 (at most 19).
+
+struct Split64 {
+    uint32_t nmod;
+    uint32_t q[RES_MAXQ], tlo[RES_MAXQ], thi[RES_MAXQ];   // bytes 2^(8j) mod q, j = 0 .. 3 and 4 .. 7
+    uint32_t kq[RES_MAXQ];                                // q - (2^63 mod q)
+    float iq[RES_MAXQ];
+};
+
+struct Prep64 {
+    const uint64_t* src;         // entry (row r, k c) at src[r s_r + c s_c]
+    int64_t s_r, s_c;
+    uint32_t R, K;               // rows and k of the operand (past them: zero)
+    uint32_t Kp;                 // bytes per output row
+    int8_t* out;
+    size_t plane;
+    uint64_t p;
+};
+
+// Residue planes of one 32-row x 128-k tile.  The entries a_b + 2^63 go through LDS as T[k][row] (row XOR 4 times
+// the 16-k chunk: the strided reads below spread over the banks), loaded along whichever index is contiguous
+// in memory; each thread then turns 16 k of one row into 16 bytes per plane, 128 contiguous bytes per row.
+// With w = a_b + 2^63 (a word of 8 bytes w_j), t = sum_j w_j (2^(8j) mod q) + q - (2^63 mod q) is congruent to
+// a_b and below 8 * 255 * 254 + 255 < 2^19, so fp32 holds it and t fl(1/q) + 1/2 is within 2^19 / 173 * 2^-22
+// < 8e-4 of t / q + 1/2, whose fractional part is at least 1 / (2q) > 0.0019 from an integer for odd q:
+// the truncation is round(t / q).  (q = 254: a tie may go either way, +-127 are the same residue.)
+__global__ __launch_bounds__(256) void prep64_kernel(Prep64 a, Split64 c) {
+    __shared__ uint64_t T[128][33];
+    const uint32_t r0 = blockIdx.x * 32, c0 = blockIdx.y * 128;
+    const int tid = threadIdx.x;
+    const uint64_t p = a.p, half = p / 2;
+    auto put = [&](uint32_t r, uint32_t cc) {
+        const uint32_t row = r0 + r, k = c0 + cc;
+        const uint64_t v = (row < a.R && k < a.K) ? a.src[(int64_t)row * a.s_r + (int64_t)k * a.s_c] : 0u;
+        T[cc][r ^ (((cc >> 4) & 7) << 2)] = (v > half ? v - p : v) + 0x8000000000000000ull;
+    };
+    if (a.s_c == 1) {
+#pragma unroll 8
+        for (int t = 0; t < 16; ++t) put((tid >> 7) + 2 * t, tid & 127);
+    } else {
+#pragma unroll 8
+        for (int t = 0; t < 16; ++t) put(tid & 31, (tid >> 5) + 8 * t);
+    }
+    __syncthreads();
+    const uint32_t r = tid >> 3, qd = tid & 7;
+    if (c0 + 16 * qd >= a.Kp) return;
+    uint64_t w[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) w[j] = T[16 * qd + j][r ^ (qd << 2)];
+    int8_t* out = a.out + (size_t)(r0 + r) * a.Kp + c0 + 16 * qd;
+    for (uint32_t i = 0; i < c.nmod; ++i) {
+        const uint32_t Q = c.q[i], TL = c.tlo[i], TH = c.thi[i], KQ = c.kq[i];
+        const float IQ = c.iq[i];
+        uint32_t o[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const uint32_t t = __builtin_amdgcn_udot4((uint32_t)(w[j] >> 32), TH,
+                                                      __builtin_amdgcn_udot4((uint32_t)w[j], TL, KQ, false), false);
+            const uint32_t qt = (uint32_t)fmaf((float)t, IQ, 0.5f);
+            o[j / 4] |= ((t - __umul24(qt, Q)) & 0xffu) << (8 * (j % 4));
+        }
+        *(uint4*)(out + (size_t)i * a.plane) = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+}
+
+// x mod p from the N product residues s_i = x (M / q_i)^-1 mod q_i (M = prod q_i): sum_i s_i M / q_i = x + T M with
+// T = round(sum_i s_i / q_i), so x = sum_i s_i (M / q_i mod p) - T (M mod p).  The 64-bit constants are split
+// in 16-bit digits (24-bit products, digit sums below 19 * 254 * 2^16 < 2^29), the fraction sum is in fixed
+// point with f_i = round(2^20 / q_i) (error <= 19 * 254 / 2 units of 2^-20 < 0.0024, inside the 0.5 - 0.488
+// margin), and the total, below 2^78, is reduced once.
+struct Crt64 {
+    const uint8_t* R;
+    size_t r_plane;
+    uint32_t ldr;
+    uint32_t nmod;
+    uint16_t c[RES_MAXQ][4];     // (M / q_i) mod p, digits of 16 bits
+    uint32_t f[RES_MAXQ];
+    uint64_t pmm;                // p - (M mod p)
+    uint32_t m, n;
+    uint64_t* C;
+    int64_t crs, ccs;
+    int op;
+};
+
+__global__ __launch_bounds__(256) void crt64_kernel(Crt64 a, Mod64 M) {
+    const uint32_t col0 = (blockIdx.y * 64 + (threadIdx.x & 63)) * 4;
+    const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= a.m || col0 >= a.n) return;
+    uint32_t d[4][4] = {}, fr[4] = {};
+    const uint8_t* src = a.R + (size_t)row * a.ldr + col0;
+#pragma unroll 4
+    for (uint32_t i = 0; i < a.nmod; ++i) {
+        const uint32_t w = *(const uint32_t*)(src + (size_t)i * a.r_plane);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const uint32_t sb = (w >> (8 * b)) & 0xffu;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d[b][e] += __umul24(sb, a.c[i][e]);
+            fr[b] += __umul24(sb, a.f[i]);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const uint32_t col = col0 + b;
+        if (col >= a.n) break;
+        const uint32_t T = (fr[b] + (1u << 19)) >> 20;
+        unsigned __int128 x = (unsigned __int128)T * a.pmm;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x += (unsigned __int128)d[b][e] << (16 * e);
+        const uint64_t r = reduce160((uint64_t)x, (uint64_t)(x >> 64), 0, M);
+        uint64_t* c = a.C + (int64_t)row * a.crs + (int64_t)col * a.ccs;
+        *c = a.op == HX_OP_SET ? r : a.op == HX_OP_ADD ? add64m(*c, r, M.p) : sub64m(*c, r, M.p);
+    }
+}
+
+// The least N with prod_{i<N} q_i > 2.05 k (p/2)^2 for 1 <= k <= RES_KMAX (the logarithms' rounding errors are
+// far below the 1e-9 kept in hand; 19 moduli reach 2^147.6, the bound stays below 2^145.1).
+uint32_t moduli64(uint64_t p, uint32_t k) {
+    const double need = std::log2(2.05) + std::log2((double)k) + 2.0 * std::log2((double)(p / 2)) + 1e-9;
+    double have = 0.0;
+    for (int i = 0; i < RES_MAXQ; ++i) {
+        have += std::log2((double)res_modulus(i));
+        if (have > need) return (uint32_t)i + 1;
+    }
+    return 0;
+}
+
+// Shallower products stay on the plain kernel: the splits and the CRT cost the same at any k, the plain kernel's
+// time grows with k (mod 2^61 - 1, us plain / residue: 2048 x 2048 x 16 59 / 109, x 64 180 / 122; 32^3 27 / 33,
+// 64^3 56 / 33; 512^3 364 / 50, 2048^3 4190 / 300).
+constexpr uint32_t RES64_MIN_K = 40;
+constexpr size_t RES64_WS = (size_t)4 << 30;      // bytes of planes held at a time; C runs in blocks that fit
+
+// C op= A B by the residue route; false, with nothing launched, where it does not apply.
+bool gemm64_residue(const hx_modctx64& ctx, const Gemm64Args& g, hipStream_t s) {
+    if (g.k == 0 || stream_capturing(s)) return false;
+    auto up = [](uint64_t x, uint64_t a) { return (x + a - 1) / a * a; };
+    const uint64_t p = ctx.p;
+    const uint32_t kc = std::min<uint32_t>(g.k, RES_KMAX / 64 * 64), N = moduli64(p, kc);
+    if (N == 0) return false;
+    const uint32_t side = residue_side(g.m, g.n, N);
+    const uint64_t Kp0 = up(kc, 64);
+    uint64_t mb = up(g.m, side), nb = up(g.n, side);
+    auto bytes = [&] { return N * (mb * Kp0 + nb * Kp0 + mb * nb); };
+    while (bytes() > RES64_WS && (mb > side || nb > side)) (mb >= nb ? mb : nb) = up((mb >= nb ? mb : nb) / 2, side);
+    char* ws;
+    try {
+        ws = (char*)stream_scratch(s, SCRATCH_LIMB, bytes());
+    } catch (const Error& e) {
+        if (e.code != HX_E_NOMEM) throw;
+        return false;
+    }
+    if (ws == nullptr) return false;
+
+    Split64 sp{};
+    ResArgs ra{};
+    Crt64 ca{};
+    sp.nmod = ca.nmod = N;
+    // M / q_i mod p from prefix and suffix products (also M / q_i mod q_i, inverted by Euclid)
+    uint64_t suf[RES_MAXQ + 1], pre = 1 % p;
+    suf[N] = 1 % p;
+    for (uint32_t i = N; i-- > 0;) suf[i] = (uint64_t)((unsigned __int128)suf[i + 1] * res_modulus((int)i) % p);
+    for (uint32_t i = 0; i < N; ++i) {
+        const uint32_t q = res_modulus((int)i);
+        const uint64_t ci = (uint64_t)((unsigned __int128)pre * suf[i + 1] % p);
+        pre = (uint64_t)((unsigned __int128)pre * q % p);
+        uint32_t mq = 1;
+        for (uint32_t j = 0; j < N; ++j)
+            if (j != i) mq = mq * res_modulus((int)j) % q;
+        int32_t r0 = (int32_t)q, r1 = (int32_t)mq, t0 = 0, t1 = 1;
+        while (r1 != 0) {
+            const int32_t d = r0 / r1, r2 = r0 - d * r1, t2 = t0 - d * t1;
+            r0 = r1, r1 = r2, t0 = t1, t1 = t2;
+        }
+        HX_CHECK(r0 == 1, "residue route: moduli not coprime");
+        const uint32_t y = (uint32_t)(t0 < 0 ? t0 + (int32_t)q : t0);
+        sp.q[i] = ra.q[i] = q;
+        uint32_t w8 = 1, wt[8];
+        for (int j = 0; j < 8; ++j) {
+            wt[j] = w8;
+            w8 = w8 * 256 % q;
+        }
+        sp.tlo[i] = wt[0] | wt[1] << 8 | wt[2] << 16 | wt[3] << 24;
+        sp.thi[i] = wt[4] | wt[5] << 8 | wt[6] << 16 | wt[7] << 24;
+        sp.kq[i] = q - (uint32_t)(0x8000000000000000ull % q);
+        sp.iq[i] = 1.0f / (float)q;
+        ra.y[i] = y;
+        ra.invq[i] = 1.0 / (double)q;
+        for (int e = 0; e < 4; ++e) ca.c[i][e] = (uint16_t)(ci >> (16 * e));
+        ca.f[i] = ((1u << 20) + q / 2) / q;
+    }
+    ca.pmm = p - pre;
+    const Mod64 M = mod64_of(ctx);
+
+    auto split = [&](const uint64_t* src, int64_t s_r, int64_t s_c, uint32_t R, uint32_t rows, uint32_t K, uint32_t Kp,
+                     int8_t* out, const char* what) {
+        const Prep64 a{src, s_r, s_c, R, K, Kp, out, (size_t)rows * Kp, p};
+        prep64_kernel<<<dim3(rows / 32, (Kp + 127) / 128), 256, 0, s>>>(a, sp);
+        after_launch(what);
+    };
+    for (uint64_t k0 = 0; k0 < g.k; k0 += kc) {
+        const uint32_t K = (uint32_t)std::min<uint64_t>(kc, g.k - k0), Kp = (uint32_t)up(K, 64);
+        for (uint64_t j0 = 0; j0 < g.n; j0 += nb) {
+            const uint32_t n = (uint32_t)std::min<uint64_t>(nb, g.n - j0), Np = (uint32_t)up(n, side);
+            int8_t* B8 = (int8_t*)ws;
+            split(g.B + (int64_t)j0 * g.bcs + (int64_t)k0 * g.brs, g.bcs, g.brs, n, Np, K, Kp, B8, "prep64(B)");
+            for (uint64_t i0 = 0; i0 < g.m; i0 += mb) {
+                const uint32_t m = (uint32_t)std::min<uint64_t>(mb, g.m - i0), Mp = (uint32_t)up(m, side);
+                int8_t* A8 = B8 + (size_t)N * Np * Kp;
+                split(g.A + (int64_t)i0 * g.ars + (int64_t)k0 * g.acs, g.ars, g.acs, m, Mp, K, Kp, A8, "prep64(A)");
+                ra.A8 = A8;
+                ra.B8 = B8;
+                ra.a_plane = (size_t)Mp * Kp;
+                ra.b_plane = (size_t)Np * Kp;
+                ra.Kp = Kp;
+                ra.ntm = Mp / side;
+                ra.ntn = Np / side;
+                ra.R = (uint8_t*)(A8 + (size_t)N * Mp * Kp);
+                ra.r_plane = (size_t)Mp * Np;
+                ra.ldr = Np;
+                residue_product(ra, N, side, s);
+                ca.R = ra.R;
+                ca.r_plane = ra.r_plane;
+                ca.ldr = Np;
+                ca.m = m;
+                ca.n = n;
+                ca.C = g.C + (int64_t)i0 * g.crs + (int64_t)j0 * g.ccs;
+                ca.crs = g.crs;
+                ca.ccs = g.ccs;
+                ca.op = k0 == 0 ? g.op : g.op == HX_OP_SUB ? HX_OP_SUB : HX_OP_ADD;
+                crt64_kernel<<<dim3((m + 3) / 4, (n + 255) / 256), 256, 0, s>>>(ca, M);
+                after_launch("crt64_kernel");
+            }
+        }
+    }
+    return true;
+}
+
 }  // namespace
 }  // namespace hx
 
@@ -209,6 +459,10 @@ HX_API int hx_gemm_u64(const hx_modctx64* ctx, hx_view A, hx_view B, hx_view C, 
         if (C.rows == 0 || C.cols == 0) return;
         Gemm64Args g{C.rows, C.cols, A.cols, (const uint64_t*)A.base, A.rs, A.cs, (const uint64_t*)B.base, B.rs, B.cs,
                      (uint64_t*)C.base, C.rs, C.cs, op};
+        if (g.k >= RES64_MIN_K && gemm64_residue(*ctx, g, (hipStream_t)s)) {
+            stat_add(ST_GEMMS, 1);
+            return;
+        }
         const uint32_t tiles = ((g.m + G64_TILE - 1) / G64_TILE) * ((g.n + G64_TILE - 1) / G64_TILE);
         gemm64_kernel<<<tiles, G64_T, 0, (hipStream_t)s>>>(g, mod64_of(*ctx));
         after_launch("gemm64_kernel");

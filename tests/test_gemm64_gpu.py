@@ -65,3 +65,71 @@ def test_gemm_u64_worst_case_carries(hx_gpu, O, p):
     E.gemm_u64(ctx, dA, dB, dC, 0)
     torch.cuda.synchronize()
     assert (E.from_device64(dC) == np.uint64(K % p)).all()
+
+
+@pytest.mark.parametrize("p", [2305843009213693951, 18446744073709551557, (1 << 64) - 2, 4294967311])
+@pytest.mark.parametrize("shape", [(128, 128, 64), (129, 127, 65), (255, 300, 129), (1, 700, 1000), (700, 1, 1000),
+                                   (1400, 1500, 70)])                              # the last: 256 x 256 tiles
+def test_gemm_u64_residue_route(hx_gpu, O, p, shape):
+    """The matrix-core route at the edges of its tiles, row- and column-major operands, every op."""
+    from hacs_amd import engine as E
+    ctx = E.ModCtx64(p)
+    m, n, k = shape
+    rng = np.random.default_rng((p ^ (m * 1000003 + n * 1009 + k)) & 0xFFFFFFFF)
+    A, B, C0 = _draw(rng, p, (m, k)), _draw(rng, p, (k, n)), _draw(rng, p, (m, n))
+    A[0, :] = p - 1
+    B[:, 0] = p // 2
+    want = [O.gemm_u64(p, A, B, C0, op, 16) for op in (0, 1, 2)]
+    At = E.to_device64(np.ascontiguousarray(A.T)).t()
+    Bt = E.to_device64(np.ascontiguousarray(B.T)).t()
+    for dA, dB, op in ((E.to_device64(A), E.to_device64(B), 0), (At, Bt, 1), (At, E.to_device64(B), 2)):
+        dC = E.to_device64(C0)
+        E.gemm_u64(ctx, dA, dB, dC, op)
+        torch.cuda.synchronize()
+        assert np.array_equal(E.from_device64(dC), want[op]), f"op {op}"
+
+
+@pytest.mark.parametrize("p", [18446744073709551557, 2305843009213693951])
+@pytest.mark.parametrize("m,n,k", [(40, 200, 133056 + 77), (1500, 300, 133000)])
+def test_gemm_u64_residue_chunks(hx_gpu, p, m, n, k):
+    """K past one chunk of int32 sums; C in blocks (planes past the workspace bound).  B holds three entries
+    per column, so every result is three products."""
+    from hacs_amd import engine as E
+    rng = np.random.default_rng(m + n)
+    dA = torch.randint(0, 1 << 62, (m, k), device="cuda", dtype=torch.int64) % (p >> 3)
+    rows = np.stack([rng.choice(k, 3, replace=False) for _ in range(n)])
+    coef = _draw(rng, p, (n, 3))
+    B = np.zeros((k, n), np.uint64)
+    for e in range(3):
+        B[rows[:, e], np.arange(n)] = coef[:, e]
+    cols = E.from_device64(dA[:, torch.from_numpy(rows.reshape(-1)).cuda()]).reshape(m, n, 3)
+    want = np.array([sum(int(cols[i, j, e]) * int(coef[j, e]) for e in range(3)) % p
+                     for i in range(m) for j in range(n)], np.uint64).reshape(m, n)
+    dC = torch.zeros((m, n), dtype=torch.int64, device="cuda")
+    E.gemm_u64(E.ModCtx64(p), dA, E.to_device64(B), dC, 1)
+    torch.cuda.synchronize()
+    assert np.array_equal(E.from_device64(dC), want)
+
+
+def test_gemm_u64_captured(hx_gpu, O):
+    """A captured product (the plain kernel: no library scratch in a graph) replayed on new operands."""
+    from hacs_amd import engine as E
+    p, m, n, k = 2305843009213693951, 150, 140, 160
+    ctx = E.ModCtx64(p)
+    rng = np.random.default_rng(3)
+    dA, dB = (torch.zeros(s, dtype=torch.int64, device="cuda") for s in ((m, k), (k, n)))
+    dC = torch.zeros((m, n), dtype=torch.int64, device="cuda")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        E.gemm_u64(ctx, dA, dB, dC)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        E.gemm_u64(ctx, dA, dB, dC)
+    for _ in range(3):
+        A, B = _draw(rng, p, (m, k)), _draw(rng, p, (k, n))
+        dA.copy_(E.to_device64(A))
+        dB.copy_(E.to_device64(B))
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(E.from_device64(dC), O.gemm_u64(p, A, B, np.zeros((m, n), np.uint64), 0, 16))
