@@ -108,7 +108,8 @@ void arena_free(void* p);
 bool stream_capturing(hipStream_t s);
 // Library-owned scratch of at least `bytes`, private to stream s and one purpose (below); grows
 // (after waiting for s) but never shrinks; nullptr when it would have to grow inside a capture.
-enum ScratchPurpose { SCRATCH_LIMB = 0, SCRATCH_MLP = 1, SCRATCH_RREF = 2, SCRATCH_SPLIT = 3, SCRATCH_PACKED = 4 };
+enum ScratchPurpose { SCRATCH_LIMB = 0, SCRATCH_MLP = 1, SCRATCH_RREF = 2, SCRATCH_SPLIT = 3, SCRATCH_PACKED = 4,
+                      SCRATCH_U64 = 5 };
 void* stream_scratch(hipStream_t s, int purpose, size_t bytes);
 void stream_scratch_release(hipStream_t s);
 // A rows x width-byte block between pageable host memory and the device (either direction, pitches in

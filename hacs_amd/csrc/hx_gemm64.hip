@@ -4,7 +4,7 @@
 //
 //  * The residue route (gemm64_residue; k >= 40, outside a stream capture): the operands modulo up to 19
 //    pairwise coprime bytes, one int8 MFMA product per modulus (res_gemm_kernel, hx_gemm.hip), and the CRT
-//    back to 64 bits.  2048^3 mod 2^61 - 1: 17 products, 0.300 ms = 2.9e13 multiply-adds/s for the whole
+//    back to 64 bits.  2048^3 mod 2^61 - 1: 17 products, 0.269 ms = 3.2e13 multiply-adds/s for the whole
 //    call, against 4.19 ms (2.05e12) on the plain kernel; 512^3 0.049 against 0.364 ms.  Bound by the int8
 //    products and the HBM passes over the residue planes (17 bytes per operand entry and per output).
 //
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256) void prep64_kernel(Prep64 a, Split64 c) {
 struct Crt64 {
     const uint8_t* R;
     size_t r_plane;
-    uint32_t ldr;
+    ResBlocks g;
     uint32_t nmod;
     uint16_t c[RES_MAXQ][4];     // (M / q_i) mod p, digits of 16 bits
     uint32_t f[RES_MAXQ];
@@ -270,34 +270,40 @@ struct Crt64 {
     int op;
 };
 
+// One 32 x 32 block per two waves: eight outputs per thread, planes read 8 bytes per lane.
 __global__ __launch_bounds__(256) void crt64_kernel(Crt64 a, Mod64 M) {
-    const uint32_t col0 = (blockIdx.y * 64 + (threadIdx.x & 63)) * 4;
-    const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= a.m || col0 >= a.n) return;
-    uint32_t d[4][4] = {}, fr[4] = {};
-    const uint8_t* src = a.R + (size_t)row * a.ldr + col0;
-#pragma unroll 4
+    const uint32_t blk = blockIdx.x * 2 + (threadIdx.x >> 7), lane = threadIdx.x & 63, h = (threadIdx.x >> 6) & 1;
+    uint32_t row0, col;
+    res_block(a.g, blk, row0, col);
+    if (row0 >= a.m || col >= a.n) return;
+    row0 += 16 * h + 4 * (lane >> 5);
+    col += lane & 31;
+    uint32_t d[8][4] = {}, fr[8] = {};
+    const uint8_t* src = a.R + (size_t)blk * 1024 + lane * 16 + 8 * h;
+#pragma unroll 2
     for (uint32_t i = 0; i < a.nmod; ++i) {
-        const uint32_t w = *(const uint32_t*)(src + (size_t)i * a.r_plane);
+        const uint2 v = *(const uint2*)(src + (size_t)i * a.r_plane);
+        const uint32_t w[2] = {v.x, v.y};
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const uint32_t sb = (w >> (8 * b)) & 0xffu;
+        for (int r = 0; r < 8; ++r) {
+            const uint32_t sb = (w[r / 4] >> (8 * (r % 4))) & 0xffu;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) d[b][e] += __umul24(sb, a.c[i][e]);
-            fr[b] += __umul24(sb, a.f[i]);
+            for (int e = 0; e < 4; ++e) d[r][e] += __umul24(sb, a.c[i][e]);
+            fr[r] += __umul24(sb, a.f[i]);
         }
     }
+    if (col >= a.n) return;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const uint32_t col = col0 + b;
-        if (col >= a.n) break;
-        const uint32_t T = (fr[b] + (1u << 19)) >> 20;
+    for (int r = 0; r < 8; ++r) {
+        const uint32_t row = row0 + (r / 4) * 8 + r % 4;
+        if (row >= a.m) continue;
+        const uint32_t T = (fr[r] + (1u << 19)) >> 20;
         unsigned __int128 x = (unsigned __int128)T * a.pmm;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x += (unsigned __int128)d[b][e] << (16 * e);
-        const uint64_t r = reduce160((uint64_t)x, (uint64_t)(x >> 64), 0, M);
+        for (int e = 0; e < 4; ++e) x += (unsigned __int128)d[r][e] << (16 * e);
+        const uint64_t res = reduce160((uint64_t)x, (uint64_t)(x >> 64), 0, M);
         uint64_t* c = a.C + (int64_t)row * a.crs + (int64_t)col * a.ccs;
-        *c = a.op == HX_OP_SET ? r : a.op == HX_OP_ADD ? add64m(*c, r, M.p) : sub64m(*c, r, M.p);
+        *c = a.op == HX_OP_SET ? res : a.op == HX_OP_ADD ? add64m(*c, res, M.p) : sub64m(*c, res, M.p);
     }
 }
 
@@ -315,7 +321,7 @@ uint32_t moduli64(uint64_t p, uint32_t k) {
 
 // Shallower products stay on the plain kernel: the splits and the CRT cost the same at any k, the plain kernel's
 // time grows with k (mod 2^61 - 1, us plain / residue: 2048 x 2048 x 16 59 / 109, x 64 180 / 122; 32^3 27 / 33,
-// 64^3 56 / 33; 512^3 364 / 50, 2048^3 4190 / 300).
+// 64^3 56 / 32; 512^3 364 / 49, 2048^3 4190 / 269).
 constexpr uint32_t RES64_MIN_K = 40;
 constexpr size_t RES64_WS = (size_t)4 << 30;      // bytes of planes held at a time; C runs in blocks that fit
 
@@ -333,7 +339,7 @@ bool gemm64_residue(const hx_modctx64& ctx, const Gemm64Args& g, hipStream_t s) 
     while (bytes() > RES64_WS && (mb > side || nb > side)) (mb >= nb ? mb : nb) = up((mb >= nb ? mb : nb) / 2, side);
     char* ws;
     try {
-        ws = (char*)stream_scratch(s, SCRATCH_LIMB, bytes());
+        ws = (char*)stream_scratch(s, SCRATCH_U64, bytes());
     } catch (const Error& e) {
         if (e.code != HX_E_NOMEM) throw;
         return false;
@@ -362,7 +368,8 @@ bool gemm64_residue(const hx_modctx64& ctx, const Gemm64Args& g, hipStream_t s) 
         }
         HX_CHECK(r0 == 1, "residue route: moduli not coprime");
         const uint32_t y = (uint32_t)(t0 < 0 ? t0 + (int32_t)q : t0);
-        sp.q[i] = ra.q[i] = q;
+        sp.q[i] = q;
+        res_modulus_consts(ra, i, q, y);
         uint32_t w8 = 1, wt[8];
         for (int j = 0; j < 8; ++j) {
             wt[j] = w8;
@@ -372,8 +379,6 @@ bool gemm64_residue(const hx_modctx64& ctx, const Gemm64Args& g, hipStream_t s) 
         sp.thi[i] = wt[4] | wt[5] << 8 | wt[6] << 16 | wt[7] << 24;
         sp.kq[i] = q - (uint32_t)(0x8000000000000000ull % q);
         sp.iq[i] = 1.0f / (float)q;
-        ra.y[i] = y;
-        ra.invq[i] = 1.0 / (double)q;
         for (int e = 0; e < 4; ++e) ca.c[i][e] = (uint16_t)(ci >> (16 * e));
         ca.f[i] = ((1u << 20) + q / 2) / q;
     }
@@ -405,18 +410,17 @@ bool gemm64_residue(const hx_modctx64& ctx, const Gemm64Args& g, hipStream_t s) 
                 ra.ntn = Np / side;
                 ra.R = (uint8_t*)(A8 + (size_t)N * Mp * Kp);
                 ra.r_plane = (size_t)Mp * Np;
-                ra.ldr = Np;
                 residue_product(ra, N, side, s);
                 ca.R = ra.R;
                 ca.r_plane = ra.r_plane;
-                ca.ldr = Np;
+                ca.g = ResBlocks{side, ra.ntn};
                 ca.m = m;
                 ca.n = n;
                 ca.C = g.C + (int64_t)i0 * g.crs + (int64_t)j0 * g.ccs;
                 ca.crs = g.crs;
                 ca.ccs = g.ccs;
                 ca.op = k0 == 0 ? g.op : g.op == HX_OP_SUB ? HX_OP_SUB : HX_OP_ADD;
-                crt64_kernel<<<dim3((m + 3) / 4, (n + 255) / 256), 256, 0, s>>>(ca, M);
+                crt64_kernel<<<(uint32_t)(ra.r_plane / 2048), 256, 0, s>>>(ca, M);
                 after_launch("crt64_kernel");
             }
         }

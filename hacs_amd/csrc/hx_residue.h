@@ -19,13 +19,35 @@ struct ResArgs {
     size_t a_plane, b_plane;
     uint32_t Kp;
     uint32_t ntm, ntn;
-    uint8_t* R;                  // product residues of modulus i at R + i * r_plane: Mp rows of ldr bytes
-    size_t r_plane;
-    uint32_t ldr;
+    uint8_t* R;                  // product residues of modulus i at R + i * r_plane (res_block's order)
+    size_t r_plane;              // ntm ntn side^2 bytes
     uint32_t q[RES_MAXQ];
-    uint32_t y[RES_MAXQ];        // (M / q_i)^-1 mod q_i, the CRT factor of modulus i
-    double invq[RES_MAXQ];
+    uint32_t tpack[RES_MAXQ];    // bytes (y 2^(8j)) mod q, j = 0 .. 3, y = (M / q_i)^-1 mod q_i (the CRT's factor)
+    uint32_t kq[RES_MAXQ];       // q - (y 2^31 mod q)
+    float iq[RES_MAXQ];
 };
+
+// The product residues of a plane lie as the MFMA accumulators do: 1 KB per 32 x 32 block, 16 bytes per lane
+// (byte r: row (r / 4) 8 + 4 (lane / 32) + r % 4, column lane % 32), so the product kernel stores and the CRT
+// kernels load 16 bytes per lane.  Blocks of a tile: 64-row strip, 128-column strip, then the upper / lower 32
+// rows and the four 32-column blocks of the 64 x 128 piece; tiles row by row.
+struct ResBlocks {
+    uint32_t side, ntn;          // tile side (256 or 128), tiles per row
+};
+__device__ __forceinline__ void res_block(const ResBlocks& g, uint32_t b, uint32_t& row, uint32_t& col) {
+    const uint32_t per = g.side * g.side / 1024, tile = b / per, in = b % per;
+    const uint32_t lb = g.side / 128, s = in / 8 / lb, t = in / 8 % lb;
+    row = tile / g.ntn * g.side + 64 * s + 32 * ((in >> 2) & 1);
+    col = tile % g.ntn * g.side + 128 * t + 32 * (in & 3);
+}
+
+// Modulus i's constants of the product's epilogue (q, y < 256).
+inline void res_modulus_consts(ResArgs& a, uint32_t i, uint32_t q, uint32_t y) {
+    a.q[i] = q;
+    a.tpack[i] = y % q | y * 256u % q << 8 | (uint32_t)(y * 65536ull % q) << 16 | (uint32_t)(y * 16777216ull % q) << 24;
+    a.kq[i] = q - (uint32_t)(y * 0x80000000ull % q);
+    a.iq[i] = 1.0f / (float)q;
+}
 
 // The side of the square output tiles of an N-moduli product: Mp and Np are multiples of it.
 uint32_t residue_side(uint32_t m, uint32_t n, uint32_t N);
