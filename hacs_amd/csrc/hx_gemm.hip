@@ -1106,7 +1106,7 @@ __global__ __launch_bounds__(256) void res_prep_kernel(PrepArgs a, ResSplit c) {
         const uint32_t v = T[r][16 * qd + j];
         w[j] = (v > a.half ? v - p : v) + 0x80000000u;      // a_b + 2^31, a_b in [-p/2, p/2]
     }
-    int8_t* out = a.out + (size_t)(r0 + r) * a.Kp + c0 + 16 * qd;
+    int8_t* out = a.out + res_chunk(r0 + r, c0 / 16 + qd, a.Kp);
 #pragma unroll
     for (int i = 0; i < RES_MAXN; ++i) {
         if (i >= (int)c.nmod) break;
@@ -1120,42 +1120,43 @@ __global__ __launch_bounds__(256) void res_prep_kernel(PrepArgs a, ResSplit c) {
     }
 }
 
-// Residue planes of a row-major operand whose rows are 16-byte aligned (no gathers, host-side sizes):
-// one wave per row and 1024 k, lane-contiguous 16-byte loads (four entries per lane and instruction,
-// 1 KB per wave instruction) and one dword per lane and plane for every four entries (256 contiguous
-// bytes per wave store), no LDS.  Entries past K and rows past R are written as zero up to Kp and the
-// plane's last row.  Grid: (ceil(Kp / 1024), rows / 4), 256 threads.
+// Residue planes of a row-major operand whose rows are 16-byte aligned (no gathers, host-side sizes): each
+// thread turns 16 consecutive k of one row (four 16-byte loads) into one 16-byte chunk per plane, no LDS.  A
+// wave takes 8 rows x 128 k: 512 contiguous bytes read per row, 128 contiguous bytes (eight rows) written per
+// 16 k and plane.  Entries past K and rows past R are written as zero up to Kp and the plane's last row.
+// Grid: (ceil(Kp / 128), rows / 32), 256 threads.
 __global__ __launch_bounds__(256) void res_prep_rows_kernel(PrepArgs a, ResSplit c) {
-    const uint32_t row = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t row = blockIdx.y * 32 + (threadIdx.x >> 3), k16 = blockIdx.x * 8 + (threadIdx.x & 7), k0 = 16 * k16;
+    if (k0 >= a.Kp) return;
     const uint32_t p = a.p;
-    const uint32_t* src = a.src + (size_t)row * a.s_r;
-    int8_t* out = a.out + (size_t)row * a.Kp;
+    const uint32_t* src = a.src + (size_t)row * a.s_r + k0;
+    uint32_t w[16];
+    if (row < a.R && k0 + 16 <= a.K) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t k4 = blockIdx.x * 1024 + (uint32_t)j * 256 + lane * 4;
-        if (k4 >= a.Kp) break;
-        uint32_t v[4] = {0, 0, 0, 0};
-        if (row < a.R) {
-            if (k4 + 3 < a.K) {
-                const uint4 q4 = *(const uint4*)(src + k4);
-                v[0] = q4.x;
-                v[1] = q4.y;
-                v[2] = q4.z;
-                v[3] = q4.w;
-            } else {
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    if (k4 + b < a.K) v[b] = src[k4 + b];
-            }
+        for (int j = 0; j < 4; ++j) {
+            const uint4 q4 = *(const uint4*)(src + 4 * j);
+            w[4 * j] = q4.x;
+            w[4 * j + 1] = q4.y;
+            w[4 * j + 2] = q4.z;
+            w[4 * j + 3] = q4.w;
         }
-        uint32_t w[4];
+    } else {
 #pragma unroll
-        for (int b = 0; b < 4; ++b) w[b] = (v[b] > a.half ? v[b] - p : v[b]) + 0x80000000u;
+        for (int j = 0; j < 16; ++j) w[j] = row < a.R && k0 + j < a.K ? src[j] : 0u;
+    }
 #pragma unroll
-        for (int i = 0; i < RES_MAXN; ++i) {
-            if (i >= (int)c.nmod) break;
-            *(uint32_t*)(out + (size_t)i * a.plane + k4) = res_bytes4(w, c, i);
+    for (int j = 0; j < 16; ++j) w[j] = (w[j] > a.half ? w[j] - p : w[j]) + 0x80000000u;
+    int8_t* out = a.out + res_chunk(row, k16, a.Kp);
+#pragma unroll
+    for (int i = 0; i < RES_MAXN; ++i) {
+        if (i >= (int)c.nmod) break;
+        v4i vw;
+#pragma unroll
+        for (int wd = 0; wd < 4; ++wd) {
+            const uint32_t w4[4] = {w[4 * wd], w[4 * wd + 1], w[4 * wd + 2], w[4 * wd + 3]};
+            vw[wd] = (int)res_bytes4(w4, c, i);
         }
+        *(v4i*)(out + (size_t)i * a.plane) = vw;
     }
 }
 
@@ -1193,7 +1194,7 @@ __global__ __launch_bounds__(256) void res_prep_cols_kernel(PrepArgs a, ResSplit
         const uint32_t v = T[16 * q + j][r ^ (q << 2)];
         w[j] = (v > a.half ? v - p : v) + 0x80000000u;
     }
-    int8_t* out = a.out + (size_t)(r0 + r) * a.Kp + c0 + 16 * q;
+    int8_t* out = a.out + res_chunk(r0 + r, c0 / 16 + q, a.Kp);
 #pragma unroll
     for (int i = 0; i < RES_MAXN; ++i) {
         if (i >= (int)c.nmod) break;
@@ -1207,91 +1208,28 @@ __global__ __launch_bounds__(256) void res_prep_cols_kernel(PrepArgs a, ResSplit
     }
 }
 
-// One modulus' int8 product on a 256 x 256 tile: the limb_tile4 pipeline (eight waves, three-stage
-// direct-to-LDS ring of 64-deep k-strips, fragments double-buffered against the MFMAs) with the
-// operand "planes" being four 64-row blocks of A and two 128-row blocks of B of one residue plane,
-// so each wave owns 4 x 2 separate 32 x 32 accumulator blocks (rows 64 s + 32 wm, columns
-// 128 t + 32 wn) and reads 6 fragments per 8 MFMAs.  The epilogue reduces every int32 sum to its
-// residue in [0, q) and stores it as a byte of the modulus' residue plane, in the accumulators' own order:
-// 5 us per tile (8192 x 8192 x 64, ten moduli: 203 us), against 12 us (490 us) with the reduction in
-// 64-bit integers and doubles and single-byte stores into row-major planes.
-// The instance the route runs: eight waves (two per SIMD, 4 x 2 blocks each), a ring of three stages.
-// (Measured at 8192^3, 10 moduli: a ring of 3, 4 or 5 stages 5.37 .. 5.43 ms; four waves with 4 x 4 blocks
-// each, a third less LDS reading per MFMA, 5.55 .. 5.93 ms; two workgroups per CU of four waves with 4 x 2
-// blocks each on 256 x 128 tiles, whose barriers are independent, 6.10 .. 6.18 ms.)
-constexpr int RES_WAVES = 8, RES_STAGES = 3;
-constexpr int RLA = 4, RLB = 2, RTM = RLA * LM, RTN = RLB * 16 * RES_WAVES;
+// One modulus' int8 product on a 256 x 256 tile (or 128 x 128) by eight waves, two down and four across, each with
+// LA x LB separate 32 x 32 accumulator blocks (rows 64 s + 32 wm, columns 128 t + 32 wn).  A goes through a
+// two-stage LDS ring of 64-deep strips, staged in registers four stages ahead; B's fragments go straight from
+// memory to registers, three stages ahead: only two waves use each, and without them the LDS port is busy 640
+// of the 1031 cycles a stage's MFMAs take (both operands through the LDS: 1024).  Bound by the matrix units'
+// power: 4.5 ms at 8192^3 and ten moduli, 75 % of the rate the chip sustains on random operands from registers.
+// (Whole call at 8192^3, same card: 5.20 ms; B two stages ahead 5.72; A by direct-to-LDS copies 5.35, the
+// compiler then waits for every outstanding load once per three stages; both operands through a three-stage
+// direct-to-LDS ring 5.65.)
+constexpr int RLA = 4, RLB = 2, RTM = 64 * RLA, RTN = 128 * RLB;
 // the small instance: 128 x 128 tiles (2 x 1 blocks per wave)
 constexpr int RSA = 2, RSB = 1;
 
-// B blocks hold 16 * WAVES rows (WAVES / 2 waves across, 32 columns each); A blocks 64 rows (two waves down).
-template <int LA, int LB, int WAVES>
-__device__ __forceinline__ void res_stage_issue(const ResArgs& a, const int8_t* Abase, const int8_t* Bbase, int wave,
-                                                uint32_t kt, uint8_t* st) {
-    constexpr int BN = 16 * WAVES, BG = BN / 16;
-    constexpr int SA = LA * LM * 64, NBLK = 4 * LA + BG * LB, PER = (NBLK + WAVES - 1) / WAVES;
-    const size_t k0 = (size_t)kt * LK;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int blk = wave + WAVES * i;
-        if (blk >= NBLK) break;
-        const int8_t* src;
-        uint8_t* dst;
-        if (blk < 4 * LA) {
-            const int s = blk >> 2, g = blk & 3;
-            src = Abase + (size_t)(s * LM + 16 * g) * a.Kp + k0;
-            dst = st + s * (LM * 64) + g * 1024;
-        } else {
-            const int s = (blk - 4 * LA) / BG, g = (blk - 4 * LA) % BG;
-            src = Bbase + (size_t)(s * BN + 16 * g) * a.Kp + k0;
-            dst = st + SA + s * (BN * 64) + g * 1024;
-        }
-        __builtin_amdgcn_global_load_lds((const void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-    }
-}
-
 template <int LA, int LB>
-struct RFrag {
-    v4i a[LA];
-    v4i b[LB];
-};
-
-template <int LA, int LB, int WAVES>
-__device__ __forceinline__ void res_stage_frag(const uint8_t* st, int ks, int wm, int wn, int lane, RFrag<LA, LB>& f) {
-    constexpr int SA = LA * LM * 64, BN = 16 * WAVES;
-    const int lr = lane & 31, q = ks * 2 + (lane >> 5);
-    const int ra = wm * 32 + lr, rb = wn * 32 + lr;
-#pragma unroll
-    for (int s = 0; s < LA; ++s) f.a[s] = *(const v4i*)(st + s * (LM * 64) + ra * 64 + 16 * (q ^ swz(ra)));
-#pragma unroll
-    for (int t = 0; t < LB; ++t) f.b[t] = *(const v4i*)(st + SA + t * (BN * 64) + rb * 64 + 16 * (q ^ swz(rb)));
-}
-
-template <int LA, int LB>
-__device__ __forceinline__ void res_mfma(const RFrag<LA, LB>& f, v16i (&acc)[LA][LB]) {
-#pragma unroll
-    for (int s = 0; s < LA; ++s)
-#pragma unroll
-        for (int t = 0; t < LB; ++t)
-            acc[s][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[s], f.b[t], acc[s][t], 0, 0, 0);
-}
-
-template <int LA, int LB, int NS, int WAVES>
 __device__ __forceinline__ void res_tile(const ResArgs& a, uint32_t tm, uint32_t tn, uint32_t mi) {
-    constexpr int BN = 16 * WAVES, SA = LA * LM * 64, SB = LB * BN * 64, STAGE = SA + SB;
-    constexpr int NBLK = 4 * LA + (BN / 16) * LB;
-    constexpr int HI = (NBLK + WAVES - 1) / WAVES, LO = NBLK / WAVES, NHI = NBLK % WAVES == 0 ? WAVES : NBLK % WAVES;
-    static_assert(NS >= 3 && NS <= 5 && NS * STAGE <= 160 * 1024, "ring of 3..5 stages within the LDS");
-    __shared__ __attribute__((aligned(1024))) uint8_t s0[STAGE];
-    __shared__ __attribute__((aligned(1024))) uint8_t s1[STAGE];
-    __shared__ __attribute__((aligned(1024))) uint8_t s2[STAGE];
-    __shared__ __attribute__((aligned(1024))) uint8_t s3[NS > 3 ? STAGE : 1];
-    __shared__ __attribute__((aligned(1024))) uint8_t s4[NS > 4 ? STAGE : 1];
-    const uint32_t m0 = tm * (LA * LM), n0 = tn * (LB * BN);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int STAGE = LA * 4096, NA = LA / 2, BN = 128;
+    __shared__ __attribute__((aligned(1024))) uint8_t ring[2][STAGE];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave & 1, wn = wave >> 1;
-    const bool hi = wave < NHI;
+    const uint32_t KT = a.Kp / 64;
+    const size_t strip = (size_t)a.Kp * 32;              // bytes of 32 rows of a plane
 
     v16i acc[LA][LB];
 #pragma unroll
@@ -1301,64 +1239,95 @@ __device__ __forceinline__ void res_tile(const ResArgs& a, uint32_t tm, uint32_t
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[s][t][r] = (int)0x80000000;
 
-    const int br = lane >> 2, bq = (lane & 3) ^ swz(br);
-    const int8_t* Abase = a.A8 + mi * a.a_plane + (size_t)(m0 + br) * a.Kp + 16 * bq;
-    const int8_t* Bbase = a.B8 + mi * a.b_plane + (size_t)(n0 + br) * a.Kp + 16 * bq;
-    // wait until at most `stages` stages of this wave's copies are in flight (0 .. NS - 1)
-    auto wait_stages = [&](int stages) {
-        const int per = hi ? HI : LO;
-        switch (stages * per) {
-#define HX_RES_WAIT(c) case c: __builtin_amdgcn_s_waitcnt(wait_imm(c, 15)); break;
-            HX_RES_WAIT(0) HX_RES_WAIT(1) HX_RES_WAIT(2) HX_RES_WAIT(3) HX_RES_WAIT(4) HX_RES_WAIT(5)
-            HX_RES_WAIT(6) HX_RES_WAIT(7) HX_RES_WAIT(8) HX_RES_WAIT(9) HX_RES_WAIT(10) HX_RES_WAIT(11)
-            HX_RES_WAIT(12) HX_RES_WAIT(13) HX_RES_WAIT(14) HX_RES_WAIT(15) HX_RES_WAIT(16)
-#undef HX_RES_WAIT
-            default: __builtin_amdgcn_s_waitcnt(wait_imm(0, 15)); break;
-        }
+    // A's strip j (32 rows), both 32-k blocks of a stage: LDS bytes [2048 j, + 2048); wave w copies blocks w and,
+    // of eight strips, w + 8
+    const int8_t* Ab = a.A8 + mi * a.a_plane + (size_t)(tm * 2 * LA + (wave >> 1)) * strip + (wave & 1) * 1024 + lane * 16;
+    const int8_t* Bb = a.B8 + mi * a.b_plane + (size_t)(tn * 4 * LB + wn) * strip + lane * 16;
+    struct AS {
+        v4i f[NA];
     };
-    const uint32_t KT = a.Kp / LK;
-    if (KT > 0) {
-        // prologue: stages 0 .. NS-1 in flight, stage 0 landed everywhere
-        res_stage_issue<LA, LB, WAVES>(a, Abase, Bbase, wave, 0, s0);
-        if (KT > 1) res_stage_issue<LA, LB, WAVES>(a, Abase, Bbase, wave, 1, s1);
-        if (KT > 2) res_stage_issue<LA, LB, WAVES>(a, Abase, Bbase, wave, 2, s2);
-        if (NS > 3 && KT > 3) res_stage_issue<LA, LB, WAVES>(a, Abase, Bbase, wave, 3, s3);
-        if (NS > 4 && KT > 4) res_stage_issue<LA, LB, WAVES>(a, Abase, Bbase, wave, 4, s4);
-        wait_stages((int)min(KT - 1, (uint32_t)NS - 1));
-        wg_barrier();
-        RFrag<LA, LB> fa, fb;
-        res_stage_frag<LA, LB, WAVES>(s0, 0, wm, wn, lane, fa);
-        __builtin_amdgcn_s_waitcnt(wait_imm(63, 0));
-        // step kt: MFMAs of (kt, ks0) while (kt, ks1) is read; stage kt+1 landed and every wave done
-        // with stage kt (barrier); stage kt+NS copied into kt's slot; MFMAs of (kt, ks1) while
-        // (kt+1, ks0) is read.  Before the barrier stages kt+2 .. min(KT-1, kt+NS-1) may be in flight.
-        auto body = [&](uint32_t kt, uint8_t* cur, const uint8_t* nxt) {
-            res_stage_frag<LA, LB, WAVES>(cur, 1, wm, wn, lane, fb);
-            __builtin_amdgcn_sched_barrier(0);
-            res_mfma<LA, LB>(fa, acc);
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_waitcnt(wait_imm(63, 0));
-            wait_stages((int)min(KT - kt - 2, (uint32_t)NS - 2));
-            wg_barrier();
-            if (kt + NS < KT) res_stage_issue<LA, LB, WAVES>(a, Abase, Bbase, wave, kt + NS, cur);
-            res_stage_frag<LA, LB, WAVES>(nxt, 0, wm, wn, lane, fa);
-            __builtin_amdgcn_sched_barrier(0);
-            res_mfma<LA, LB>(fb, acc);
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_waitcnt(wait_imm(63, 0));
-        };
-        uint8_t* const ring[5] = {s0, s1, s2, s3, s4};
-        for (uint32_t kt = 0; kt + 1 < KT; kt += NS) {
+    struct BF {
+        v4i f[2][LB];
+    };
+    struct AF {
+        v4i f[LA];
+    };
+    auto load_a = [&](uint32_t kt, AS& x) {
 #pragma unroll
-            for (int j = 0; j < NS; ++j)
-                if (kt + j + 1 < KT) body(kt + j, ring[j], ring[(j + 1) % NS]);
-        }
-        const uint32_t ls = (KT - 1) % NS;
-        const uint8_t* cur = ls == 0 ? s0 : ls == 1 ? s1 : ls == 2 ? s2 : ls == 3 ? s3 : s4;
-        res_stage_frag<LA, LB, WAVES>(cur, 1, wm, wn, lane, fb);
-        res_mfma<LA, LB>(fa, acc);
-        res_mfma<LA, LB>(fb, acc);
+        for (int i = 0; i < NA; ++i) x.f[i] = *(const v4i*)(Ab + (4 * i) * strip + (size_t)kt * 2048);
+    };
+    auto store_a = [&](uint8_t* st, const AS& x) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) *(v4i*)(st + (wave + 8 * i) * 1024 + lane * 16) = x.f[i];
+    };
+    auto load_b = [&](uint32_t kt, BF& b) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int t = 0; t < LB; ++t) b.f[ks][t] = *(const v4i*)(Bb + (4 * t) * strip + (size_t)kt * 2048 + ks * 1024);
+    };
+    auto read_a = [&](const uint8_t* st, int ks, AF& f) {
+#pragma unroll
+        for (int s = 0; s < LA; ++s) f.f[s] = *(const v4i*)(st + (2 * s + wm) * 2048 + ks * 1024 + lane * 16);
+    };
+    auto mfma = [&](const AF& x, const v4i (&y)[LB]) {
+#pragma unroll
+        for (int s = 0; s < LA; ++s)
+#pragma unroll
+            for (int t = 0; t < LB; ++t)
+                acc[s][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x.f[s], y[t], acc[s][t], 0, 0, 0);
+    };
+
+    // Stage kt uses ring slot and A registers kt % 2.  MFMAs of the first half while A's second half is read;
+    // barrier (A's stage kt + 1 is in the ring, every wave is done reading stage kt); A's stage kt + 2 into the
+    // freed slot and its registers reloaded with stage kt + 4; MFMAs of the second half while the next stage's
+    // first half is read; B's stage kt + 3 into the registers just used (three sets).  Loads past the last stage
+    // read the last one again (never used).
+    const uint32_t KL = KT - 1;
+    AS x0, x1;
+    BF b0, b1, b2;
+    AF fa, fb;
+    load_a(0, x0);
+    load_b(0, b0);
+    load_a(min(1u, KL), x1);
+    load_b(min(1u, KL), b1);
+    load_b(min(2u, KL), b2);
+    store_a(ring[0], x0);
+    load_a(min(2u, KL), x0);
+    store_a(ring[1], x1);
+    load_a(min(3u, KL), x1);
+    __builtin_amdgcn_s_waitcnt(wait_imm(63, 0));
+    wg_barrier();
+    read_a(ring[0], 0, fa);
+    auto body = [&](uint32_t kt, uint8_t* cur, const uint8_t* nxt, AS& x, BF& b) {
+        read_a(cur, 1, fb);
+        __builtin_amdgcn_sched_barrier(0);
+        mfma(fa, b.f[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(wait_imm(63, 0));
+        wg_barrier();
+        store_a(cur, x);
+        load_a(min(kt + 4, KL), x);
+        read_a(nxt, 0, fa);
+        __builtin_amdgcn_sched_barrier(0);
+        mfma(fb, b.f[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_b(min(kt + 3, KL), b);
+    };
+    uint32_t kt = 0;
+    for (; kt + 6 <= KT; kt += 6) {
+        body(kt, ring[0], ring[1], x0, b0);
+        body(kt + 1, ring[1], ring[0], x1, b1);
+        body(kt + 2, ring[0], ring[1], x0, b2);
+        body(kt + 3, ring[1], ring[0], x1, b0);
+        body(kt + 4, ring[0], ring[1], x0, b1);
+        body(kt + 5, ring[1], ring[0], x1, b2);
     }
+    if (kt < KT) body(kt, ring[0], ring[1], x0, b0);
+    if (kt + 1 < KT) body(kt + 1, ring[1], ring[0], x1, b1);
+    if (kt + 2 < KT) body(kt + 2, ring[0], ring[1], x0, b2);
+    if (kt + 3 < KT) body(kt + 3, ring[1], ring[0], x1, b0);
+    if (kt + 4 < KT) body(kt + 4, ring[0], ring[1], x0, b1);
     // s = v y mod q (y = (M / q)^-1 mod q, the CRT's factor, folded in here) from w = v + 2^31, what the
     // accumulators hold (they start at -2^31): t = sum_j byte_j(w) (y 2^(8j) mod q) + q - (y 2^31 mod q) is
     // congruent to v y and below 2^18, and (t + 1/2) / q is at least 1 / (2q) > 0.0019 from an integer, fp32's
@@ -1386,11 +1355,11 @@ __device__ __forceinline__ void res_tile(const ResArgs& a, uint32_t tm, uint32_t
         }
 }
 
-template <int LA, int LB, int NS, int WAVES>
-__global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void res_gemm_kernel(ResArgs a) {
+template <int LA, int LB>
+__global__ __launch_bounds__(512, 1) void res_gemm_kernel(ResArgs a) {
     uint32_t tm, tn;
     tile_of(blockIdx.x, a.ntm, a.ntn, tm, tn);
-    res_tile<LA, LB, NS, WAVES>(a, tm, tn, blockIdx.y);
+    res_tile<LA, LB>(a, tm, tn, blockIdx.y);
 }
 
 // CRT of the N product residues of sixteen outputs per thread into x mod p, then op into C.
@@ -1696,20 +1665,34 @@ size_t residue_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t nmod
     return (size_t)nmod * (Mp * Kp + Np * Kp + Mp * Np);
 }
 
-// The moduli count of the residue route when the limb variant takes it for this product, else 0.  It
-// needs host-side sizes, 1 <= k <= RES_KMAX and enough moduli; tile kResidueTile asks for it wherever it
-// applies; the default (tile 0) takes it where it runs at most L^2 - 4 int8 products (four-limb moduli:
-// 10 or 11 for 16) and m, n, k >= 4096, where the saved MFMA work pays for the operand splits and the CRT
-// pass (mod 2147483629, wall ms limb kernel 4 / residue route: 8192^3 7.76 / 6.26, 4096^3 1.13 / 1.01,
-// 8192^2 x 2048 2.05 / 2.11, 2048^2 x 16384 1.14 / 1.18, 2048^3 0.17 / 0.24).
-uint32_t residue_choice(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, bool device_sizes, int tile) {
+// Whether the automatic choice splits a thin deep product over K on the plain kernel: its limb tiles cannot fill
+// the GPU (256 x 256 x 65536: plain split 64 ways 0.87 ms, limb route 1.50 ms, plain unsplit 11.7 ms).
+bool auto_splits(uint32_t m, uint32_t n, uint32_t k) {
+    const uint64_t limb_tiles = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
+    return limb_tiles < 32 && plain_suggest_splits(m, n, k) > 1;
+}
+
+// The moduli count of the residue route when this product takes it, else 0.  It needs host-side sizes,
+// 1 <= k <= RES_KMAX and enough moduli; tile kResidueTile asks for it wherever it applies.  The limb variant's
+// default (tile 0) takes it where it runs at most L^2 - 4 int8 products (four-limb moduli: 10 or 11 for 16) and
+// m, n, k >= 4096.  The automatic variant takes it at every m, n once k is deep enough to pay for the splits
+// and the CRT, whose cost does not grow with k: k >= 768 for four limbs, k >= 1536 for three (us, limb kernel 4
+// / residue route; mod 2147483629: 768^3 42 / 40, 1024^3 54 / 47, 2048^3 152 / 145, 4096^3 1027 / 770,
+// 8192^3 7400 / 5200, 8192^2 x 512 606 / 680, x 1024 1131 / 953; mod 65521: 1024^3 39 / 40, 2048^3 101 / 99,
+// 4096^3 621 / 480, 8192^2 x 512 427 / 480; mod 1000003: 1024^3 40 / 41, 2048^3 107 / 109, 4096^3 675 / 550).
+// Two-limb moduli stay on the limb kernels (mod 61001: 2048^2 x 1024 49 / 66, 8192^2 x 1024 411 / 670).
+uint32_t residue_choice(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, bool device_sizes, int tile,
+                        bool automatic) {
     if (device_sizes || (tile != 0 && tile != kResidueTile)) return 0;
     const uint32_t N = residue_moduli(ctx.p, k);
     if (N == 0 || tile == kResidueTile) return N;
+    if (automatic && ctx.limbs >= 3 && k >= (ctx.limbs == 4 ? 768u : 1536u)) return N;
     const bool large = m >= 4096 && n >= 4096 && k >= 4096;
     return large && ctx.limbs > 0 && N + 4 <= ctx.limbs * ctx.limbs ? N : 0;
 }
 
+// 256 x 256 tiles once they fill the 256 compute units twice (3072^3, ten moduli: 1440 tiles, 370 us against 418
+// with 128 x 128; 4096^3 770 / 913); below, the smaller tiles cost at most as much (2048^3, 640 tiles: 145 / 147).
 uint32_t residue_side(uint32_t m, uint32_t n, uint32_t N) {
     const uint64_t tiles = (uint64_t)((m + RTM - 1) / RTM) * ((n + RTN - 1) / RTN) * N;
     return tiles >= 512 ? RTM : RTM / 2;
@@ -1717,8 +1700,8 @@ uint32_t residue_side(uint32_t m, uint32_t n, uint32_t N) {
 
 void residue_product(const ResArgs& a, uint32_t N, uint32_t side, hipStream_t s) {
     const dim3 grid(a.ntm * a.ntn, N);
-    if (side == RTM) res_gemm_kernel<RLA, RLB, RES_STAGES, RES_WAVES><<<grid, RES_WAVES * 64, 0, s>>>(a);
-    else res_gemm_kernel<RSA, RSB, RES_STAGES, RES_WAVES><<<grid, RES_WAVES * 64, 0, s>>>(a);
+    if (side == RTM) res_gemm_kernel<RLA, RLB><<<grid, 512, 0, s>>>(a);
+    else res_gemm_kernel<RSA, RSB><<<grid, 512, 0, s>>>(a);
     after_launch("res_gemm_kernel");
 }
 
@@ -1733,7 +1716,8 @@ void gemm_residue(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32
     HX_CHECK(ws != nullptr && ws_bytes >= residue_workspace_bytes(g.m, g.n, g.k, N),
              "residue route: workspace too small");
     const uint32_t p = ctx.p;
-    const uint32_t Mp = round_up(g.m, RTM), Np = round_up(g.n, RTN), Kp = round_up(g.k, 64);
+    const uint32_t side = residue_side(g.m, g.n, N);
+    const uint32_t Mp = round_up(g.m, side), Np = round_up(g.n, side), Kp = round_up(g.k, 64);
     int8_t* A8 = (int8_t*)ws;
     int8_t* B8 = A8 + (size_t)N * Mp * Kp;
     uint8_t* R = (uint8_t*)(B8 + (size_t)N * Np * Kp);
@@ -1766,7 +1750,7 @@ void gemm_residue(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32
         const bool direct = pr.rlist == nullptr && pr.clist == nullptr && pr.s_c == 1 && pr.s_r % 4 == 0 &&
                             ((uintptr_t)pr.src & 15) == 0;
         const bool cols = pr.rlist == nullptr && pr.clist == nullptr && pr.s_r == 1;
-        if (direct) res_prep_rows_kernel<<<dim3((Kp + 1023) / 1024, rows / 4), 256, 0, s>>>(pr, rs);
+        if (direct) res_prep_rows_kernel<<<dim3((Kp + 127) / 128, rows / 32), 256, 0, s>>>(pr, rs);
         else if (cols) res_prep_cols_kernel<<<dim3((Kp + 127) / 128, rows / 32), 256, 0, s>>>(pr, rs);
         else res_prep_kernel<<<dim3(Kp / 64, rows / 64), 256, 0, s>>>(pr, rs);
         after_launch(what);
@@ -1789,8 +1773,8 @@ void gemm_residue(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32
     ra.a_plane = (size_t)Mp * Kp;
     ra.b_plane = (size_t)Np * Kp;
     ra.Kp = Kp;
-    ra.ntm = Mp / RTM;
-    ra.ntn = Np / RTN;
+    ra.ntm = Mp / side;
+    ra.ntn = Np / side;
     ra.R = R;
     ra.r_plane = (size_t)Mp * Np;
     CrtArgs ca{};
@@ -1811,12 +1795,12 @@ void gemm_residue(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32
     }
     ca.pmm = p - (uint32_t)(M % p);
     if (ev0) HX_HIP(hipEventRecord(ev0, s));
-    residue_product(ra, N, RTM, s);
+    residue_product(ra, N, side, s);
     if (ev1) HX_HIP(hipEventRecord(ev1, s));
 
     ca.R = R;
     ca.r_plane = ra.r_plane;
-    ca.g = ResBlocks{RTM, ra.ntn};
+    ca.g = ResBlocks{side, ra.ntn};
     ca.nmod = N;
     ca.m = g.m;
     ca.n = g.n;
@@ -1847,22 +1831,24 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
                    int tile, hipEvent_t ev0, hipEvent_t ev1, uint32_t splits, void* split_ws, size_t split_ws_bytes) {
     const bool automatic = variant == HX_GEMM_AUTO;
     if (automatic) variant = gemm_auto_variant(ctx, g.m, g.n, g.k);
-    // a thin deep product whose limb tiles cannot fill the GPU runs faster on the plain kernel split
-    // over K (256 x 256 x 65536: plain split 64 ways 0.87 ms, limb route 1.50 ms, plain unsplit 11.7 ms)
-    if (automatic && variant == HX_GEMM_LIMB && splits != 1 && g.m_dev == nullptr && g.k_dev == nullptr) {
-        const uint64_t limb_tiles = (uint64_t)((g.m + LM - 1) / LM) * ((g.n + LN - 1) / LN);
-        if (limb_tiles < 32 && plain_suggest_splits(g.m, g.n, g.k) > 1) variant = HX_GEMM_PLAIN;
-    }
+    if (automatic && variant == HX_GEMM_LIMB && splits != 1 && g.m_dev == nullptr && g.k_dev == nullptr &&
+        auto_splits(g.m, g.n, g.k))
+        variant = HX_GEMM_PLAIN;
     uint32_t rn = 0;            // moduli of the residue route, 0 = the limb kernels
     if (variant == HX_GEMM_LIMB && g.m != 0 && g.n != 0)
-        rn = residue_choice(ctx, g.m, g.n, g.k, g.m_dev != nullptr || g.k_dev != nullptr, tile);
+        rn = residue_choice(ctx, g.m, g.n, g.k, g.m_dev != nullptr || g.k_dev != nullptr, tile, automatic);
     if (rn != 0) {
         // the default route falls back to the limb kernels when its planes do not fit (a caller workspace
-        // sized for the limb planes, or the library's own that cannot grow inside a capture)
+        // sized for the limb planes, the library's own that cannot grow inside a capture, device memory)
         const bool asked = tile == kResidueTile;
         const size_t need = residue_workspace_bytes(g.m, g.n, g.k, rn);
         if (ws == nullptr) {
-            void* own = stream_scratch(s, SCRATCH_LIMB, need);
+            void* own = nullptr;
+            try {
+                own = stream_scratch(s, SCRATCH_LIMB, need);
+            } catch (const Error& e) {
+                if (asked || e.code != HX_E_NOMEM) throw;
+            }
             if (own != nullptr) {
                 ws = own;
                 ws_bytes = need;
@@ -2221,9 +2207,10 @@ extern "C" {
 HX_API size_t hx_gemm_workspace_bytes_tile(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant,
                                            int tile) {
     if (ctx == nullptr) return 0;
-    if (variant == HX_GEMM_AUTO) variant = gemm_auto_variant(*ctx, m, n, k);
+    const bool automatic = variant == HX_GEMM_AUTO;
+    if (automatic) variant = gemm_auto_variant(*ctx, m, n, k);
     if (variant != HX_GEMM_LIMB) return 0;
-    const uint32_t rn = residue_choice(*ctx, m, n, k, false, tile);
+    const uint32_t rn = residue_choice(*ctx, m, n, k, false, tile, automatic);
     return rn ? residue_workspace_bytes(m, n, k, rn) : limb_workspace_bytes(*ctx, m, n, k);
 }
 
@@ -2235,9 +2222,10 @@ HX_API uint32_t hx_gemm_residue_moduli(uint32_t p, uint32_t k) { return p >= 2 ?
 
 HX_API int hx_gemm_route(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile) {
     if (ctx == nullptr) return -1;
-    if (variant == HX_GEMM_AUTO) variant = gemm_auto_variant(*ctx, m, n, k);
+    const bool automatic = variant == HX_GEMM_AUTO;
+    if (automatic) variant = gemm_auto_variant(*ctx, m, n, k);
     if (variant != HX_GEMM_LIMB || ctx->limbs == 0) return 0;
-    if (residue_choice(*ctx, m, n, k, false, tile) != 0) return kResidueTile;
+    if (residue_choice(*ctx, m, n, k, false, tile, automatic) != 0) return kResidueTile;
     return limb_version(tile);
 }
 

@@ -4,7 +4,7 @@
 //
 //  * The residue route (gemm64_residue; k >= 40, outside a stream capture): the operands modulo up to 19
 //    pairwise coprime bytes, one int8 MFMA product per modulus (res_gemm_kernel, hx_gemm.hip), and the CRT
-//    back to 64 bits.  2048^3 mod 2^61 - 1: 17 products, 0.269 ms = 3.2e13 multiply-adds/s for the whole
+//    back to 64 bits.  2048^3 mod 2^61 - 1: 17 products, 0.256 ms = 3.4e13 multiply-adds/s for the whole
 //    call, against 4.19 ms (2.05e12) on the plain kernel; 512^3 0.049 against 0.364 ms.  Bound by the int8
 //    products and the HBM passes over the residue planes (17 bytes per operand entry and per output).
 //
@@ -207,7 +207,7 @@ struct Prep64 {
 
 // Residue planes of one 32-row x 128-k tile.  The entries a_b + 2^63 go through LDS as T[k][row] (row XOR 4 times
 // the 16-k chunk: the strided reads below spread over the banks), loaded along whichever index is contiguous
-// in memory; each thread then turns 16 k of one row into 16 bytes per plane, 128 contiguous bytes per row.
+// in memory; each thread then turns 16 k of one row into 16 bytes per plane (res_chunk: 128 contiguous bytes per eight rows).
 // With w = a_b + 2^63 (a word of 8 bytes w_j), t = sum_j w_j (2^(8j) mod q) + q - (2^63 mod q) is congruent to
 // a_b and below 8 * 255 * 254 + 255 < 2^19, so fp32 holds it and t fl(1/q) + 1/2 is within 2^19 / 173 * 2^-22
 // < 8e-4 of t / q + 1/2, whose fractional part is at least 1 / (2q) > 0.0019 from an integer for odd q:
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void prep64_kernel(Prep64 a, Split64 c) {
     uint64_t w[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) w[j] = T[16 * qd + j][r ^ (qd << 2)];
-    int8_t* out = a.out + (size_t)(r0 + r) * a.Kp + c0 + 16 * qd;
+    int8_t* out = a.out + res_chunk(r0 + r, c0 / 16 + qd, a.Kp);
     for (uint32_t i = 0; i < c.nmod; ++i) {
         const uint32_t Q = c.q[i], TL = c.tlo[i], TH = c.thi[i], KQ = c.kq[i];
         const float IQ = c.iq[i];
@@ -321,7 +321,7 @@ uint32_t moduli64(uint64_t p, uint32_t k) {
 
 // Shallower products stay on the plain kernel: the splits and the CRT cost the same at any k, the plain kernel's
 // time grows with k (mod 2^61 - 1, us plain / residue: 2048 x 2048 x 16 59 / 109, x 64 180 / 122; 32^3 27 / 33,
-// 64^3 56 / 32; 512^3 364 / 49, 2048^3 4190 / 269).
+// 64^3 56 / 32; 512^3 364 / 49, 2048^3 4190 / 256).
 constexpr uint32_t RES64_MIN_K = 40;
 constexpr size_t RES64_WS = (size_t)4 << 30;      // bytes of planes held at a time; C runs in blocks that fit
 

@@ -14,8 +14,8 @@ constexpr uint8_t RES_Q[RES_MAXQ] = {255, 254, 253, 251, 247, 241, 239, 233, 229
 __host__ __device__ constexpr uint32_t res_modulus(int i) { return RES_Q[i]; }
 
 struct ResArgs {
-    const int8_t* A8;            // residue plane i of A at A8 + i * a_plane: Mp rows of Kp bytes
-    const int8_t* B8;            // residue plane i of B at B8 + i * b_plane: Np rows of Kp bytes
+    const int8_t* A8;            // residue plane i of A at A8 + i * a_plane: Mp rows of Kp bytes (res_chunk's order)
+    const int8_t* B8;            // residue plane i of B at B8 + i * b_plane: Np rows of Kp bytes (the same)
     size_t a_plane, b_plane;
     uint32_t Kp;
     uint32_t ntm, ntn;
@@ -26,6 +26,13 @@ struct ResArgs {
     uint32_t kq[RES_MAXQ];       // q - (y 2^31 mod q)
     float iq[RES_MAXQ];
 };
+
+// An operand plane lies as the MFMA fragments do: 1 KB per 32 rows x 32 k, 16 bytes per lane (row lane % 32, k
+// 16 (lane / 32) .. + 15), the k blocks of 32 rows one after the other.  The byte offset of a row's 16-byte
+// chunk c (k = 16 c ..) in a plane of Kp bytes per row (Kp a multiple of 64):
+__device__ __forceinline__ size_t res_chunk(uint32_t row, uint32_t c, uint32_t Kp) {
+    return ((size_t)(row >> 5) * (Kp >> 5) + (c >> 1)) * 1024 + (c & 1) * 512 + (row & 31) * 16;
+}
 
 // The product residues of a plane lie as the MFMA accumulators do: 1 KB per 32 x 32 block, 16 bytes per lane
 // (byte r: row (r / 4) 8 + 4 (lane / 32) + r % 4, column lane % 32), so the product kernel stores and the CRT

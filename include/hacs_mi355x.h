@@ -86,7 +86,8 @@ typedef struct hx_gemm_opts {   /* GemmOpts, CudaKernels.h:64-79 */
                                coprime moduli and a CRT recombination (N = 10 for p < 2^32, k <= 8192;
                                host-side sizes and k <= 133144 only, else the limb kernels; its workspace
                                is hx_gemm_workspace_bytes_tile's, all of it: K is not chunked).  0 takes
-                               the residue route for large four-limb products when its workspace fits
+                               the residue route for large four-limb products (under HX_GEMM_AUTO for
+                               every deep three- and four-limb product) when its workspace fits
                                (hx_gemm_route), else kernel 4 */
     void *workspace;        /* the limb route's planes (the reference's imma_workspace, CudaKernels.h:72-75):
                                hx_gemm_workspace_bytes() runs K in one piece, less (at least the bytes of one

@@ -1,0 +1,46 @@
+"""The automatic choice's residue route against the plain kernel over every operand form it accepts: the depths
+where the rule switches, both tile sizes and their edges, orders, strides, unaligned bases and ops."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _draw(p, m, n, seed, form):
+    """An m x n residue matrix: row-major, column-major, a window of a wider matrix (unaligned base), every
+    second column."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    r = lambda a, b: torch.randint(0, p, (a, b), generator=g, device="cuda").to(torch.int32)
+    if form == "row":
+        return r(m, n)
+    if form == "col":
+        return r(n, m).t()
+    if form == "window":
+        return r(m + 2, n + 5)[1:1 + m, 3:3 + n]
+    return r(m, 2 * n)[:, ::2]
+
+
+@pytest.mark.parametrize("p,k,route", [(2147483629, 767, 4), (2147483629, 768, 6), (4278124259, 1000, 6),
+                                       (65521, 1535, 4), (65521, 1536, 6), (61001, 2000, 4)])
+def test_auto_route_rule(p, k, route):
+    from hacs_amd import engine as E
+    assert E.gemm_route(E.ModCtx(p), 700, 700, k, E.HX_GEMM_AUTO) == route
+
+
+@pytest.mark.parametrize("fa,fb,fc", [("row", "row", "row"), ("col", "col", "col"), ("window", "row", "window"),
+                                      ("row", "window", "row"), ("step", "col", "step"), ("col", "step", "row")])
+@pytest.mark.parametrize("p,m,n,k", [(2147483629, 515, 700, 770), (65521, 640, 513, 1537), (1000003, 1025, 257, 1600),
+                                     (2147483647, 1793, 2049, 833)])      # the last: 256 x 256 tiles
+def test_auto_route_equals_plain(hx_gpu, p, m, n, k, fa, fb, fc):
+    from hacs_amd import engine as E
+    ctx = E.ModCtx(p)
+    assert E.gemm_route(ctx, m, n, k, E.HX_GEMM_AUTO) == 6
+    A, B = _draw(p, m, k, 1, fa), _draw(p, k, n, 2, fb)
+    for op in (E.GemmOp.Set, E.GemmOp.Add, E.GemmOp.Sub):
+        C, D = _draw(p, m, n, 3, fc), _draw(p, m, n, 3, fc)
+        E.gemm(ctx, A, B, C, op)
+        E.gemm(ctx, A, B, D, op, variant=E.HX_GEMM_PLAIN, splits=1)
+        assert torch.equal(C, D), (fa, fb, fc, op)
+    E.gemm_nt(ctx, A, _draw(p, k, n, 2, fb).t(), C)
+    E.gemm(ctx, A, B, D, variant=E.HX_GEMM_PLAIN, splits=1)
+    assert torch.equal(C, D)
