@@ -151,3 +151,22 @@ def test_f2_gemm_matches_oracle(hx_gpu, O, m, n, k):
         torch.cuda.synchronize()
         got = E.unpack_bits(dC.cpu().numpy().view(np.uint64), n)
         assert np.array_equal(got, want ^ C0 if acc else want), f"accumulate={acc}"
+
+
+@pytest.mark.parametrize("m,n,block", [(2000, 200, 140), (1100, 130, 64), (9000, 190, 1100), (3000, 257, 20)])
+def test_f2_rref_repeated_rows(hx_gpu, O, m, n, block):
+    """Runs of equal rows, the later runs holding the lower columns: a panel's first rows with a bit span
+    little, its pivots are found out of column order and by the search over all rows."""
+    from hacs_amd import engine as E
+    rng = np.random.default_rng(m + n)
+    base = rng.integers(0, 2, ((m + block - 1) // block, n)).astype(np.uint32)
+    for i in range(base.shape[0]):
+        base[i, :max(0, 60 - 4 * i)] = 0
+        base[i, 64:64 + max(0, 50 - 3 * i)] = 0
+    A = np.repeat(base, block, axis=0)[:m]
+    A[-80:] = rng.integers(0, 2, (80, n))
+    rank, piv, out = _device_rref(E, A)
+    r, opiv, _, R = O.rref_rule(2, A, threads=16)
+    assert rank == r and np.array_equal(piv, opiv)
+    got = E.unpack_bits(out, n)
+    assert np.array_equal(got[:r], R) and not got[r:].any()
