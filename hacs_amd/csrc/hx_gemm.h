@@ -47,6 +47,10 @@ uint32_t limb_k_chunk(uint32_t limbs);
 uint32_t limb_k_chunk_for(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, size_t bytes);
 // The variant the automatic policy picks for this shape.
 int gemm_auto_variant(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k);
+// Products of small depth, and small ones (hx_thin.hip): whether the automatic choice runs this shape there, and
+// the product (any strides, op; host-side sizes, no gathers, p < 2^31 with limbs).
+bool thin_applies(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k);
+void gemm_thin(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s);
 // splits: 1 = never split K, 0 = the automatic policy, > 1 = that many (plain kernel only); split_ws NULL =
 // the stream's own partials.
 void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int variant, void* ws, size_t ws_bytes,

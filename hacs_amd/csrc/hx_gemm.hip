@@ -1831,9 +1831,22 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
                    int tile, hipEvent_t ev0, hipEvent_t ev1, uint32_t splits, void* split_ws, size_t split_ws_bytes) {
     const bool automatic = variant == HX_GEMM_AUTO;
     if (automatic) variant = gemm_auto_variant(ctx, g.m, g.n, g.k);
-    if (automatic && variant == HX_GEMM_LIMB && splits != 1 && g.m_dev == nullptr && g.k_dev == nullptr &&
-        auto_splits(g.m, g.n, g.k))
-        variant = HX_GEMM_PLAIN;
+    const bool split = automatic && variant == HX_GEMM_LIMB && splits != 1 && g.m_dev == nullptr && g.k_dev == nullptr &&
+                       auto_splits(g.m, g.n, g.k);
+    if (split) variant = HX_GEMM_PLAIN;
+    if (automatic && splits <= 1 && g.m_dev == nullptr && g.k_dev == nullptr && g.a_rows == nullptr &&
+        g.a_cols == nullptr && g.c_rows == nullptr && thin_applies(ctx, g.m, g.n, g.k)) {
+        if (ev0) HX_HIP(hipEventRecord(ev0, s));
+        gemm_thin(ctx, g, s);
+        if (ev1) HX_HIP(hipEventRecord(ev1, s));
+        stat_add(ST_GEMMS, 1);
+        stat_add(ST_LIMB, 1);
+        return;
+    }
+    // small but deep: the limb kernels' few tiles still beat the plain kernel's serial depth (32 x 32 x 512: 28
+    // against 97 us)
+    if (automatic && variant == HX_GEMM_PLAIN && ctx.limbs > 0 && !split && splits <= 1 && g.k > 256 && g.m_dev == nullptr && g.k_dev == nullptr)
+        variant = HX_GEMM_LIMB;
     uint32_t rn = 0;            // moduli of the residue route, 0 = the limb kernels
     if (variant == HX_GEMM_LIMB && g.m != 0 && g.n != 0)
         rn = residue_choice(ctx, g.m, g.n, g.k, g.m_dev != nullptr || g.k_dev != nullptr, tile, automatic);
@@ -2223,7 +2236,12 @@ HX_API uint32_t hx_gemm_residue_moduli(uint32_t p, uint32_t k) { return p >= 2 ?
 HX_API int hx_gemm_route(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile) {
     if (ctx == nullptr) return -1;
     const bool automatic = variant == HX_GEMM_AUTO;
-    if (automatic) variant = gemm_auto_variant(*ctx, m, n, k);
+    if (automatic) {
+        if (thin_applies(*ctx, m, n, k)) return 7;
+        variant = gemm_auto_variant(*ctx, m, n, k);
+        if (variant == HX_GEMM_LIMB && auto_splits(m, n, k)) return 0;
+        if (ctx->limbs > 0 && k > 256) variant = HX_GEMM_LIMB;
+    }
     if (variant != HX_GEMM_LIMB || ctx->limbs == 0) return 0;
     if (residue_choice(*ctx, m, n, k, false, tile, automatic) != 0) return kResidueTile;
     return limb_version(tile);

@@ -71,7 +71,7 @@ enum { HX_OP_SET = 0, HX_OP_ADD = 1, HX_OP_SUB = 2 };
 
 /* GEMM kernel variants (no counterpart: the reference has one u32 kernel and the p <= 127 IMMA route) */
 enum {
-    HX_GEMM_AUTO = 0,   /* the library picks: LIMB when m*n*k >= 4e6 and k >= 64, else PLAIN (never changes a value) */
+    HX_GEMM_AUTO = 0,   /* the library picks by shape and limb count (hx_gemm_route; never changes a value) */
     HX_GEMM_PLAIN = 1,  /* u32 x u32 -> exact u64 (+carry word) accumulation on the VALU, Barrett epilogue */
     HX_GEMM_LIMB = 2    /* balanced residues as signed 8-bit limbs on the INT8 MFMA cores, exact recombination */
 };
@@ -238,9 +238,10 @@ HX_API size_t hx_gemm_workspace_bytes_tile(const hx_modctx *ctx, uint32_t m, uin
  * counterpart in the reference. */
 HX_API uint32_t hx_gemm_residue_moduli(uint32_t p, uint32_t k);
 /* The kernel a product with host-side sizes runs for (variant, tile), given a large enough workspace: 0 = the
- * plain kernel, 1 .. 5 = that limb kernel, 6 = the residue route; -1 for a NULL ctx.  The default (tile 0)
- * takes the residue route where it needs at most limbs^2 - 4 int8 products and m, n, k >= 4096, else limb
- * kernel 4.  No counterpart in the reference. */
+ * plain kernel, 1 .. 5 = that limb kernel, 6 = the residue route, 7 = the thin kernel (limbs split on the fly, AUTO
+ * only: k <= 64, and k <= 256 for small products); -1 for a NULL ctx.  LIMB's default (tile 0) takes the residue
+ * route where it needs at most limbs^2 - 4 int8 products and m, n, k >= 4096, else limb kernel 4; AUTO takes it
+ * from k = 768 (four limbs) or 1536 (three).  No counterpart in the reference. */
 HX_API int hx_gemm_route(const hx_modctx *ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile);
 /* The K chunk a limb workspace of workspace_bytes runs (imma_k_chunk, CudaKernels.h:100-110): min(k, the
  * int32-exact chunk) when its planes fit, else the largest multiple of 64 that fits; 0 when not even a
