@@ -58,8 +58,8 @@ struct RArgs {
     uint32_t region;      // LDS words for the panel / pivot-row block
     uint32_t mmax, nmax;
     DevMod M;
-    LimbConsts lc;        // the limb split of the MFMA trailing update (hx_limbs.h)
     uint32_t half;        // (p - 1) / 2
+    double inv;           // 1 / p (limb_small_product)
     int L;                // limbs per residue (1..4)
 };
 
@@ -76,21 +76,30 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 // limb products accumulate per anti-diagonal in int32, and the exact recombination (hx_limbs.h)
 // gives the residue subtracted from the entry.  A wave takes a 32-row block of either set, loads
 // the block's k coefficients into registers before any write, then walks the 32-column blocks.
+// The limb fragment of 16 residues get(0 .. 15), one per k-byte.
+template <int L, class F>
+__device__ __forceinline__ void split16(F&& get, uint32_t p, uint32_t half, v4i (&f)[L]) {
+    uint32_t v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = get(i);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const uint32_t x[4] = {v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+        uint32_t w[L];
+        limb_split4<L>(x, p, half, w);
+#pragma unroll
+        for (int s = 0; s < L; ++s) f[s][g] = (int)w[s];
+    }
+}
+
 template <int L>
 __device__ void trailing_mfma(const RJob& job, const RArgs& a, const uint32_t* B, bool planes, uint32_t nb,
                               uint32_t wc, uint32_t k, uint32_t c, uint32_t mu, const uint32_t* list,
                               const uint8_t* chosen, const uint32_t* s_q, uint32_t r) {
-    constexpr int ND = 2 * L - 1;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 31, lg = lane >> 5;
     const uint32_t p = a.M.p, half = a.half;
     const uint32_t nrb_u = nb > wc ? (mu + 31) / 32 : 0, nrb = nrb_u + (r + 31) / 32;
-    // the limb planes of 16 residues (one per k-byte) into L fragment registers
-    auto split_into = [&](uint32_t x, int i, v4i (&f)[L]) {
-        int32_t d[4] = {0, 0, 0, 0};
-        limbs_of(x, p, half, L, d);
-#pragma unroll
-        for (int s = 0; s < L; ++s) f[s][i >> 2] |= (int)(((uint32_t)d[s] & 0xffu) << (8 * (i & 3)));
-    };
+    const SmallConsts sc{p, a.inv};
     for (uint32_t rb = wave; rb < nrb; rb += RT / 64) {
         const bool urows = rb >= nrb_u;                       // a block of stored pivot rows
         const uint32_t b0 = (urows ? rb - nrb_u : rb) * 32, nrows = urows ? r : mu, jbeg = urows ? 0 : wc;
@@ -101,14 +110,11 @@ __device__ void trailing_mfma(const RJob& job, const RArgs& a, const uint32_t* B
         const uint32_t u = b0 + lr;
         const bool live = live_row(u);
         const int64_t rowoff = live ? (urows ? (int64_t)u : (int64_t)list[u]) * ld + c : 0;
-        v4i fa[L];
-#pragma unroll
-        for (int s = 0; s < L; ++s) fa[s] = v4i{0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
+        v4i fa[1][L];
+        split16<L>([&](int i) {
             const uint32_t t = 16 * lg + i;
-            split_into((live && t < k) ? base[rowoff + s_q[t]] : 0u, i, fa);
-        }
+            return (live && t < k) ? base[rowoff + s_q[t]] : 0u;
+        }, p, half, fa[0]);
         // the 16 output rows this lane touches (accumulator element e), as matrix row indices;
         // NOROW for rows that take no update
         constexpr uint32_t NOROW = 0xffffffffu;
@@ -126,45 +132,28 @@ __device__ void trailing_mfma(const RJob& job, const RArgs& a, const uint32_t* B
             uint32_t cv[16];
 #pragma unroll
             for (int e = 0; e < 16; ++e) cv[e] = (j < nb && orow[e] != NOROW) ? basec[(int64_t)orow[e] * ld + j] : 0u;
-            v4i fb[L];
+            v4i fb[1][L];
 #pragma unroll
-            for (int s = 0; s < L; ++s) fb[s] = v4i{0, 0, 0, 0};
+            for (int s = 0; s < L; ++s) fb[0][s] = v4i{0, 0, 0, 0};
             if (planes) {
                 if (j < nb) {
                     const uint8_t* P8 = (const uint8_t*)B + 32 * j + 16 * lg;
 #pragma unroll
-                    for (int s = 0; s < L; ++s) fb[s] = *(const v4i*)(P8 + (size_t)s * 32 * nb);
+                    for (int s = 0; s < L; ++s) fb[0][s] = *(const v4i*)(P8 + (size_t)s * 32 * nb);
                 }
             } else {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
+                split16<L>([&](int i) {
                     const uint32_t t = 16 * lg + i;
-                    split_into((j < nb && t < k) ? B[t * nb + j] : 0u, i, fb);
-                }
+                    return (j < nb && t < k) ? B[t * nb + j] : 0u;
+                }, p, half, fb[0]);
             }
-            v16i acc[ND];
-#pragma unroll
-            for (int d = 0; d < ND; ++d)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[d][e] = 0;
-#pragma unroll
-            for (int s = 0; s < L; ++s)
-#pragma unroll
-                for (int t = 0; t < L; ++t)
-                    acc[s + t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[s], fb[t], acc[s + t], 0, 0, 0);
+            uint32_t x[16];
+            limb_small_product<L, 1>(fa, fb, sc, x);
             if (j < nb) {
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    if (orow[e] == NOROW) continue;
-                    int32_t D[ND];
-                    bool nzd = false;
-#pragma unroll
-                    for (int d = 0; d < ND; ++d) {
-                        D[d] = acc[d][e];
-                        nzd |= D[d] != 0;
-                    }
-                    if (!nzd) continue;                           // a zero update leaves the entry
-                    basec[(int64_t)orow[e] * ld + j] = subm(cv[e], limb_recombine<ND>(D, a.lc, a.M), p);
+                    if (orow[e] == NOROW || x[e] == 0) continue;      // a zero update leaves the entry
+                    basec[(int64_t)orow[e] * ld + j] = subm(cv[e], x[e], p);
                 }
             }
         }
@@ -208,7 +197,7 @@ template <int L, class Ar>
 __device__ void pivot_solve(const RJob& job, const RArgs& a, const Ar& ar, uint32_t* pan, uint32_t k, uint32_t c,
                             uint32_t nb, uint32_t r, bool planes, const uint32_t* s_P, const uint32_t* s_q,
                             uint32_t* s_inv) {
-    constexpr int ND = 2 * L - 1, GS = 64;
+    constexpr int GS = 64;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 31, lg = lane >> 5;
     const uint32_t p = ar.p;
     uint32_t* G0 = pan;
@@ -265,67 +254,41 @@ __device__ void pivot_solve(const RJob& job, const RArgs& a, const Ar& ar, uint3
         s_inv[tid] = ar.prep(iv);
     }
     __syncthreads();
-    auto split_into = [&](uint32_t x, int i, v4i (&f)[L]) {
-        int32_t d[4] = {0, 0, 0, 0};
-        limbs_of(x, p, a.half, L, d);
-#pragma unroll
-        for (int s = 0; s < L; ++s) f[s][i >> 2] |= (int)(((uint32_t)d[s] & 0xffu) << (8 * (i & 3)));
-    };
     // W's fragment: row lr, k-bytes 16 lg .. 16 lg + 15
-    v4i fa[L];
-#pragma unroll
-    for (int s = 0; s < L; ++s) fa[s] = v4i{0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    v4i fa[1][L];
+    split16<L>([&](int i) {
         const uint32_t t2 = 16 * lg + i;
-        split_into((lr < k && t2 < k) ? ar.mul(Gk[lr * GS + k + t2], s_inv[lr]) : 0u, i, fa);
-    }
+        return (lr < k && t2 < k) ? ar.mul(Gk[lr * GS + k + t2], s_inv[lr]) : 0u;
+    }, p, a.half, fa[0]);
+    const SmallConsts sc{p, a.inv};
     __syncthreads();                                  // every wave holds W: the region may be overwritten
     uint32_t* B = pan;
     const uint32_t ncb = (nb + 31) / 32;
     for (uint32_t cb = wave; cb < ncb; cb += RT / 64) {
         const uint32_t j = cb * 32 + lr;
-        v4i fb[L];
-#pragma unroll
-        for (int s = 0; s < L; ++s) fb[s] = v4i{0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
+        v4i fb[1][L];
+        split16<L>([&](int i) {
             const uint32_t t2 = 16 * lg + i;
-            split_into((j < nb && t2 < k) ? job.A[(int64_t)s_P[t2] * job.lda + c + j] : 0u, i, fb);
-        }
-        v16i acc[ND];
-#pragma unroll
-        for (int d = 0; d < ND; ++d)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[d][e] = 0;
-#pragma unroll
-        for (int s = 0; s < L; ++s)
-#pragma unroll
-            for (int t = 0; t < L; ++t)
-                acc[s + t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[s], fb[t], acc[s + t], 0, 0, 0);
+            return (j < nb && t2 < k) ? job.A[(int64_t)s_P[t2] * job.lda + c + j] : 0u;
+        }, p, a.half, fb[0]);
+        uint32_t x[16];
+        limb_small_product<L, 1>(fa, fb, sc, x);       // (rows at or past k: W's are zero, so is x)
         if (j >= nb) continue;
         uint32_t word[4][L];                          // limb bytes of rows g*8 + lg*4 .. +3, per plane
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const uint32_t t = (e / 4) * 8 + lg * 4 + (e % 4);
-            int32_t D[ND];
-#pragma unroll
-            for (int d = 0; d < ND; ++d) D[d] = acc[d][e];
-            const uint32_t x = t < k ? limb_recombine<ND>(D, a.lc, a.M) : 0u;
-            if (t < k) job.U[(size_t)(r + t) * job.n + c + j] = x;
-            if (planes) {
-                int32_t dg[4] = {0, 0, 0, 0};
-                limbs_of(x, p, a.half, L, dg);
-#pragma unroll
-                for (int sp = 0; sp < L; ++sp) {
-                    const uint32_t byte = ((uint32_t)dg[sp] & 0xffu) << (8 * (e % 4));
-                    word[e / 4][sp] = (e % 4) == 0 ? byte : (word[e / 4][sp] | byte);
-                }
-            } else if (t < k) {
-                B[t * nb + j] = x;
+            if (t < k) {
+                job.U[(size_t)(r + t) * job.n + c + j] = x[e];
+                if (!planes) B[t * nb + j] = x[e];
             }
         }
         if (planes) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const uint32_t x4[4] = {x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3]};
+                limb_split4<L>(x4, p, a.half, word[g]);
+            }
             // plane sp, column j: 32 k-bytes (rows t = 0..31) at byte sp * 32 nb + 32 j + t
             uint8_t* P8 = (uint8_t*)B;
 #pragma unroll
@@ -655,7 +618,7 @@ int rref_batch_run_impl(void* vb, hipStream_t s) {
     a.mmax = b->mmax;
     a.nmax = b->nmax;
     a.M = devmod(b->ctx);
-    a.lc = limb_consts(b->ctx.p);
+    a.inv = 1.0 / (double)b->ctx.p;
     a.half = (b->ctx.p - 1) / 2;
     const uint32_t pp = b->ctx.p;                       // limbs from p itself (balanced digits)
     a.L = pp <= 255u ? 1 : (pp <= 65279u ? 2 : (pp <= 16711423u ? 3 : 4));

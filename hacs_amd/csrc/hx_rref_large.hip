@@ -545,13 +545,12 @@ struct UpdArgs {
     uint32_t* Cout;
     int64_t cors;
     DevMod M;
-    LimbConsts lc;
+    double inv;                      // 1 / p (limb_small_product)
     uint32_t half;
 };
 
 template <int L>
 __global__ __launch_bounds__(256) void upd32_kernel(UpdArgs u) {
-    constexpr int ND = 2 * L - 1;
     if (u.chain) __builtin_amdgcn_s_setprio(2);     // the next panel's columns: on the panel chain
     const uint32_t m = min(*u.m_dev, u.m), k = min(*u.k_dev, 32u);
     if (k == 0 && u.Cin == u.Cout && u.c_rows == nullptr && u.cirs == u.cors) return;   // in place, nothing to do
@@ -577,16 +576,16 @@ __global__ __launch_bounds__(256) void upd32_kernel(UpdArgs u) {
         const uint32_t r = b0 + (e / 4) * 8 + lg * 4 + (e % 4);
         crow[e] = r < m ? (u.c_rows ? u.c_rows[r] : r) : 0u;
     }
-    v4i fa[L];
+    v4i fa[1][L];
 #pragma unroll
-    for (int s2 = 0; s2 < L; ++s2) fa[s2] = v4i{0, 0, 0, 0};
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t x4[4] = {av[4 * i], av[4 * i + 1], av[4 * i + 2], av[4 * i + 3]};
+        uint32_t w[L];
+        limb_split4<L>(x4, p, u.half, w);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        int32_t d[4] = {0, 0, 0, 0};
-        limbs_of(av[i], p, u.half, L, d);
-#pragma unroll
-        for (int s2 = 0; s2 < L; ++s2) fa[s2][i >> 2] |= (int)(((uint32_t)d[s2] & 0xffu) << (8 * (i & 3)));
+        for (int s2 = 0; s2 < L; ++s2) fa[0][s2][i] = (int)w[s2];
     }
+    const SmallConsts sc{p, u.inv};
     for (uint32_t cb = 0; cb < u.ucb; ++cb) {
         const uint32_t jb = (cg * u.ucb + cb) * 32;
         if (jb >= u.n) break;
@@ -598,44 +597,25 @@ __global__ __launch_bounds__(256) void upd32_kernel(UpdArgs u) {
         for (int e = 0; e < 16; ++e) asm volatile("" : "+v"(crow[e]));
         uint32_t obase = b0 + lg * 4;
         asm volatile("" : "+v"(obase));
-        v4i fb[L];
+        v4i fb[1][L];
 #pragma unroll
         for (int s2 = 0; s2 < L; ++s2)
-            fb[s2] = jok ? *(const v4i*)(u.planes + (size_t)s2 * u.pstride + (size_t)(u.pcol0 + j) * 32 + 16 * lg)
-                         : v4i{0, 0, 0, 0};
+            fb[0][s2] = jok ? *(const v4i*)(u.planes + (size_t)s2 * u.pstride + (size_t)(u.pcol0 + j) * 32 + 16 * lg)
+                            : v4i{0, 0, 0, 0};
         uint32_t cv[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const uint32_t r = obase + (e / 4) * 8 + (e % 4);
             cv[e] = (jok && r < m) ? u.Cin[(int64_t)crow[e] * u.cirs + j] : 0u;
         }
-        int64_t xs[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) xs[e] = 0;
-#pragma unroll
-        for (int dg = 0; dg < ND; ++dg) {
-            v16i acc;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[e] = 0;
-#pragma unroll
-            for (int s2 = 0; s2 < L; ++s2) {
-                const int t = dg - s2;
-                if (t >= 0 && t < L) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[s2], fb[t], acc, 0, 0, 0);
-            }
-            const int64_t wd = limb_weight(dg, u.lc);
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                xs[e] += (int64_t)acc[e] * wd;
-                asm volatile("" : "+v"(xs[e]));  // folded here, not sunk to the epilogue: one accumulator live
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        uint32_t x[16];
+        limb_small_product<L, 1>(fa, fb, sc, x);
         if (!jok) continue;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const uint32_t r = obase + (e / 4) * 8 + (e % 4);
             if (r >= m) continue;
-            u.Cout[(int64_t)r * u.cors + j] = subm(cv[e], red64((uint64_t)xs[e] + u.lc.off, u.M), p);
+            u.Cout[(int64_t)r * u.cors + j] = subm(cv[e], x[e], p);
         }
     }
 }
@@ -910,7 +890,7 @@ void enqueue_large(const hx_modctx& ctx, const Ar& ar, uint32_t m, uint32_t n, c
     // the limb split of the k <= 32 products (balanced digits of residues mod p)
     const uint32_t L = ctx.p <= 255u ? 1 : (ctx.p <= 65279u ? 2 : (ctx.p <= 16711423u ? 3 : 4));
     const uint32_t half = (ctx.p - 1) / 2;
-    const LimbConsts lc = limb_consts(ctx.p);
+    const double inv = 1.0 / (double)ctx.p;
     const DevMod dm = devmod(ctx);
     uint64_t n_upd = 0;
     const uint64_t launches0 = stat_value(ST_KERNELS);
@@ -1001,7 +981,7 @@ void enqueue_large(const hx_modctx& ctx, const Ar& ar, uint32_t m, uint32_t n, c
                 u.c_rows = Rl;
                 u.cors = n;
                 u.M = dm;
-                u.lc = lc;
+                u.inv = inv;
                 u.half = half;
                 u.n = n1;
                 u.ucb = 1;
@@ -1053,7 +1033,7 @@ void enqueue_large(const hx_modctx& ctx, const Ar& ar, uint32_t m, uint32_t n, c
                 u.Cout = U + c;
                 u.cors = n;
                 u.M = dm;
-                u.lc = lc;
+                u.inv = inv;
                 u.half = half;
                 upd(u, s3);
                 HX_HIP(hipEventRecord(side.ev_gj[slot], s3));
