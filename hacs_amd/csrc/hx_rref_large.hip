@@ -434,16 +434,32 @@ __device__ void merge_group(const uint32_t* S, int64_t ld, uint32_t wc, const Ar
 }
 
 template <class Ar>
-__global__ __launch_bounds__(RT) void rrp_pivot_kernel(const uint32_t* S, int64_t ld, LState* st, uint32_t wc, Ar ar,
-                                                       uint32_t* P, uint32_t* J, uint32_t* R, const uint32_t* rows_orig,
-                                                       uint32_t* rows_orig_next, uint32_t* Wg, uint32_t* cand0,
-                                                       uint32_t* cnt0, uint32_t* cand1, uint32_t* cnt1, uint32_t nchunk) {
+struct PivotArgs {
+    const uint32_t* S;
+    int64_t ld;
+    LState* st;
+    uint32_t wc;
+    Ar ar;
+    uint32_t *P, *J, *R;
+    const uint32_t* rows_orig;
+    uint32_t *rows_orig_next, *Wg, *cand0, *cnt0, *cand1, *cnt1;
+    uint32_t nchunk;                         // blocks of the search (0: no panel)
+};
+
+template <class Ar>
+__device__ void pivot_block(const PivotArgs<Ar>& pv) {
+    const uint32_t* S = pv.S;
+    const int64_t ld = pv.ld;
+    LState* st = pv.st;
+    const uint32_t wc = pv.wc, nchunk = pv.nchunk;
+    const Ar& ar = pv.ar;
+    uint32_t *P = pv.P, *J = pv.J, *R = pv.R;
+    const uint32_t* rows_orig = pv.rows_orig;
+    uint32_t *rows_orig_next = pv.rows_orig_next, *Wg = pv.Wg, *cand0 = pv.cand0, *cnt0 = pv.cnt0, *cand1 = pv.cand1,
+             *cnt1 = pv.cnt1;
     __shared__ uint32_t pool[MG_LDS > CH_LDS ? MG_LDS : CH_LDS];
     __shared__ uint32_t s_u[LW], s_q[LW], s_res[3];
     __shared__ uint32_t s_last;
-    // the panel chain (pivot search, X, the next panel's columns) is the critical path: its waves
-    // take issue priority over the wide trailing update running beside them on the other stream
-    __builtin_amdgcn_s_setprio(2);
     unsigned t_panel = 0;
 #ifdef HX_PANEL_TIMERS
     __shared__ unsigned s_tp;
@@ -471,7 +487,7 @@ __global__ __launch_bounds__(RT) void rrp_pivot_kernel(const uint32_t* S, int64_
     HX_TMARK(7);
     if (threadIdx.x == 0) {
         const uint32_t n = __hip_atomic_fetch_add(&st->arrive, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = n + 1 == gridDim.x ? 1u : 0u;
+        s_last = n + 1 == nchunk ? 1u : 0u;
     }
     __syncthreads();
     if (!s_last) return;
@@ -516,12 +532,9 @@ __global__ __launch_bounds__(RT) void rrp_pivot_kernel(const uint32_t* S, int64_
 // sum_{q<k} A[a_rows[i], a_cols[q]] X[q, j] mod p.  A's entries are split into L balanced 8-bit
 // limbs on the fly; X's limb planes come from panel_x (plane s, column j: 32 k-bytes).  One wave per
 // 32-row block and ucb consecutive 32-column blocks: the row block's A fragment (gathered, split)
-// and its Cin row indices are loaded once and serve every column block.  Per column block the X
-// fragments are loaded before the Cin entries (so the MFMAs wait for the first only), and the L^2
-// limb products of the one 32-deep k-step are taken one anti-diagonal at a time: each diagonal's
-// int32 sum is folded into an int64 accumulator at once (sum_d D_d w_d, exact: below 2^63, the
-// recombination of hx_limbs.h in another order), so 16 accumulator words serve all 2L - 1
-// diagonals and more waves fit a SIMD.  Every output is written, also when k = 0 (Cout = Cin: the
+// is loaded once and serves every column block, its Cin row indices wait in the wave's own LDS words.  Per
+// column block the X fragments are loaded before the Cin entries, so the MFMAs wait for the first only; the
+// reduction is limb_small_product's.  Every output is written, also when k = 0 (Cout = Cin: the
 // trailing update doubles as the compaction into the next Schur complement).  No barriers: a wave
 // past the rows returns at once.
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -530,7 +543,6 @@ constexpr uint32_t UPD_UCB = 4;          // column blocks per wave of the wide p
 struct UpdArgs {
     uint32_t m, n;                           // row bound (m_dev caps it) and columns
     uint32_t ucb;                            // 32-column blocks per wave
-    uint32_t chain;                          // 1: on the panel chain (issue priority)
     const uint32_t* m_dev;
     const uint32_t* k_dev;                   // k <= 32
     const uint32_t* A;
@@ -549,14 +561,13 @@ struct UpdArgs {
     uint32_t half;
 };
 
-template <int L>
-__global__ __launch_bounds__(256) void upd32_kernel(UpdArgs u) {
-    if (u.chain) __builtin_amdgcn_s_setprio(2);     // the next panel's columns: on the panel chain
+template <int L, int WAVES>
+__device__ __forceinline__ void upd_block(const UpdArgs& u, uint32_t blk, uint32_t (*s_row)[32]) {
     const uint32_t m = min(*u.m_dev, u.m), k = min(*u.k_dev, 32u);
     if (k == 0 && u.Cin == u.Cout && u.c_rows == nullptr && u.cirs == u.cors) return;   // in place, nothing to do
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 31, lg = lane >> 5;
     const uint32_t ncg = (u.n + 32 * u.ucb - 1) / (32 * u.ucb);
-    const uint32_t b0 = ((blockIdx.x / ncg) * 4 + wave) * 32, cg = blockIdx.x % ncg;
+    const uint32_t b0 = ((blk / ncg) * WAVES + wave) * 32, cg = blk % ncg;
     if (b0 >= m) return;                     // (k = 0 still copies Cin to Cout: the compaction)
     const uint32_t p = u.M.p;
     // A fragment: row b0 + lr, k-bytes 16 lg .. 16 lg + 15, all loads first
@@ -569,13 +580,9 @@ __global__ __launch_bounds__(256) void upd32_kernel(UpdArgs u) {
         const uint32_t t = 16 * lg + i;
         av[i] = (alive && t < k) ? u.A[aoff + (u.a_cols ? (int64_t)u.a_cols[t] : (int64_t)t)] : 0u;
     }
-    // the Cin rows of this lane's 16 outputs (accumulator element e: row b0 + (e / 4) 8 + 4 lg + e % 4)
-    uint32_t crow[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const uint32_t r = b0 + (e / 4) * 8 + lg * 4 + (e % 4);
-        crow[e] = r < m ? (u.c_rows ? u.c_rows[r] : r) : 0u;
-    }
+    // the Cin rows of the wave's 32 rows (accumulator element e: row b0 + (e / 4) 8 + 4 lg + e % 4)
+    if (lane < 32) s_row[wave][lane] = b0 + lane < m ? (u.c_rows ? u.c_rows[b0 + lane] : b0 + lane) : 0u;
+    __builtin_amdgcn_wave_barrier();
     v4i fa[1][L];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -591,12 +598,9 @@ __global__ __launch_bounds__(256) void upd32_kernel(UpdArgs u) {
         if (jb >= u.n) break;
         const uint32_t j = jb + lr;
         const bool jok = j < u.n;
-        // the row addresses are rebuilt per column block from 32-bit row indices (kept opaque), not
-        // hoisted as 32 pointers for the whole loop: fewer registers, more waves per SIMD
-#pragma unroll
-        for (int e = 0; e < 16; ++e) asm volatile("" : "+v"(crow[e]));
-        uint32_t obase = b0 + lg * 4;
-        asm volatile("" : "+v"(obase));
+        // (kept opaque: the row addresses are rebuilt per column block, not hoisted as 32 pointers)
+        uint32_t obase = b0 + lg * 4, srow = lg * 4;
+        asm volatile("" : "+v"(obase), "+v"(srow));
         v4i fb[1][L];
 #pragma unroll
         for (int s2 = 0; s2 < L; ++s2)
@@ -606,7 +610,7 @@ __global__ __launch_bounds__(256) void upd32_kernel(UpdArgs u) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const uint32_t r = obase + (e / 4) * 8 + (e % 4);
-            cv[e] = (jok && r < m) ? u.Cin[(int64_t)crow[e] * u.cirs + j] : 0u;
+            cv[e] = (jok && r < m) ? u.Cin[(int64_t)s_row[wave][srow + (e / 4) * 8 + (e % 4)] * u.cirs + j] : 0u;
         }
         uint32_t x[16];
         limb_small_product<L, 1>(fa, fb, sc, x);
@@ -620,6 +624,29 @@ __global__ __launch_bounds__(256) void upd32_kernel(UpdArgs u) {
     }
 }
 
+template <int L>
+__global__ __launch_bounds__(256) void upd32_kernel(UpdArgs u) {
+    __shared__ __attribute__((aligned(16))) uint32_t s_row[4][32];
+    upd_block<L, 4>(u, blockIdx.x, s_row);
+}
+
+// One launch beside each other: the pivot search of a panel (the first pv.nchunk blocks), the rest of the previous
+// panel's trailing update (the next nrest), and its Gauss-Jordan product.  The search reads only its panel's
+// columns, which were updated before; nothing the three write is read by another.  In one launch because the
+// markers between the streams they would need cost more than the products: 84 us per panel at 4096^2 with the
+// products on two side streams, of it 24 us hand-overs; STEP_FIGURE.
+template <class Ar, int L>
+__global__ __launch_bounds__(RT) void rrp_step_kernel(PivotArgs<Ar> pv, UpdArgs rest, UpdArgs gj, uint32_t nrest) {
+    if (blockIdx.x < pv.nchunk) {
+        pivot_block(pv);
+        return;
+    }
+    __shared__ __attribute__((aligned(16))) uint32_t s_row[RT / 64][32];
+    const uint32_t b = blockIdx.x - pv.nchunk;
+    if (b < nrest) upd_block<L, RT / 64>(rest, b, s_row);
+    else upd_block<L, RT / 64>(gj, b - nrest, s_row);
+}
+
 // X[:, slab] = S[P, J]^{-1} S[P, slab]; also the pivots / pivot rows of this panel (block 0).
 // Every workgroup reduces the same k x k pivot block beside its own SL-column slab: narrow slabs
 // spread the (multiply-latency-bound) elimination over many CUs.
@@ -631,10 +658,9 @@ __global__ __launch_bounds__(PXT) void panel_x_kernel(const uint32_t* S, int64_t
                                                      uint32_t* U, int64_t ldu, uint32_t c, const uint32_t* rows_orig,
                                                      uint32_t* pivots, uint32_t* pivot_rows, uint8_t* Xp,
                                                      uint32_t pstride, uint32_t L, uint32_t half, int slot,
-                                                     const uint32_t* Wg) {
+                                                     const uint32_t* Wg, uint32_t nslab, uint32_t* T) {
     __shared__ uint32_t B[LW * (LW + SL)];
     __shared__ uint32_t s_inv[LW], s_q[LW];
-    __builtin_amdgcn_s_setprio(2);                    // on the panel chain (see rrp_pivot_kernel)
     if (blockIdx.x == 0 && threadIdx.x == 0) {        // the sizes of this panel's products, slot i & 1
         st->snap_k[slot] = st->k;
         st->snap_m[slot] = st->m_new;
@@ -642,6 +668,16 @@ __global__ __launch_bounds__(PXT) void panel_x_kernel(const uint32_t* S, int64_t
     }
     const uint32_t k = st->k;
     if (k == 0) return;
+    if (blockIdx.x >= nslab) {
+        // T[t, q] = U[t, c + J[q]] for the pivot rows stored before the panel (the Gauss-Jordan product's left
+        // operand, gathered before that product overwrites it; zero past the panel's k pivots)
+        const uint32_t count = st->r * LW;
+        for (uint32_t idx = (blockIdx.x - nslab) * PXT + threadIdx.x; idx < count; idx += (gridDim.x - nslab) * PXT) {
+            const uint32_t t = idx / LW, q = idx % LW;
+            T[idx] = q < k ? U[(int64_t)t * ldu + c + J[q]] : 0u;
+        }
+        return;
+    }
     const uint32_t j0 = blockIdx.x * SL;
     if (j0 >= na) return;
     const uint32_t sw = min((uint32_t)SL, na - j0), bw = k + sw, p = ar.p;
@@ -764,46 +800,7 @@ __global__ void init_state_kernel(LState* st, uint32_t m, uint32_t* rows_orig, u
     for (size_t t = i; t < ucount; t += (size_t)gridDim.x * blockDim.x) U[t] = 0;
 }
 
-// T[t, q] = U[t, c + J[q]] for the r pivot rows stored before the panel (the Gauss-Jordan product's
-// left operand; zero past the panel's k pivots).
-__global__ void gj_gather_kernel(const uint32_t* U, int64_t ldu, uint32_t c, const uint32_t* J, const LState* st,
-                                 int slot, uint32_t* T) {
-    const uint32_t r = st->snap_r[slot], k = st->snap_k[slot];
-    for (uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x; idx < r * LW; idx += gridDim.x * blockDim.x) {
-        const uint32_t t = idx / LW, q = idx % LW;
-        T[idx] = q < k ? U[(int64_t)t * ldu + c + J[q]] : 0u;
-    }
-}
-
 inline uint32_t gsz(uint64_t n) { return (uint32_t)std::min<uint64_t>((n + 255) / 256, 65536); }
-
-// A second stream and two events for the lookahead, per calling stream (created once, reused by
-// every elimination issued on that stream, so a call allocates nothing and can be captured).
-// The streams beside the caller's (non-blocking, created once per caller stream): s2 takes the wide
-// trailing updates, s3 the Gauss-Jordan gathers and products, sc the panel chain when the caller's
-// stream is the legacy null stream.  (A CU-masked queue for s2, which leaves CUs free for the chain,
-// was measured: 3 % faster alone, but a masked stream is a blocking one, so every launch on it waits
-// for the null stream, and when the null stream shares a hardware queue with another side stream the
-// updates serialise behind it -- 16.3 ms instead of 10 for C2 once other streams existed.)
-struct SideStream {
-    hipStream_t s2 = nullptr, s3 = nullptr, sc = nullptr;
-    hipEvent_t ev_x = nullptr, ev_rest = nullptr, ev_gj[2] = {nullptr, nullptr}, ev_fork = nullptr,
-               ev_join = nullptr;
-};
-SideStream side_for(hipStream_t s) {
-    static std::mutex mu;
-    static std::unordered_map<hipStream_t, SideStream> map;
-    std::lock_guard<std::mutex> lk(mu);
-    SideStream& ss = map[s];
-    if (ss.sc == nullptr) {
-        HX_HIP(hipStreamCreateWithFlags(&ss.s2, hipStreamNonBlocking));
-        HX_HIP(hipStreamCreateWithFlags(&ss.s3, hipStreamNonBlocking));
-        HX_HIP(hipStreamCreateWithFlags(&ss.sc, hipStreamNonBlocking));
-        for (hipEvent_t* e : {&ss.ev_x, &ss.ev_rest, &ss.ev_gj[0], &ss.ev_gj[1], &ss.ev_fork, &ss.ev_join})
-            HX_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
-    }
-    return ss;
-}
 
 // The results on the device: rank = r (0xffffffff when a pivot had no inverse), pivots, pivot rows.
 __global__ void finish_kernel(const LState* st, const uint32_t* piv, const uint32_t* prow, uint32_t mn, uint32_t* d_rank,
@@ -872,7 +869,7 @@ size_t large_state_offset_words(uint32_t m, uint32_t n) {
 template <class Ar>
 void enqueue_large(const hx_modctx& ctx, const Ar& ar, uint32_t m, uint32_t n, const uint32_t* A, int64_t lda,
                    uint32_t* Rout, int64_t ldr, uint32_t* d_rank, uint32_t* d_piv, uint32_t* d_prow, uint32_t* base,
-                   hipStream_t s, const SideStream& side) {
+                   hipStream_t s) {
     const uint32_t mn = std::min(m, n);
     const uint32_t nchunk = (m + CH - 1) / CH;
     const std::vector<size_t> sizes = large_sizes(m, n);
@@ -894,15 +891,15 @@ void enqueue_large(const hx_modctx& ctx, const Ar& ar, uint32_t m, uint32_t n, c
     const DevMod dm = devmod(ctx);
     uint64_t n_upd = 0;
     const uint64_t launches0 = stat_value(ST_KERNELS);
-    auto upd = [&](const UpdArgs& u, hipStream_t st_) {
+    auto upd = [&](const UpdArgs& u) {
         const uint32_t grid = (u.m + 127) / 128 * ((u.n + 32 * u.ucb - 1) / (32 * u.ucb));
         if (grid == 0) return;
         ++n_upd;
         switch (L) {
-            case 1: upd32_kernel<1><<<grid, 256, 0, st_>>>(u); break;
-            case 2: upd32_kernel<2><<<grid, 256, 0, st_>>>(u); break;
-            case 3: upd32_kernel<3><<<grid, 256, 0, st_>>>(u); break;
-            default: upd32_kernel<4><<<grid, 256, 0, st_>>>(u); break;
+            case 1: upd32_kernel<1><<<grid, 256, 0, s>>>(u); break;
+            case 2: upd32_kernel<2><<<grid, 256, 0, s>>>(u); break;
+            case 3: upd32_kernel<3><<<grid, 256, 0, s>>>(u); break;
+            default: upd32_kernel<4><<<grid, 256, 0, s>>>(u); break;
         }
         after_launch("upd32_kernel");
     };
@@ -912,20 +909,33 @@ void enqueue_large(const hx_modctx& ctx, const Ar& ar, uint32_t m, uint32_t n, c
     uint32_t* cnt[2] = {at(9), at(10)};
     uint32_t *Pb = at(11), *Jb = at(12), *piv = at(13), *prow = at(14);
     LState* st = (LState*)at(WS_STATE);
-    // lookahead: the trailing update of panel i is split into the next panel's LW columns (on the
-    // chain's stream) and the rest (on s2, overlapping panel i+1's pivot search); the Gauss-Jordan
-    // gather and product run on s3.  Panel i+1's X waits for s2 (its rows are read whole); panel
-    // i+2, which reuses panel i's slot (P, J, X, its limb planes, the sizes), waits for s3.
-    hipStream_t sc = s == nullptr ? side.sc : s;            // the panel chain
-    hipStream_t s2 = side.s2, s3 = side.s3;
-    if (sc != s) {
-        HX_HIP(hipEventRecord(side.ev_fork, s));
-        HX_HIP(hipStreamWaitEvent(sc, side.ev_fork, 0));
-    }
-    bool rest_pending = false, gj_pending[2] = {false, false};
+    // Three launches per panel, all on the caller's stream: the step kernel (this panel's pivot search beside the
+    // previous panel's trailing update and Gauss-Jordan product), X (and the gather of the Gauss-Jordan product's
+    // left operand), and the next panel's columns of the trailing update, which its search reads.
+    UpdArgs rest{}, gj{};
+    uint32_t nrest = 0, ngj = 0;                            // blocks of the products still to run
+    auto blocks = [&](UpdArgs& u) {
+        // column blocks per wave: fewer where the launch would leave compute units idle
+        auto grid = [&] { return (u.m + 32 * (RT / 64) - 1) / (32 * (RT / 64)) * ((u.n + 32 * u.ucb - 1) / (32 * u.ucb)); };
+        for (u.ucb = UPD_UCB; u.ucb > 1 && grid() < 192; u.ucb /= 2) {}
+        ++n_upd;
+        return grid();
+    };
+    auto step = [&](const PivotArgs<Ar>& pv) {
+        const uint32_t grid = pv.nchunk + nrest + ngj;
+        if (grid == 0) return;
+        switch (L) {
+            case 1: rrp_step_kernel<Ar, 1><<<grid, RT, 0, s>>>(pv, rest, gj, nrest); break;
+            case 2: rrp_step_kernel<Ar, 2><<<grid, RT, 0, s>>>(pv, rest, gj, nrest); break;
+            case 3: rrp_step_kernel<Ar, 3><<<grid, RT, 0, s>>>(pv, rest, gj, nrest); break;
+            default: rrp_step_kernel<Ar, 4><<<grid, RT, 0, s>>>(pv, rest, gj, nrest); break;
+        }
+        after_launch("rrp_step_kernel");
+        nrest = ngj = 0;
+    };
     {
-        HX_HIP(hipMemcpy2DAsync(Sb[0], (size_t)n * 4, A, (size_t)lda * 4, (size_t)n * 4, m, hipMemcpyDeviceToDevice, sc));
-        init_state_kernel<<<gsz(std::max<size_t>(m, (size_t)mn * n)), 256, 0, sc>>>(st, m, ro[0], U, (size_t)mn * n);
+        HX_HIP(hipMemcpy2DAsync(Sb[0], (size_t)n * 4, A, (size_t)lda * 4, (size_t)n * 4, m, hipMemcpyDeviceToDevice, s));
+        init_state_kernel<<<gsz(std::max<size_t>(m, (size_t)mn * n)), 256, 0, s>>>(st, m, ro[0], U, (size_t)mn * n);
         after_launch("init_state_kernel");
         int cur = 0;
         for (uint32_t c = 0, panel = 0; c < n; c += LW, ++panel) {
@@ -937,125 +947,82 @@ void enqueue_large(const hx_modctx& ctx, const Ar& ar, uint32_t m, uint32_t n, c
             uint32_t* X = Xb + (size_t)slot * LW * n;
             uint8_t* Xp = Xpb + (size_t)slot * 4 * pstride;
             uint32_t* Rl = Rlb + (size_t)slot * m;
-            // panel i - 2's Gauss-Jordan product still reads this slot's J, X, planes and sizes
-            if (gj_pending[slot]) {
-                HX_HIP(hipStreamWaitEvent(sc, side.ev_gj[slot], 0));
-                gj_pending[slot] = false;
-            }
             // 1. the pivot search (reads only this panel's LW columns, already up to date): the search
             //    over the first SPR rows, which settles most panels alone, else the tournament
-            rrp_pivot_kernel<Ar><<<nchunk, RT, 0, sc>>>(S, n, st, wc, ar, P, J, Rl, ro[cur], ro[cur ^ 1], Wg, cand[0],
-                                                        cnt[0], cand[1], cnt[1], nchunk);
-            after_launch("rrp_pivot_kernel");
-            // the previous panel's update must be complete before its rows are read whole
-            if (rest_pending) {
-                HX_HIP(hipStreamWaitEvent(sc, side.ev_rest, 0));
-                rest_pending = false;
-            }
-            // 2. X = S[P,J]^{-1} S[P,:] into the U store and the contiguous copy
-            panel_x_kernel<Ar><<<(na + SL - 1) / SL, PXT, 0, sc>>>(S, n, na, P, J, st, ar, X, n, U, n, c, ro[cur], piv,
-                                                                   prow, Xp, pstride, L, half, slot, Wg);
+            step(PivotArgs<Ar>{S, (int64_t)n, st, wc, ar, P, J, Rl, ro[cur], ro[cur ^ 1], Wg, cand[0], cnt[0], cand[1],
+                               cnt[1], nchunk});
+            // 2. X = S[P,J]^{-1} S[P,:] into the U store and the contiguous copy; the Gauss-Jordan product has at
+            //    most min(c, mn) stored pivot rows, and is not needed when only the rank, pivots and pivot rows
+            //    are asked for
+            const uint32_t rmax = Rout ? std::min<uint32_t>(c, mn) : 0u;
+            const uint32_t nslab = (na + SL - 1) / SL, ngather = std::min<uint32_t>(64, (rmax * LW + 4 * PXT - 1) / (4 * PXT));
+            panel_x_kernel<Ar><<<nslab + ngather, PXT, 0, s>>>(S, n, na, P, J, st, ar, X, n, U, n, c, ro[cur], piv, prow,
+                                                               Xp, pstride, L, half, slot, Wg, nslab, T);
             after_launch("panel_x_kernel");
-            // 3. the next Schur complement, compacted: first the next panel's columns, then the rest.  The
-            //    other streams start after the next panel's columns (no marker between the chain's kernels)
-            bool x_marked = false;
-            auto mark_x = [&] {
-                if (!x_marked) HX_HIP(hipEventRecord(side.ev_x, sc));   // X, the row list and the sizes are ready
-                x_marked = true;
-            };
+            UpdArgs u{};
+            u.k_dev = &st->snap_k[slot];
+            u.planes = Xp;
+            u.pstride = pstride;
+            u.cirs = n;
+            u.cors = n;
+            u.M = dm;
+            u.inv = inv;
+            u.half = half;
+            // 3. the next Schur complement, compacted: the next panel's columns now, the rest in the next step
             if (na > wc) {
                 const uint32_t nt = na - wc, n1 = std::min<uint32_t>(LW, nt);
                 // S'[i, j] = S[R_i, wc + j] - sum_t S[R_i, J_t] X[t, wc + j] on the matrix cores
-                UpdArgs u;
                 u.m = m;
                 u.m_dev = &st->snap_m[slot];
-                u.k_dev = &st->snap_k[slot];
                 u.A = S;
                 u.ars = n;
                 u.a_rows = Rl;
                 u.a_cols = J;
-                u.planes = Xp;
-                u.pstride = pstride;
                 u.Cin = S + wc;
-                u.cirs = n;
                 u.c_rows = Rl;
-                u.cors = n;
-                u.M = dm;
-                u.inv = inv;
-                u.half = half;
                 u.n = n1;
                 u.ucb = 1;
-                u.chain = 1;
                 u.pcol0 = wc;
                 u.Cout = Sb[cur ^ 1];
-                upd(u, sc);
+                upd(u);
                 if (nt > n1) {
-                    mark_x();
-                    HX_HIP(hipStreamWaitEvent(s2, side.ev_x, 0));
-                    u.n = nt - n1;
-                    u.ucb = UPD_UCB;
-                    u.chain = 0;
-                    u.pcol0 = wc + n1;
-                    u.Cin = S + wc + n1;
-                    u.Cout = Sb[cur ^ 1] + n1;
-                    upd(u, s2);
-                    HX_HIP(hipEventRecord(side.ev_rest, s2));
-                    rest_pending = true;
+                    rest = u;
+                    rest.n = nt - n1;
+                    rest.pcol0 = wc + n1;
+                    rest.Cin = S + wc + n1;
+                    rest.Cout = Sb[cur ^ 1] + n1;
+                    nrest = blocks(rest);
                 }
                 cur ^= 1;
             }
-            // 4. Gauss-Jordan on the stored pivot rows (at most min(c, mn) of them), on s3; not needed
-            //    when only the rank, pivots and pivot rows are asked for
-            const uint32_t rmax = Rout ? std::min<uint32_t>(c, mn) : 0u;
+            // 4. Gauss-Jordan on the stored pivot rows: U[0:r, c + j] -= sum_t T[., t] X[t, j], in place
             if (rmax > 0) {
-                mark_x();
-                HX_HIP(hipStreamWaitEvent(s3, side.ev_x, 0));
-                gj_gather_kernel<<<gsz((uint64_t)rmax * LW), 256, 0, s3>>>(U, n, c, J, st, slot, T);
-                after_launch("gj_gather_kernel");
-                // U[0:r, c + j] -= sum_t T[., t] X[t, j] on the matrix cores (in place)
-                UpdArgs u;
-                u.m = rmax;
-                u.n = na;
-                u.ucb = UPD_UCB;
-                u.chain = 0;
-                u.m_dev = &st->snap_r[slot];
-                u.k_dev = &st->snap_k[slot];
-                u.A = T;
-                u.ars = LW;
-                u.a_rows = nullptr;
-                u.a_cols = nullptr;
-                u.planes = Xp;
-                u.pstride = pstride;
-                u.pcol0 = 0;
-                u.Cin = U + c;
-                u.cirs = n;
-                u.c_rows = nullptr;
-                u.Cout = U + c;
-                u.cors = n;
-                u.M = dm;
-                u.inv = inv;
-                u.half = half;
-                upd(u, s3);
-                HX_HIP(hipEventRecord(side.ev_gj[slot], s3));
-                gj_pending[slot] = true;
+                gj = u;
+                gj.m = rmax;
+                gj.n = na;
+                gj.m_dev = &st->snap_r[slot];
+                gj.A = T;
+                gj.ars = LW;
+                gj.a_rows = nullptr;
+                gj.a_cols = nullptr;
+                gj.pcol0 = 0;
+                gj.Cin = U + c;
+                gj.c_rows = nullptr;
+                gj.Cout = U + c;
+                ngj = blocks(gj);
             }
         }
-        advance_kernel<<<1, 64, 0, sc>>>(st);           // past the last panel (the pivot search does it for the others)
+        PivotArgs<Ar> none{};
+        none.ar = ar;
+        step(none);                                         // the last panel's products
+        advance_kernel<<<1, 64, 0, s>>>(st);                // past the last panel (the pivot search does it for the others)
         after_launch("advance_kernel");
-        // every product on s2 and s3 (the last Gauss-Jordan product included) before U is read
-        if (rest_pending) HX_HIP(hipStreamWaitEvent(sc, side.ev_rest, 0));
-        for (int sl = 0; sl < 2; ++sl)
-            if (gj_pending[sl]) HX_HIP(hipStreamWaitEvent(sc, side.ev_gj[sl], 0));
         // the results, on the device: rank (0xffffffff when a pivot had no inverse), pivots, pivot rows, R
-        finish_kernel<<<gsz(std::max<uint32_t>(mn, 1)), 256, 0, sc>>>(st, piv, prow, mn, d_rank, d_piv, d_prow);
+        finish_kernel<<<gsz(std::max<uint32_t>(mn, 1)), 256, 0, s>>>(st, piv, prow, mn, d_rank, d_piv, d_prow);
         after_launch("finish_kernel");
         if (Rout) {
-            rref_out_dev_kernel<<<gsz((uint64_t)m * n), 256, 0, sc>>>(U, n, st, m, Rout, ldr);
+            rref_out_dev_kernel<<<gsz((uint64_t)m * n), 256, 0, s>>>(U, n, st, m, Rout, ldr);
             after_launch("rref_out_dev_kernel");
-        }
-        if (sc != s) {
-            HX_HIP(hipEventRecord(side.ev_join, sc));
-            HX_HIP(hipStreamWaitEvent(s, side.ev_join, 0));
         }
     }
     elim_stat_add(EL_CALLS, 1);
@@ -1078,11 +1045,10 @@ void rref_large_enqueue(const hx_modctx& ctx, uint32_t m, uint32_t n, const uint
                         hipStream_t s) {
     HX_CHECK(ws != nullptr && ws_bytes >= rref_large_workspace_bytes(m, n), "rref: workspace too small");
     HX_CHECK(d_rank != nullptr, "rref: rank is NULL");
-    const SideStream side = side_for(s);
     if (ctx.p & 1u)
-        enqueue_large(ctx, make_mont(ctx.p), m, n, A, lda, R, ldr, d_rank, d_piv, d_prow, (uint32_t*)ws, s, side);
+        enqueue_large(ctx, make_mont(ctx.p), m, n, A, lda, R, ldr, d_rank, d_piv, d_prow, (uint32_t*)ws, s);
     else
-        enqueue_large(ctx, make_barrett(ctx.p), m, n, A, lda, R, ldr, d_rank, d_piv, d_prow, (uint32_t*)ws, s, side);
+        enqueue_large(ctx, make_barrett(ctx.p), m, n, A, lda, R, ldr, d_rank, d_piv, d_prow, (uint32_t*)ws, s);
 }
 
 bool rref_large(const hx_modctx& ctx, uint32_t m, uint32_t n, const uint32_t* A, int64_t lda, uint32_t* R,
