@@ -1,7 +1,7 @@
 // hx_howell.hip -- the Howell form over Z/2^k (1 <= k <= 32) of many uneven matrices in ONE
 // persistent launch (ring2k::howell, Binary/Ring2k.h:959-969; ENGINE_API.md Sec. 13.5).
 //
-// One 256-thread workgroup per job, jobs pulled from an atomic counter (largest first).  Per job the
+// One workgroup per job (256 to 1024 threads by its size), jobs pulled from an atomic counter (largest first).  Per job the
 // Sec. 13.5 pass runs on the rows of A (copied into the job's work rows), in native u32 wraparound
 // (Z/2^k is the quotient of Z/2^32, Ring2k.h:17-22; only valuations, zero tests and the output look
 // at the value mod 2^k):
@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <mutex>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "hx_common.h"
@@ -45,16 +46,21 @@ struct HArgs {
 };
 
 __device__ __forceinline__ uint32_t inv_odd(uint32_t u) {
-    uint32_t x = u;   // u * u == 1 mod 8: 3 correct bits, each Newton step doubles them
+    uint32_t x = (3u * u) ^ 2u;   // right to 5 bits; each Newton step doubles them
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x = x * (2u - u * x);
+    for (int i = 0; i < 3; ++i) x = x * (2u - u * x);
     return x;
 }
 
+// The wave's minimum in every lane: inside the rows of 16 lanes by DPP moves, then the four rows' through scalars.
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x = min(x, (uint32_t)__shfl_xor((int)x, off));
-    return x;
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0xB1, 0xf, 0xf, false));    // quad [1, 0, 3, 2]
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x4E, 0xf, 0xf, false));    // quad [2, 3, 0, 1]
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x141, 0xf, 0xf, false));   // half-row mirror
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x140, 0xf, 0xf, false));   // row mirror
+    const uint32_t a = __builtin_amdgcn_readlane((int)x, 0), b = __builtin_amdgcn_readlane((int)x, 16);
+    const uint32_t c = __builtin_amdgcn_readlane((int)x, 32), d = __builtin_amdgcn_readlane((int)x, 48);
+    return min(min(a, b), min(c, d));
 }
 
 __device__ void howell_one(const HJob& job, uint32_t k) {
@@ -169,14 +175,15 @@ __device__ void howell_one(const HJob& job, uint32_t k) {
 // ------------------------------------------------------------------------------------------
 constexpr uint32_t HW = 16;            // panel width / reduce-above block
 constexpr uint32_t kBlockedRows = 1024;
+constexpr uint32_t HCOL = 256;         // trailing columns per sweep (four per lane)
 constexpr uint32_t NONE = 0xffffffffu;
 
 // Panel entries and multipliers are stored in elements of `eb` bytes: 2 when k <= 16 (every stored
 // value is reduced mod 2^k), else 4; the halved store lets the largest job class (m + n <= 1024)
-// run two workgroups per CU.  The panel region holds at least HW x HT words: during the trailing
-// sweep it holds the panel's pivot rows over HT columns instead (the panel entries are dead then).
+// run two workgroups per CU.  The panel region holds at least HW x HCOL words: during the trailing
+// sweep it holds the panel's pivot rows over HCOL columns instead (the panel entries are dead then).
 __host__ __device__ constexpr uint32_t pan_rows(uint32_t rc, uint32_t eb) {
-    return rc * eb >= HT * 4u ? rc : HT * 4u / eb;
+    return rc * eb >= HCOL * 4u ? rc : HCOL * 4u / eb;
 }
 __host__ __device__ constexpr size_t blocked_lds_bytes(uint32_t rc, uint32_t eb) {
     return (size_t)pan_rows(rc, eb) * HW * eb + (size_t)rc * HW * eb + (size_t)rc * 4 * 2 + rc;
@@ -191,11 +198,13 @@ __device__ __forceinline__ uint32_t kmul(uint32_t a, uint32_t b) {
     else return a * b;
 }
 
-template <bool SMALLK, class PT>
+// RPT: active positions per thread (RPT NT >= the class's rows).
+template <bool SMALLK, class PT, int NT, int RPT>
 __device__ void howell_blocked(const HJob& job, uint32_t k, uint32_t rc, uint32_t* lds) {
-    __shared__ uint32_t s_red[2][HT / 64];
+    constexpr int NW = NT / 64, UC = 2, NC = HCOL / (64 * UC), GR = 4;   // sweep: columns per lane, column groups, rows
+    __shared__ __attribute__((aligned(16))) uint32_t s_red[2][NW];
     __shared__ uint32_t s_pid[HW], s_ui[HW], s_v[HW], s_c[HW];
-    __shared__ uint32_t s_hb[HW * HW];
+    __shared__ __attribute__((aligned(16))) uint32_t s_hb[HW * HW];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t m = job.m, n = job.n;
     const uint32_t mask = k >= 32 ? 0xffffffffu : ((1u << k) - 1u);
@@ -204,14 +213,90 @@ __device__ void howell_blocked(const HJob& job, uint32_t k, uint32_t rc, uint32_
         return;
     }
     PT* pan = (PT*)lds;                        // [rc][HW] panel entries of active rows
-    uint32_t* s_T = lds;                       // [HW][HT] the panel's pivot rows over HT trailing columns
+    uint32_t* s_T = lds;                       // [HW][HCOL] the panel's pivot rows over HCOL trailing columns
                                                // (phase B only, when the panel entries are dead)
     PT* qm = pan + (size_t)pan_rows(rc, sizeof(PT)) * HW;   // [rc][HW] multipliers (later: reduce-above q's)
     uint32_t* act = (uint32_t*)(qm + (size_t)rc * HW);     // active order: row ids, NONE once chosen
     uint32_t* prow = act + rc;                 // pivot row ids in pivot order
     uint8_t* nz = (uint8_t*)(prow + rc);       // row has a non-zero multiplier in this panel
     uint32_t* rows = job.work;                 // row id i at rows + i * n
-    for (uint32_t i = wave; i < m; i += HT / 64) {     // a wave per row, four words per lane in flight
+    // a row's panel entries or multipliers, 16 bytes at a time (rows are 32- or 64-byte aligned)
+    auto get = [](const PT* p, auto& x, auto count) {
+        constexpr int N = decltype(count)::value, V = 16 / sizeof(PT);
+#pragma unroll
+        for (int g = 0; g < N / V; ++g) {
+            const uint4 q = ((const uint4*)p)[g];
+            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+            for (int e = 0; e < V; ++e) x[V * g + e] = V == 4 ? w[e] : (w[e / 2] >> (16 * (e % 2))) & 0xffffu;
+        }
+    };
+    auto put = [](PT* p, const uint32_t (&x)[HW]) {
+        constexpr int V = 16 / sizeof(PT);
+#pragma unroll
+        for (int g = 0; g < (int)HW / V; ++g) {
+            uint32_t w[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = V == 4 ? x[4 * g + e] : x[8 * g + (2 * e) % HW] | x[8 * g + (2 * e + 1) % HW] << 16;
+            ((uint4*)p)[g] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    };
+    using N16 = std::integral_constant<int, (int)HW>;
+    // rows[id][j] -= sum_t q[id][t] s_T[t][j - j0] for the columns j0 .. j0 + HCOL and the rows id_of(pos) (NONE: no
+    // row), masked by `keep`.  A wave takes 64 UC columns (64 apart per lane: coalesced) and every NW / NC-th group of
+    // GR rows; the next group's ids and entries are loaded before this group's are written back (different rows).
+    auto sweep = [&](uint32_t* base, uint32_t j0, uint32_t npos, auto id_of, uint32_t keep) {
+        const uint32_t c0 = (wave % NC) * (64 * UC) + lane;
+        uint32_t Tr[HW][UC];
+#pragma unroll
+        for (uint32_t t = 0; t < HW; ++t)
+#pragma unroll
+            for (int u = 0; u < UC; ++u) Tr[t][u] = s_T[t * HCOL + c0 + 64 * u];
+        bool in[UC];
+#pragma unroll
+        for (int u = 0; u < UC; ++u) in[u] = j0 + c0 + 64 * u < n;
+        if (j0 + (wave % NC) * (64 * UC) >= n) return;           // (whole waves; no barrier inside)
+        uint32_t ids[GR], xs[GR][UC];
+        auto load_group = [&](uint32_t pos, uint32_t (&gid)[GR], uint32_t (&gx)[GR][UC]) {
+#pragma unroll
+            for (int r = 0; r < GR; ++r) gid[r] = pos + r < npos ? id_of(pos + r) : NONE;
+#pragma unroll
+            for (int r = 0; r < GR; ++r)
+#pragma unroll
+                for (int u = 0; u < UC; ++u)
+                    gx[r][u] = (gid[r] != NONE && in[u]) ? base[(size_t)gid[r] * n + j0 + c0 + 64 * u] : 0u;
+        };
+        constexpr uint32_t STEP = GR * (NW / NC);
+        uint32_t pos = wave / NC * GR;
+        if (pos < npos) load_group(pos, ids, xs);
+        for (; pos < npos; pos += STEP) {
+            uint32_t nids[GR], nxs[GR][UC];
+            if (pos + STEP < npos) load_group(pos + STEP, nids, nxs);
+#pragma unroll
+            for (int r = 0; r < GR; ++r) {
+                if (ids[r] == NONE) continue;
+                uint32_t q[HW];
+                get(qm + (size_t)ids[r] * HW, q, N16{});
+#pragma unroll
+                for (int u = 0; u < UC; ++u) {
+                    if (!in[u]) continue;
+                    uint32_t x = xs[r][u];
+#pragma unroll
+                    for (uint32_t t = 0; t < HW; ++t) x -= kmul<SMALLK>(q[t], Tr[t][u]);
+                    base[(size_t)ids[r] * n + j0 + c0 + 64 * u] = x & keep;
+                }
+            }
+            if (pos + STEP < npos) {
+#pragma unroll
+                for (int r = 0; r < GR; ++r) {
+                    ids[r] = nids[r];
+#pragma unroll
+                    for (int u = 0; u < UC; ++u) xs[r][u] = nxs[r][u];
+                }
+            }
+        }
+    };
+    for (uint32_t i = wave; i < m; i += NW) {     // a wave per row, four words per lane in flight
         const uint32_t* Ai = job.A + (int64_t)i * job.lda;
         uint32_t* Ri = rows + (size_t)i * n;
         for (uint32_t j0 = lane; j0 < n; j0 += 256) {
@@ -223,12 +308,12 @@ __device__ void howell_blocked(const HJob& job, uint32_t k, uint32_t rc, uint32_
                 if (j0 + 64 * e < n) Ri[j0 + 64 * e] = v[e] & mask;
         }
     }
-    for (uint32_t i = tid; i < m; i += HT) act[i] = i;
+    for (uint32_t i = tid; i < m; i += NT) act[i] = i;
     __syncthreads();
     uint32_t na = m, h = 0, ncl = 0;
     for (uint32_t c0 = 0; c0 < n; c0 += HW) {
         const uint32_t wc = min(HW, n - c0), c1 = c0 + wc;
-        for (uint32_t idx = tid; idx < na * HW; idx += HT) {
+        for (uint32_t idx = tid; idx < na * HW; idx += NT) {
             const uint32_t pos = idx / HW, t = idx % HW, id = act[pos];
             if (id == NONE) continue;
             pan[id * HW + t] = t < wc ? rows[(size_t)id * n + c0 + t] & mask : 0u;
@@ -238,28 +323,38 @@ __device__ void howell_blocked(const HJob& job, uint32_t k, uint32_t rc, uint32_
         if (tid < HW) s_pid[tid] = NONE;
         const uint32_t ncl0 = ncl;
         __syncthreads();
-        // (A) the pass on the panel columns.  Row position pos belongs to thread pos % HT for the
-        // whole panel (scan, elimination, closure rows appended there, the chosen mark), and the
-        // pivot row is left unscaled (the eliminating multiplier is q u^-1 instead), so the only
-        // exchange per step is the pivot search: one barrier per step.
-        uint32_t chosen = 0;                                   // bit j: position tid + j HT picked
-        for (uint32_t t = 0; t < wc; ++t) {
+        // (A) the pass on the panel columns.  Position pos belongs to thread pos % NT for the whole panel: its
+        // entries stay in that thread's registers (a copy in LDS for the step that chooses the row), and the
+        // pivot row is left unscaled (the eliminating multiplier is q u^-1 instead), so the only exchange per
+        // step is the pivot search: one barrier per step.
+        uint32_t R[RPT][HW], id[RPT];
+        bool live[RPT], picked[RPT];
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+            const uint32_t pos = tid + j * NT;
+            id[j] = pos < na ? act[pos] : NONE;
+            live[j] = id[j] != NONE;
+            picked[j] = false;
+#pragma unroll
+            for (uint32_t e = 0; e < HW; ++e) R[j][e] = 0;
+            if (live[j]) get(pan + (size_t)id[j] * HW, R[j], N16{});
+        }
+        auto step = [&](const uint32_t t) {
             uint32_t best = NONE;
-            for (uint32_t pos = tid, j = 0; pos < na; pos += HT, ++j) {
-                const uint32_t id = act[pos];                  // NONE: chosen in an earlier panel
-                if (id == NONE || (chosen >> j & 1u)) continue;
-                const uint32_t x = pan[id * HW + t] & mask;
-                if (x != 0) best = min(best, ((uint32_t)__builtin_ctz(x) << 24) | pos);
-            }
+#pragma unroll
+            for (int j = 0; j < RPT; ++j)
+                if (live[j] && R[j][t] != 0) best = min(best, ((uint32_t)__builtin_ctz(R[j][t]) << 24) | (tid + j * NT));
             best = wave_min_u32(best);
             if (lane == 0) s_red[t & 1][wave] = best;
             __syncthreads();
-            best = min(min(s_red[t & 1][0], s_red[t & 1][1]), min(s_red[t & 1][2], s_red[t & 1][3]));
-            if (best == NONE) continue;
+            best = s_red[t & 1][0];
+#pragma unroll
+            for (int e = 1; e < NW; ++e) best = min(best, s_red[t & 1][e]);
+            if (best == NONE) return;                          // (uniform)
             const uint32_t bpos = best & 0xffffffu, v = best >> 24, pid = act[bpos];
-            const PT* P = pan + pid * HW;                      // unscaled: P[t] = u 2^v
-            const uint32_t ui = inv_odd((P[t] & mask) >> v) & mask;
-            if (bpos % HT == tid) chosen |= 1u << (bpos / HT);
+            uint32_t P[HW];                                    // unscaled: P[t] = u 2^v
+            get(pan + (size_t)pid * HW, P, N16{});
+            const uint32_t ui = inv_odd(P[t] >> v) & mask;
             if (tid == 0) {
                 s_pid[t] = pid;
                 s_ui[t] = ui;
@@ -267,147 +362,109 @@ __device__ void howell_blocked(const HJob& job, uint32_t k, uint32_t rc, uint32_
                 job.pivots[h] = c0 + t;
                 job.pivot_v[h] = v;
             }
-            for (uint32_t pos = tid, j = 0; pos < na; pos += HT, ++j) {
-                const uint32_t id = act[pos];
-                if (id == NONE || (chosen >> j & 1u)) continue;
-                PT* R = pan + id * HW;
-                const uint32_t q = (R[t] & mask) >> v;
-                if (q == 0) continue;
-                qm[id * HW + t] = q;                           // w.r.t. the scaled pivot row
-                nz[id] = 1;
-                const uint32_t qe = kmul<SMALLK>(q, ui) & mask;
-                uint32_t t2 = t;                               // four columns per round, reads first
-                for (; t2 + 4 <= wc; t2 += 4) {
-                    uint32_t rv[4], pv[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        rv[e] = R[t2 + e];
-                        pv[e] = P[t2 + e];
-                    }
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) R[t2 + e] = (rv[e] - kmul<SMALLK>(qe, pv[e])) & mask;
+            for (int j = 0; j < RPT; ++j) {
+                if (bpos == tid + j * NT) {
+                    live[j] = false;
+                    picked[j] = true;
                 }
-                for (; t2 < wc; ++t2) R[t2] = (R[t2] - kmul<SMALLK>(qe, P[t2])) & mask;
+                const uint32_t q = R[j][t] >> v;
+                if (!live[j] || q == 0) continue;
+                qm[id[j] * HW + t] = (PT)q;                    // w.r.t. the scaled pivot row
+                nz[id[j]] = 1;
+                const uint32_t qe = kmul<SMALLK>(q, ui) & mask;
+                R[j][t] = 0;
+#pragma unroll
+                for (uint32_t e = t + 1; e < HW; ++e) R[j][e] = (R[j][e] - kmul<SMALLK>(qe, P[e])) & mask;
+                put(pan + (size_t)id[j] * HW, R[j]);
             }
             if (v > 0) {                                       // closure row 2^(k-v) u^-1 P at the bottom
                 const uint32_t cid = m + ncl, sh = k - v;      // 1 <= sh <= 31
-                if (na % HT == tid) {
+                if (na % NT == tid) {
                     act[na] = cid;
                     nz[cid] = 1;
-                    for (uint32_t t2 = 0; t2 < HW; ++t2) {
-                        pan[cid * HW + t2] = (t2 <= t || t2 >= wc) ? 0u : (kmul<SMALLK>(P[t2], ui) << sh) & mask;
-                        qm[cid * HW + t2] = t2 == t ? (0u - (1u << sh)) & mask : 0u;
+                    uint32_t C[HW];
+#pragma unroll
+                    for (uint32_t e = 0; e < HW; ++e) {
+                        C[e] = (e <= t || e >= wc) ? 0u : (kmul<SMALLK>(P[e], ui) << sh) & mask;
+                        qm[cid * HW + e] = (PT)(e == t ? (0u - (1u << sh)) & mask : 0u);
                     }
+                    put(pan + (size_t)cid * HW, C);
+#pragma unroll
+                    for (int j = 0; j < RPT; ++j)
+                        if (na / NT == (uint32_t)j) {
+                            id[j] = cid;
+                            live[j] = true;
+                            picked[j] = false;
+#pragma unroll
+                            for (uint32_t e = 0; e < HW; ++e) R[j][e] = C[e];
+                        }
                 }
                 ++na;
                 ++ncl;
             }
             ++h;
-        }
+        };
+#pragma unroll
+        for (uint32_t t = 0; t < HW; ++t)
+            if (t < wc) step(t);
         __syncthreads();
-        for (uint32_t pos = tid, j = 0; pos < na; pos += HT, ++j)
-            if (chosen >> j & 1u) act[pos] = NONE;
+#pragma unroll
+        for (int j = 0; j < RPT; ++j)
+            if (picked[j]) act[tid + j * NT] = NONE;
         // the panel's pivot rows keep their panel entries; new closure rows start from zero
-        for (uint32_t idx = tid; idx < HW * HW; idx += HT) {
+        for (uint32_t idx = tid; idx < HW * HW; idx += NT) {
             const uint32_t t = idx / HW, t2 = idx % HW, pid = s_pid[t];
             if (pid != NONE && t2 < wc) rows[(size_t)pid * n + c0 + t2] = kmul<SMALLK>(pan[pid * HW + t2], s_ui[t]) & mask;
         }
         const uint32_t tw = n - c1;
-        for (uint64_t idx = tid; idx < (uint64_t)(ncl - ncl0) * tw; idx += HT)
+        for (uint64_t idx = tid; idx < (uint64_t)(ncl - ncl0) * tw; idx += NT)
             rows[(size_t)(m + ncl0 + idx / tw) * n + c1 + idx % tw] = 0;
         __syncthreads();
         // (B) the trailing columns, 256 at a time: (B1) one thread per column brings the panel's
         // pivot rows up to date (T_t, in step order) into s_T and back to their rows; (B2) every
-        // wave sweeps a quarter of the active rows over the 256 columns, 4 columns per lane (64
-        // apart: coalesced) and 8 rows at a time, so 32 independent loads are in flight per lane.
-        for (uint32_t j0 = c1; j0 < n; j0 += HT) {
+        // wave sweeps its columns over its groups of active rows.
+        for (uint32_t j0 = c1; j0 < n; j0 += HCOL) {
             const uint32_t j = j0 + tid;
-            if (j < n) {
+            if (tid < HCOL) {
                 // all HW pivot-row entries are loaded before any is written back (the rows are
                 // distinct), so the loads are in flight together instead of one after another
                 uint32_t T[HW];
 #pragma unroll
                 for (uint32_t t = 0; t < HW; ++t) {
                     const uint32_t pid = s_pid[t];
-                    T[t] = pid == NONE ? 0u : rows[(size_t)pid * n + j];
+                    T[t] = pid == NONE || j >= n ? 0u : rows[(size_t)pid * n + j];
                 }
 #pragma unroll
                 for (uint32_t t = 0; t < HW; ++t) {
                     const uint32_t pid = s_pid[t];
                     if (pid == NONE) { T[t] = 0; continue; }
-                    uint32_t x = T[t];
-                    const PT* qr = qm + pid * HW;
+                    uint32_t x = T[t], qr[HW];
+                    get(qm + (size_t)pid * HW, qr, N16{});
 #pragma unroll
                     for (uint32_t s2 = 0; s2 < t; ++s2) x -= kmul<SMALLK>(qr[s2], T[s2]);
                     T[t] = kmul<SMALLK>(x & mask, s_ui[t] & mask) & mask;
+                    __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
                 for (uint32_t t = 0; t < HW; ++t) {
                     const uint32_t pid = s_pid[t];
-                    if (pid != NONE) rows[(size_t)pid * n + j] = T[t];
+                    if (pid != NONE && j < n) rows[(size_t)pid * n + j] = T[t];
                 }
 #pragma unroll
-                for (uint32_t t = 0; t < HW; ++t) s_T[t * HT + tid] = T[t];
+                for (uint32_t t = 0; t < HW; ++t) s_T[t * HCOL + tid] = T[t];
             }
             __syncthreads();
-            uint32_t Tr[HW][4];
-#pragma unroll
-            for (uint32_t t = 0; t < HW; ++t)
-#pragma unroll
-                for (uint32_t u = 0; u < 4; ++u) Tr[t][u] = s_T[t * HT + lane + 64 * u];
-            bool in[4];
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) in[u] = j0 + lane + 64 * u < n;
-            // groups of 8 active rows per wave; the next group's ids and entries are loaded before
-            // this group's entries are written back (different rows)
-            uint32_t ids[8], xs[8][4];
-            auto load_group = [&](uint32_t pos, uint32_t (&gid)[8], uint32_t (&gx)[8][4]) {
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const uint32_t id = pos + r < na ? act[pos + r] : NONE;
-                    gid[r] = (id != NONE && nz[id]) ? id : NONE;
-                }
-#pragma unroll
-                for (int r = 0; r < 8; ++r)
-#pragma unroll
-                    for (uint32_t u = 0; u < 4; ++u)
-                        gx[r][u] = (gid[r] != NONE && in[u]) ? rows[(size_t)gid[r] * n + j0 + lane + 64 * u] : 0u;
-            };
-            if (wave * 8 < na) load_group(wave * 8, ids, xs);
-            for (uint32_t pos = wave * 8; pos < na; pos += 32) {
-                uint32_t nids[8], nxs[8][4];
-                if (pos + 32 < na) load_group(pos + 32, nids, nxs);
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    if (ids[r] == NONE) continue;
-                    const PT* qr = qm + ids[r] * HW;
-                    uint32_t q[HW];
-#pragma unroll
-                    for (uint32_t t = 0; t < HW; ++t) q[t] = qr[t];
-#pragma unroll
-                    for (uint32_t u = 0; u < 4; ++u) {
-                        if (!in[u]) continue;
-                        uint32_t x = xs[r][u];
-#pragma unroll
-                        for (uint32_t t = 0; t < HW; ++t) x -= kmul<SMALLK>(q[t], Tr[t][u]);
-                        rows[(size_t)ids[r] * n + j0 + lane + 64 * u] = x;
-                    }
-                }
-                if (pos + 32 < na) {
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) {
-                        ids[r] = nids[r];
-#pragma unroll
-                        for (uint32_t u = 0; u < 4; ++u) xs[r][u] = nxs[r][u];
-                    }
-                }
-            }
+            sweep(rows, j0, na, [&](uint32_t pos) {
+                const uint32_t i = act[pos];
+                return i != NONE && nz[i] ? i : NONE;
+            }, 0xffffffffu);
             __syncthreads();
         }
     }
     // H rows in pivot order (masked).  Left of its pivot column a pivot row is zero mod 2^k; its
     // stored entries there may be stale (panel entries are written back for pivot rows only).
-    for (uint32_t i = wave; i < h; i += HT / 64) {     // a wave per row, four words per lane in flight
+    for (uint32_t i = wave; i < h; i += NW) {     // a wave per row, four words per lane in flight
         const uint32_t* Ri = rows + (size_t)prow[i] * n;
         uint32_t* Hi = job.H + (size_t)i * n;
         const uint32_t pc = job.pivots[i];
@@ -432,51 +489,33 @@ __device__ void howell_blocked(const HJob& job, uint32_t k, uint32_t rc, uint32_
             s_v[tid] = tid < bw ? job.pivot_v[i0 + tid] : 0u;
         }
         __syncthreads();
-        for (uint32_t idx = tid; idx < HW * HW; idx += HT) {
+        for (uint32_t idx = tid; idx < HW * HW; idx += NT) {
             const uint32_t t = idx / HW, t2 = idx % HW;
             s_hb[idx] = (t < bw && t2 < bw) ? job.H[(size_t)(i0 + t) * n + s_c[t2]] : 0u;
         }
         __syncthreads();
-        for (uint32_t ip = tid; ip < i1; ip += HT) {
-            uint32_t cur[HW];
+        for (uint32_t ip = tid; ip < i1; ip += NT) {
+            uint32_t cur[HW], q[HW];
 #pragma unroll
             for (uint32_t t2 = 0; t2 < HW; ++t2) cur[t2] = t2 < bw ? job.H[(size_t)ip * n + s_c[t2]] : 0u;
-#pragma unroll 1
+#pragma unroll
             for (uint32_t t = 0; t < HW; ++t) {
-                uint32_t q = 0;
-                if (t < bw && i0 + t > ip) q = (cur[t] & mask) >> s_v[t];
+                q[t] = t < bw && i0 + t > ip ? (cur[t] & mask) >> s_v[t] : 0u;
 #pragma unroll
-                for (uint32_t t2 = t + 1; t2 < HW; ++t2) cur[t2] -= kmul<SMALLK>(q, s_hb[t * HW + t2]);
-                qm[ip * HW + t] = q;
+                for (uint32_t t2 = t + 1; t2 < HW; ++t2) cur[t2] -= kmul<SMALLK>(q[t], s_hb[t * HW + t2]);
+                __builtin_amdgcn_sched_barrier(0);     // (one step's coefficients in registers at a time)
             }
+            put(qm + (size_t)ip * HW, q);
         }
-        __syncthreads();
-        for (uint32_t j = s_c[0] + tid; j < n; j += HT) {
-            uint32_t Hr[HW];
-#pragma unroll
-            for (uint32_t t = 0; t < HW; ++t) Hr[t] = t < bw ? job.H[(size_t)(i0 + t) * n + j] : 0u;
-            // rows in groups of 8; the next group's entries are loaded before this group's are
-            // written back (different rows), so a load's latency overlaps the previous group
-            uint32_t xs[8];
-#pragma unroll
-            for (uint32_t u = 0; u < 8; ++u) xs[u] = u < i1 ? job.H[(size_t)u * n + j] : 0u;
-            for (uint32_t ip0 = 0; ip0 < i1; ip0 += 8) {
-                uint32_t xn[8];
-#pragma unroll
-                for (uint32_t u = 0; u < 8; ++u)
-                    xn[u] = ip0 + 8 + u < i1 ? job.H[(size_t)(ip0 + 8 + u) * n + j] : 0u;
-#pragma unroll
-                for (uint32_t u = 0; u < 8; ++u) {
-                    if (ip0 + u >= i1) continue;
-                    const PT* qr = qm + (ip0 + u) * HW;
-                    uint32_t x = xs[u];
-#pragma unroll
-                    for (uint32_t t = 0; t < HW; ++t) x -= kmul<SMALLK>(qr[t], Hr[t]);
-                    job.H[(size_t)(ip0 + u) * n + j] = x & mask;
-                }
-#pragma unroll
-                for (uint32_t u = 0; u < 8; ++u) xs[u] = xn[u];
+        // 256 columns at a time: the block's rows into LDS before any of them is updated, then the sweep
+        for (uint32_t jb = s_c[0]; jb < n; jb += HCOL) {
+            __syncthreads();                      // the multipliers are written; the last sweep is done with s_T
+            for (uint32_t idx = tid; idx < HW * HCOL; idx += NT) {
+                const uint32_t t = idx / HCOL, j = jb + idx % HCOL;
+                s_T[idx] = t < bw && j < n ? job.H[(size_t)(i0 + t) * n + j] : 0u;
             }
+            __syncthreads();
+            sweep(job.H, jb, i1, [](uint32_t pos) { return pos; }, mask);
         }
         __syncthreads();
     }
@@ -485,8 +524,8 @@ __device__ void howell_blocked(const HJob& job, uint32_t k, uint32_t rc, uint32_
 }
 
 // Persistent: one workgroup per job of this row-capacity class, jobs from the class's counter.
-template <bool SMALLK, class PT>
-__global__ __launch_bounds__(HT) void howell_blocked_kernel(HArgs a, uint32_t rc) {
+template <bool SMALLK, class PT, int NT, int RPT>
+__global__ __launch_bounds__(NT, 4) void howell_blocked_kernel(HArgs a, uint32_t rc) {
     extern __shared__ __attribute__((aligned(16))) uint32_t hlds[];
     __shared__ uint32_t s_job;
     for (;;) {
@@ -495,15 +534,23 @@ __global__ __launch_bounds__(HT) void howell_blocked_kernel(HArgs a, uint32_t rc
         const uint32_t jj = s_job;
         __syncthreads();
         if (jj >= a.njobs) break;
-        howell_blocked<SMALLK, PT>(a.jobs[a.order[jj]], a.k, rc, hlds);
+        howell_blocked<SMALLK, PT, NT, RPT>(a.jobs[a.order[jj]], a.k, rc, hlds);
     }
 }
 
-// The blocked kernel for this k: 16-bit stores for k <= 16, the 24-bit multiply for k <= 24.
-inline const void* blocked_kernel_for(uint32_t k) {
-    if (k <= 16) return (const void*)howell_blocked_kernel<true, uint16_t>;
-    if (k <= 24) return (const void*)howell_blocked_kernel<true, uint32_t>;
-    return (const void*)howell_blocked_kernel<false, uint32_t>;
+// The blocked kernel for this k, row capacity and thread count: 16-bit stores for k <= 16, the 24-bit multiply for
+// k <= 24.
+using BlockedKernel = void (*)(HArgs, uint32_t);
+template <int NT, int RPT>
+BlockedKernel blocked_kernel_of(uint32_t k) {
+    if (k <= 16) return howell_blocked_kernel<true, uint16_t, NT, RPT>;
+    if (k <= 24) return howell_blocked_kernel<true, uint32_t, NT, RPT>;
+    return howell_blocked_kernel<false, uint32_t, NT, RPT>;
+}
+inline BlockedKernel blocked_kernel_for(uint32_t k, uint32_t rc, int nt) {
+    if (rc <= 256) return blocked_kernel_of<256, 1>(k);
+    if (rc <= 512) return blocked_kernel_of<512, 1>(k);
+    return nt == 1024 ? blocked_kernel_of<1024, 1>(k) : blocked_kernel_of<512, 2>(k);
 }
 inline uint32_t blocked_elt_bytes(uint32_t k) { return k <= 16 ? 2u : 4u; }
 
@@ -681,6 +728,7 @@ constexpr uint32_t kClassRows[NCLASS - 1] = {256, 512, kBlockedRows};
 
 struct HClass {
     uint32_t njobs = 0, grid = 0, rc = 0;
+    int nt = HT;                         // threads per job (blocked classes)
     size_t lds = 0;
     uint32_t* d_order = nullptr;
 };
@@ -770,8 +818,11 @@ HBatch* batch_create(uint32_t ell, uint32_t k, const hx_howell_job* jobs, uint32
         static std::once_flag once;
         std::call_once(once, [] {
             for (uint32_t kk : {16u, 24u, 32u})
-                (void)hipFuncSetAttribute(blocked_kernel_for(kk), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)blocked_lds_bytes(kBlockedRows, blocked_elt_bytes(kk)));
+                for (uint32_t rows : kClassRows)
+                    for (int nt : {512, 1024})
+                        (void)hipFuncSetAttribute((const void*)blocked_kernel_for(kk, rows, nt),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                  (int)blocked_lds_bytes(rows, blocked_elt_bytes(kk)));
         });
         for (int c = 0; c < NCLASS; ++c) {
             HClass& cl = b->cls[c];
@@ -785,13 +836,17 @@ HBatch* batch_create(uint32_t ell, uint32_t k, const hx_howell_job* jobs, uint32
                 for (uint32_t i : per[c]) rc = std::max(rc, hj[i].m + hj[i].n);
                 cl.rc = rc;
                 cl.lds = blocked_lds_bytes(rc, blocked_elt_bytes(k));
-                int nb = 0;
-                const void* kern = blocked_kernel_for(k);
-                if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, HT, cl.lds) == hipSuccess &&
-                    nb > 0)
-                    per_cu = nb;
-                else
-                    per_cu = 1;
+                auto per_unit = [&](int nt) {
+                    int nb = 0;
+                    const void* kern = (const void*)blocked_kernel_for(k, rc, nt);
+                    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, nt, cl.lds) == hipSuccess && nb > 0 ? nb : 1;
+                };
+                // Rows past 512: two jobs of 512 threads on a compute unit for throughput, all of it for one job of
+                // 1024 threads when the jobs are no more than the units (the largest job decides) or only one fits.
+                // (m + n to 1024, k = 16: 250 large jobs 3.5 ms on 1024 threads, 4.8 on 512; 1000 large jobs 8.5 / 8.2.)
+                cl.nt = rc <= 256 ? 256 : 512;
+                if (rc > 512 && (cl.njobs <= (uint32_t)cus || per_unit(512) < 2)) cl.nt = 1024;
+                per_cu = per_unit(cl.nt);
             }
             cl.grid = std::max<uint32_t>(1, std::min<uint32_t>(cl.njobs, (uint32_t)cus * per_cu));
         }
@@ -864,12 +919,7 @@ HX_API int hx_howell_batch_run(hx_howell_batch vb, hx_stream s) {
                 howell_batch_kernel<<<cl.grid, HT, 0, sc>>>(a);
                 after_launch("howell_batch_kernel");
             } else {
-                if (b->k <= 16)
-                    howell_blocked_kernel<true, uint16_t><<<cl.grid, HT, cl.lds, sc>>>(a, cl.rc);
-                else if (b->k <= 24)
-                    howell_blocked_kernel<true, uint32_t><<<cl.grid, HT, cl.lds, sc>>>(a, cl.rc);
-                else
-                    howell_blocked_kernel<false, uint32_t><<<cl.grid, HT, cl.lds, sc>>>(a, cl.rc);
+                blocked_kernel_for(b->k, cl.rc, cl.nt)<<<cl.grid, cl.nt, cl.lds, sc>>>(a, cl.rc);
                 after_launch("howell_blocked_kernel");
             }
         }

@@ -113,3 +113,26 @@ def test_howell_batch_graph_replay(hx_gpu, O):
                 assert np.array_equal(res.pivots, piv) and np.array_equal(res.pivot_v, pv), (rep, A.shape)
                 assert np.array_equal(res.H, H), (rep, A.shape)
         _lib.check(_lib.lib().hx_graph_destroy(g))
+
+
+@pytest.mark.parametrize("k", [5, 16, 20, 32])
+@pytest.mark.parametrize("m,n,count", [(500, 16, 260), (30, 490, 1), (510, 514, 1), (250, 262, 2), (100, 156, 3), (1007, 17, 2)])
+def test_howell_thread_classes(hx_gpu, O, k, m, n, count):
+    """The row classes at their edges (256, 512, 1024 rows) and both thread counts of the largest (260 jobs: two
+    per compute unit): uniform words with planted powers of two, so closure rows come in every class."""
+    from hacs_amd import engine as E
+    rng = np.random.default_rng(k * 1000 + m + n)
+    mats = []
+    for _ in range(count):
+        A = rng.integers(0, 1 << 32, (m, n), dtype=np.uint64).astype(np.uint32)
+        A <<= rng.integers(0, min(k, 6), (1, n)).astype(np.uint32)
+        A[rng.random((m, n)) < 0.3] = 0
+        mats.append(A & np.uint32((1 << k) - 1))
+    hb = E.HowellBatch(k, [E.to_device(A) for A in mats])
+    for _ in range(2):                                   # the second run finds the first one's work rows
+        hb.run()
+    torch.cuda.synchronize()
+    for i in {0, count // 2, count - 1}:
+        got = hb.results([i])[0]
+        H, piv, v = O.howell_fast(k, mats[i])
+        assert np.array_equal(got.H, H) and np.array_equal(got.pivots, piv) and np.array_equal(got.pivot_v, v), i
