@@ -322,15 +322,12 @@ __device__ __forceinline__ void prep_tile(const PrepArgs& a, uint32_t bx, uint32
     uint32_t w[4][4];   // [plane][word]: 16 k-bytes of this row per plane
 #pragma unroll
     for (int wd = 0; wd < 4; ++wd) {
+        uint32_t x4[4], l4[4];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) w[s][wd] = 0;
+        for (int b = 0; b < 4; ++b) x4[b] = T[r][16 * q + 4 * wd + b];
+        limb_split4<4>(x4, a.p, a.half, l4);         // (planes at or past L are not stored)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            int32_t d[4] = {0, 0, 0, 0};
-            limbs_of(T[r][16 * q + 4 * wd + b], a.p, a.half, a.L, d);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) w[s][wd] |= ((uint32_t)d[s] & 0xffu) << (8 * b);
-        }
+        for (int s = 0; s < 4; ++s) w[s][wd] = l4[s];
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -723,16 +720,17 @@ __device__ __forceinline__ void limb_tile3(const LimbArgs& a, uint32_t tm, uint3
 // limb_tile3's pipeline with eight waves per workgroup: the same 64 x 128 tile and LDS ring, each
 // wave owning one 32 x 32 block (wm = wave & 1: rows, wn = wave >> 1: columns), so the
 // accumulators (2L-1 x 16 registers) leave room for two waves per SIMD and one wave's barrier
-// waits and epilogue overlap the other's MFMAs.  The 12L copy blocks of a stage are dealt
-// round-robin over the eight waves (blk = wave + 8 i).
-template <int L>
+// waits and epilogue overlap the other's MFMAs.  The copy blocks of a stage are dealt
+// round-robin over the waves (blk = wave + 2 NWN i).  NWN: waves across, 4 for the 64 x 128 tile, 2 for a 64 x 64
+// tile on four waves: twice the workgroups where the wide tiles leave compute units idle.
+template <int L, int NWN>
 __device__ __forceinline__ void stage_issue8(const LimbArgs& a, const int8_t* Abase, const int8_t* Bbase, int wave,
                                              uint32_t kt, uint8_t* st) {
-    constexpr int SA = L * LM * 64, NBLK = 12 * L, PER = (NBLK + 7) / 8;
+    constexpr int W = 2 * NWN, BG = 2 * NWN, SA = L * LM * 64, NBLK = (4 + BG) * L, PER = (NBLK + W - 1) / W;
     const size_t k0 = (size_t)kt * LK;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        const int blk = wave + 8 * i;
+        const int blk = wave + W * i;
         if (blk >= NBLK) break;
         const int8_t* src;
         uint8_t* dst;
@@ -741,9 +739,9 @@ __device__ __forceinline__ void stage_issue8(const LimbArgs& a, const int8_t* Ab
             src = Abase + s * a.a_plane + (size_t)(16 * g) * a.Kp + k0;
             dst = st + s * (LM * 64) + g * 1024;
         } else {
-            const int s = (blk - 4 * L) >> 3, g = (blk - 4 * L) & 7;
+            const int s = (blk - 4 * L) / BG, g = (blk - 4 * L) % BG;
             src = Bbase + s * a.b_plane + (size_t)(16 * g) * a.Kp + k0;
-            dst = st + SA + s * (LN * 64) + g * 1024;
+            dst = st + SA + s * (BG * 1024) + g * 1024;
         }
         __builtin_amdgcn_global_load_lds((const void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
     }
@@ -755,7 +753,7 @@ struct LFrag1 {
     v4i b[L];
 };
 
-template <int L>
+template <int L, int NWN>
 __device__ __forceinline__ void stage_frag1(const uint8_t* st, int ks, int wm, int wn, int lane, LFrag1<L>& f) {
     constexpr int SA = L * LM * 64;
     const int lr = lane & 31, q = ks * 2 + (lane >> 5);
@@ -763,7 +761,7 @@ __device__ __forceinline__ void stage_frag1(const uint8_t* st, int ks, int wm, i
 #pragma unroll
     for (int s = 0; s < L; ++s) f.a[s] = *(const v4i*)(st + s * (LM * 64) + ra * 64 + 16 * (q ^ swz(ra)));
 #pragma unroll
-    for (int s = 0; s < L; ++s) f.b[s] = *(const v4i*)(st + SA + s * (LN * 64) + rb * 64 + 16 * (q ^ swz(rb)));
+    for (int s = 0; s < L; ++s) f.b[s] = *(const v4i*)(st + SA + s * (NWN * 2048) + rb * 64 + 16 * (q ^ swz(rb)));
 }
 
 template <int L>
@@ -775,17 +773,17 @@ __device__ __forceinline__ void frag_mfma1(const LFrag1<L>& f, v16i (&acc)[1][2 
             acc[0][s + t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[s], f.b[t], acc[0][s + t], 0, 0, 0);
 }
 
-template <int L>
+template <int L, int NWN = 4>
 __device__ __forceinline__ void limb_tile4(const LimbArgs& a, uint32_t tm, uint32_t tn) {
-    constexpr int SA = L * LM * 64, SB = L * LN * 64, STAGE = SA + SB;
-    constexpr int ND = 2 * L - 1, NBLK = 12 * L;
-    // DMA instructions per wave per stage: waves below NBLK % 8 issue one more
-    constexpr int HI = (NBLK + 7) / 8, LO = NBLK / 8, NHI = NBLK % 8 == 0 ? 8 : NBLK % 8;
+    constexpr int W = 2 * NWN, SA = L * LM * 64, SB = L * NWN * 2048, STAGE = SA + SB;
+    constexpr int ND = 2 * L - 1, NBLK = (4 + 2 * NWN) * L;
+    // DMA instructions per wave per stage: waves below NBLK % W issue one more
+    constexpr int HI = (NBLK + W - 1) / W, LO = NBLK / W, NHI = NBLK % W == 0 ? W : NBLK % W;
     __shared__ __attribute__((aligned(1024))) uint8_t s0[STAGE];
     __shared__ __attribute__((aligned(1024))) uint8_t s1[STAGE];
     __shared__ __attribute__((aligned(1024))) uint8_t s2[STAGE];
     const uint32_t m = a.m_dev ? min(*a.m_dev, a.m) : a.m;
-    const uint32_t m0 = tm * LM, n0 = tn * LN;
+    const uint32_t m0 = tm * LM, n0 = tn * (32 * NWN);
     if (m0 >= m) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -815,24 +813,24 @@ __device__ __forceinline__ void limb_tile4(const LimbArgs& a, uint32_t tm, uint3
     };
     const uint32_t KT = a.Kp / LK;
     if (KT > 0) {
-        stage_issue8<L>(a, Abase, Bbase, wave, 0, s0);
-        if (KT > 1) stage_issue8<L>(a, Abase, Bbase, wave, 1, s1);
-        if (KT > 2) stage_issue8<L>(a, Abase, Bbase, wave, 2, s2);
+        stage_issue8<L, NWN>(a, Abase, Bbase, wave, 0, s0);
+        if (KT > 1) stage_issue8<L, NWN>(a, Abase, Bbase, wave, 1, s1);
+        if (KT > 2) stage_issue8<L, NWN>(a, Abase, Bbase, wave, 2, s2);
         wait_stages(KT > 2 ? 2 : (KT > 1 ? 1 : 0));
         wg_barrier();
         LFrag1<L> fa, fb;
-        stage_frag1<L>(s0, 0, wm, wn, lane, fa);
+        stage_frag1<L, NWN>(s0, 0, wm, wn, lane, fa);
         __builtin_amdgcn_s_waitcnt(wait_imm(63, 0));
         auto body = [&](uint32_t kt, uint8_t* cur, const uint8_t* nxt) {
-            stage_frag1<L>(cur, 1, wm, wn, lane, fb);
+            stage_frag1<L, NWN>(cur, 1, wm, wn, lane, fb);
             __builtin_amdgcn_sched_barrier(0);
             frag_mfma1<L>(fa, acc);
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_s_waitcnt(wait_imm(63, 0));
             wait_stages(kt + 2 < KT ? 1 : 0);
             wg_barrier();
-            if (kt + 3 < KT) stage_issue8<L>(a, Abase, Bbase, wave, kt + 3, cur);
-            stage_frag1<L>(nxt, 0, wm, wn, lane, fa);
+            if (kt + 3 < KT) stage_issue8<L, NWN>(a, Abase, Bbase, wave, kt + 3, cur);
+            stage_frag1<L, NWN>(nxt, 0, wm, wn, lane, fa);
             __builtin_amdgcn_sched_barrier(0);
             frag_mfma1<L>(fb, acc);
             __builtin_amdgcn_sched_barrier(0);
@@ -845,7 +843,7 @@ __device__ __forceinline__ void limb_tile4(const LimbArgs& a, uint32_t tm, uint3
         }
         const uint32_t ls = (KT - 1) % 3;
         const uint8_t* cur = ls == 0 ? s0 : (ls == 1 ? s1 : s2);
-        stage_frag1<L>(cur, 1, wm, wn, lane, fb);
+        stage_frag1<L, NWN>(cur, 1, wm, wn, lane, fb);
         frag_mfma1<L>(fa, acc);
         frag_mfma1<L>(fb, acc);
     }
@@ -954,13 +952,12 @@ __global__ __launch_bounds__(768, 1) void limb5_kernel(LimbArgs a) {
     limb_tile5<L>(a, tm, tn);
 }
 
-template <int L>
-__global__ __launch_bounds__(512, 1) void limb4_kernel(LimbArgs a) {
+template <int L, int NWN = 4>
+__global__ __launch_bounds__(128 * NWN, 1) void limb4_kernel(LimbArgs a) {
     uint32_t tm, tn;
     tile_of(blockIdx.x, a.ntm, a.ntn, tm, tn);
-    limb_tile4<L>(a, tm, tn);
+    limb_tile4<L, NWN>(a, tm, tn);
 }
-
 template <int L>
 __global__ __launch_bounds__(512, 1) void limb4_batch_kernel(const LimbArgs* jobs, const uint32_t* prefix,
                                                              uint32_t njobs) {
@@ -1430,6 +1427,10 @@ __global__ __launch_bounds__(256) void crt_kernel(CrtArgs a) {
 // pipelined against the MFMAs (limb3_kernel), 4 = limb3's pipeline on eight waves
 // (limb4_kernel), 5 = the 96 x 128 tile on twelve waves (limb5_kernel); 0 = the default.
 constexpr int kLimbDefault = 4;
+// (internal) limb kernel 4 on 64 x 64 tiles, the default's choice where the 64 x 128 tiles are fewer than the units
+// (64 x 128 / 64 x 64, us a call: 1024^3 mod 65521 36 / 31, mod 2147483629 51 / 45; 512^2 x 8192 193 / 120; 2048^3, 512
+// wide tiles, 146 / 147)
+constexpr int kLimb4Narrow = 40;
 inline int limb_version(int tile) { return tile >= 1 && tile <= 5 ? tile : kLimbDefault; }
 // tile 6 of the limb variant: the residue route (res_gemm_kernel) in place of the limb kernels
 constexpr int kResidueTile = 6;
@@ -1445,6 +1446,13 @@ void launch_limb(const LimbArgs& la, hipStream_t s, int ver) {
     if (ver == 3) {
         limb3_kernel<L><<<blocks, 256, 0, s>>>(la);
         after_launch("limb3_kernel");
+        return;
+    }
+    if (ver == kLimb4Narrow) {
+        LimbArgs l4 = la;
+        l4.ntn = 2 * la.ntn;
+        limb4_kernel<L, 2><<<2 * blocks, 256, 0, s>>>(l4);
+        after_launch("limb4_kernel");
         return;
     }
     if (ver == 4) {
@@ -1624,7 +1632,8 @@ void gemm_limb(const hx_modctx& ctx, const GemmArgs& g0, hipStream_t s, void* ws
         limb_epilogue_consts(p, la);
         la.M = devmod(ctx);
         const bool last = k0 + kc >= g.k;
-        const int ver = limb_version(tile);
+        int ver = limb_version(tile);
+        if (tile == 0 && la.ntm * la.ntn < 256) ver = kLimb4Narrow;
         if (ev0 && k0 == 0) HX_HIP(hipEventRecord(ev0, s));
         switch (L) {
             case 1: launch_limb<1>(la, s, ver); break;
@@ -1676,17 +1685,19 @@ bool auto_splits(uint32_t m, uint32_t n, uint32_t k) {
 // 1 <= k <= RES_KMAX and enough moduli; tile kResidueTile asks for it wherever it applies.  The limb variant's
 // default (tile 0) takes it where it runs at most L^2 - 4 int8 products (four-limb moduli: 10 or 11 for 16) and
 // m, n, k >= 4096.  The automatic variant takes it at every m, n once k is deep enough to pay for the splits
-// and the CRT, whose cost does not grow with k: k >= 768 for four limbs, k >= 1536 for three (us, limb kernel 4
-// / residue route; mod 2147483629: 768^3 42 / 40, 1024^3 54 / 47, 2048^3 152 / 145, 4096^3 1027 / 770,
-// 8192^3 7400 / 5200, 8192^2 x 512 606 / 680, x 1024 1131 / 953; mod 65521: 1024^3 39 / 40, 2048^3 101 / 99,
-// 4096^3 621 / 480, 8192^2 x 512 427 / 480; mod 1000003: 1024^3 40 / 41, 2048^3 107 / 109, 4096^3 675 / 550).
-// Two-limb moduli stay on the limb kernels (mod 61001: 2048^2 x 1024 49 / 66, 8192^2 x 1024 411 / 670).
+// and the CRT, whose cost does not grow with k: k >= 1536, and k >= 768 for four limbs where the limb kernel's
+// 64 x 128 tiles fill the units, as its 64 x 64 tiles are the better ones below (us, limb kernel 4 / residue
+// route; mod 2147483629: 768^3 33 / 40, 1024^3 45 / 48, 1677 x 1419 x 2049 133 / 114, 512^2 x 8192 120 / 80, 2048^3
+// 147 / 145, 4096^3 990 / 760, 8192^3 7400 / 5200, 8192^2 x 512 600 / 680, x 1024 1131 / 953; mod 65521: 2048^3
+// 96 / 96, 4096^3 596 / 473, 512^2 x 8192 85 / 65, 8192^2 x 512 421 / 480; mod 1000003: 2048^3 107 / 109, 4096^3
+// 675 / 550).  Two-limb moduli stay on the limb kernels (mod 61001: 2048^2 x 1024 49 / 66, 8192^2 x 1024 411 / 670).
 uint32_t residue_choice(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, bool device_sizes, int tile,
                         bool automatic) {
     if (device_sizes || (tile != 0 && tile != kResidueTile)) return 0;
     const uint32_t N = residue_moduli(ctx.p, k);
     if (N == 0 || tile == kResidueTile) return N;
-    if (automatic && ctx.limbs >= 3 && k >= (ctx.limbs == 4 ? 768u : 1536u)) return N;
+    const uint64_t limb_tiles = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
+    if (automatic && ctx.limbs >= 3 && k >= (ctx.limbs == 4 && limb_tiles >= 256 ? 768u : 1536u)) return N;
     const bool large = m >= 4096 && n >= 4096 && k >= 4096;
     return large && ctx.limbs > 0 && N + 4 <= ctx.limbs * ctx.limbs ? N : 0;
 }
