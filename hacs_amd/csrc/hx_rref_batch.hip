@@ -1,6 +1,6 @@
 // hx_rref_batch.hip -- RREF over F_p for many independent, uneven matrices in ONE persistent launch.
 //
-// One 256-thread workgroup eliminates one job at a time and pulls the next job index from an atomic
+// One workgroup of 256 or 512 threads eliminates one job at a time and pulls the next job index from an atomic
 // counter (jobs pre-sorted by decreasing work), so thousands of jobs of shapes 16..1024 share the
 // chip without a launch per job.  Per job (in place on its buffer, like elim::rref, DenseElim.h:149-151):
 //
@@ -35,7 +35,6 @@
 namespace hx {
 namespace {
 
-constexpr int RT = 256;   // threads per job workgroup
 constexpr int RW = 32;    // widest panel
 
 struct RJob {
@@ -46,6 +45,8 @@ struct RJob {
     uint32_t* pivot_rows;
     uint32_t* rank;
     uint32_t* U;          // min(m, n) x n, row stride n
+    uint32_t* S;          // the matrix being eliminated: A itself, or a copy of row stride n
+    uint32_t ld4;         // row stride of S in bytes
     uint32_t panel;       // widest panel for this job (a tuning choice)
 };
 
@@ -60,11 +61,33 @@ struct RArgs {
     DevMod M;
     uint32_t half;        // (p - 1) / 2
     double inv;           // 1 / p (limb_small_product)
-    int L;                // limbs per residue (1..4)
 };
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
+
+// S and U are reached through buffer resources: an entry is a 32-bit byte offset, and an offset at or past the
+// buffer's size reads 0 and stores nothing, so rows that take no update and columns past the matrix need no
+// branch (with one per entry the 16 loads and 16 stores of a block were 32 small exec regions with 64-bit addresses,
+// flat accesses among them; 4096 jobs of 16..512: 3.43 -> 2.20 ms, 512 jobs of 512 x 512: 5.05 -> 3.12 ms).  A dead row's offset plus a dead column's still does not wrap.
+constexpr uint32_t kDeadRow = 0x80000000u, kDeadCol = 0x7ff00000u;
+constexpr uint64_t kMaxBytes = kDeadCol;     // a larger matrix (its row stride included) is eliminated in a copy
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ __forceinline__ uint32_t scalar(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+__device__ __forceinline__ uint32_t* scalar(uint32_t* x) {
+    const uint64_t v = (uint64_t)x;
+    return (uint32_t*)((uint64_t)scalar((uint32_t)(v >> 32)) << 32 | scalar((uint32_t)v));
+}
+__device__ __forceinline__ rsrc_t buffer_of(uint32_t* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(scalar(base), 0, (int)scalar(bytes), 0x00020000);
+}
+__device__ __forceinline__ uint32_t bload(rsrc_t r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0);
+}
+__device__ __forceinline__ void bstore(rsrc_t r, uint32_t off, uint32_t v) {
+    __builtin_amdgcn_raw_buffer_store_b32(v, r, (int)off, 0, 0);
+}
+__device__ __forceinline__ uint32_t bytes_s(const RJob& job) { return (job.m - 1) * job.ld4 + 4 * job.n; }
+__device__ __forceinline__ uint32_t bytes_u(const RJob& job) { return 4 * min(job.m, job.n) * job.n; }
 
 // (d) on the INT8 matrix cores, k <= 32 (one 32-deep MFMA k-step), for two row sets:
 //   the unused rows u:        S[list[u], c + j] -= sum_{t<k} S[list[u], c + J_t] X[t, j],  j in [wc, nb)
@@ -92,46 +115,41 @@ __device__ __forceinline__ void split16(F&& get, uint32_t p, uint32_t half, v4i 
     }
 }
 
-template <int L>
+template <int L, int NT>
 __device__ void trailing_mfma(const RJob& job, const RArgs& a, const uint32_t* B, bool planes, uint32_t nb,
                               uint32_t wc, uint32_t k, uint32_t c, uint32_t mu, const uint32_t* list,
                               const uint8_t* chosen, const uint32_t* s_q, uint32_t r) {
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 31, lg = lane >> 5;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
+    const uint32_t wave = scalar(tid >> 6);
     const uint32_t p = a.M.p, half = a.half;
     const uint32_t nrb_u = nb > wc ? (mu + 31) / 32 : 0, nrb = nrb_u + (r + 31) / 32;
     const SmallConsts sc{p, a.inv};
-    for (uint32_t rb = wave; rb < nrb; rb += RT / 64) {
+    uint32_t *const ubase = job.U, *const sbase = job.S;
+    const uint32_t ubytes = bytes_u(job), sbytes = bytes_s(job), uld4 = 4 * job.n, sld4 = job.ld4;
+    for (uint32_t rb = wave; rb < nrb; rb += NT / 64) {
         const bool urows = rb >= nrb_u;                       // a block of stored pivot rows
         const uint32_t b0 = (urows ? rb - nrb_u : rb) * 32, nrows = urows ? r : mu, jbeg = urows ? 0 : wc;
-        uint32_t* base = urows ? job.U : job.A;
-        const int64_t ld = urows ? (int64_t)job.n : job.lda;
-        auto live_row = [&](uint32_t u) { return u < nrows && (urows || !chosen[u]); };
+        const uint32_t ld4 = urows ? uld4 : sld4;
+        const rsrc_t buf = buffer_of(urows ? ubase : sbase, urows ? ubytes : sbytes);
+        auto row_off = [&](uint32_t u) {                      // entry (u, c)'s offset, kDeadRow for no update
+            const uint32_t uc = min(u, nrows - 1);
+            const bool dead = u >= nrows || (!urows && chosen[uc]);
+            return dead ? kDeadRow : (urows ? uc : list[uc]) * ld4 + 4 * c;
+        };
         // this lane's row of the block and its 16 k-values (k-bytes 16 lg .. 16 lg + 15)
-        const uint32_t u = b0 + lr;
-        const bool live = live_row(u);
-        const int64_t rowoff = live ? (urows ? (int64_t)u : (int64_t)list[u]) * ld + c : 0;
+        const uint32_t aoff = row_off(b0 + lr);
         v4i fa[1][L];
-        split16<L>([&](int i) {
-            const uint32_t t = 16 * lg + i;
-            return (live && t < k) ? base[rowoff + s_q[t]] : 0u;
-        }, p, half, fa[0]);
-        // the 16 output rows this lane touches (accumulator element e), as matrix row indices;
-        // NOROW for rows that take no update
-        constexpr uint32_t NOROW = 0xffffffffu;
-        uint32_t orow[16];
+        split16<L>([&](int i) { return bload(buf, aoff + 4 * s_q[16 * lg + i]); }, p, half, fa[0]);
+        uint32_t orow[16];                                    // the 16 output rows (accumulator element e)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const uint32_t ur = b0 + (e / 4) * 8 + lg * 4 + (e % 4);
-            orow[e] = live_row(ur) ? (urows ? ur : list[ur]) : NOROW;
-        }
-        uint32_t* const basec = base + c;
+        for (int e = 0; e < 16; ++e) orow[e] = row_off(b0 + (e / 4) * 8 + lg * 4 + (e % 4));
         const uint32_t ncb = (nb - jbeg + 31) / 32;
         for (uint32_t cb = 0; cb < ncb; ++cb) {
-            const uint32_t j = jbeg + cb * 32 + lr;
+            const uint32_t j = jbeg + cb * 32 + lr, j4 = j < nb ? 4 * j : kDeadCol;
             // the block's entries are loaded before the MFMAs, so their latency overlaps them
             uint32_t cv[16];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) cv[e] = (j < nb && orow[e] != NOROW) ? basec[(int64_t)orow[e] * ld + j] : 0u;
+            for (int e = 0; e < 16; ++e) cv[e] = bload(buf, orow[e] + j4);
             v4i fb[1][L];
 #pragma unroll
             for (int s = 0; s < L; ++s) fb[0][s] = v4i{0, 0, 0, 0};
@@ -149,13 +167,9 @@ __device__ void trailing_mfma(const RJob& job, const RArgs& a, const uint32_t* B
             }
             uint32_t x[16];
             limb_small_product<L, 1>(fa, fb, sc, x);
-            if (j < nb) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    if (orow[e] == NOROW || x[e] == 0) continue;      // a zero update leaves the entry
-                    basec[(int64_t)orow[e] * ld + j] = subm(cv[e], x[e], p);
-                }
-            }
+            for (int e = 0; e < 16; ++e)                      // a zero update leaves the entry
+                bstore(buf, x[e] != 0 ? orow[e] + j4 : kDeadRow, subm(cv[e], x[e], p));
         }
     }
 }
@@ -193,26 +207,29 @@ __device__ __forceinline__ void elim_row(uint32_t* row, const uint32_t* prow, ui
 //       wave (all waves hold the same A fragment), S[P, c + j] gathered from HBM per 32-column
 //       block; the exact recombination is X's entry.  X overwrites the region (after a barrier,
 //       so every wave holds W first), k rows of nb words.
-template <int L, class Ar>
+template <int L, int NT, class Ar>
 __device__ void pivot_solve(const RJob& job, const RArgs& a, const Ar& ar, uint32_t* pan, uint32_t k, uint32_t c,
                             uint32_t nb, uint32_t r, bool planes, const uint32_t* s_P, const uint32_t* s_q,
                             uint32_t* s_inv) {
     constexpr int GS = 64;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 31, lg = lane >> 5;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
+    const uint32_t wave = scalar(tid >> 6);
     const uint32_t p = ar.p;
+    const rsrc_t sbuf = buffer_of(job.S, bytes_s(job)), ubuf = buffer_of(job.U, bytes_u(job));
     uint32_t* G0 = pan;
     uint32_t* G1 = pan + 32 * GS;
-    {   // K's k^2 <= 4 x 256 entries gathered with all loads in flight, then [K | I] stored
+    {   // K's k^2 <= 32^2 entries gathered with all loads in flight, then [K | I] stored
+        constexpr int KE = RW * RW / NT;
         const uint32_t kk = k * k;
-        uint32_t v[4];
+        uint32_t v[KE];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t idx = e * RT + tid, i = idx / k, j = idx - i * k;
-            v[e] = idx < kk ? job.A[(int64_t)s_P[i] * job.lda + c + s_q[j]] : 0u;
+        for (int e = 0; e < KE; ++e) {
+            const uint32_t idx = e * NT + tid, i = idx / k, j = idx - i * k;
+            v[e] = bload(sbuf, idx < kk ? s_P[i] * job.ld4 + 4 * (c + s_q[j]) : kDeadRow);
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t idx = e * RT + tid, i = idx / k, j = idx - i * k;
+        for (int e = 0; e < KE; ++e) {
+            const uint32_t idx = e * NT + tid, i = idx / k, j = idx - i * k;
             if (idx < kk) {
                 G0[i * GS + j] = v[e];
                 G0[i * GS + k + j] = i == j ? 1u : 0u;
@@ -226,8 +243,9 @@ __device__ void pivot_solve(const RJob& job, const RArgs& a, const Ar& ar, uint3
     // were eliminated, right columns > t are still identity columns).  A zero stays zero under
     // row_i <- v row_i - f row_t (row t is zero there too), so step t writes k + 1 entries per row:
     // left (t, k), right [0, t] (right column t read as zero in rows i != t) and the own entry
-    // (row t is zero at both own positions of a row i != t).  Eight threads share a row.
-    const uint32_t gi = tid >> 3, gsub = tid & 7;
+    // (row t is zero at both own positions of a row i != t).  NT / 32 threads share a row.
+    constexpr uint32_t GT = NT / RW;
+    const uint32_t gi = tid / GT, gsub = tid % GT;
     for (uint32_t t = 0; t < k; ++t) {
         const uint32_t* src = (t & 1) ? G1 : G0;
         uint32_t* dst = (t & 1) ? G0 : G1;
@@ -237,7 +255,7 @@ __device__ void pivot_solve(const RJob& job, const RArgs& a, const Ar& ar, uint3
             uint32_t* drow = dst + gi * GS;
             const uint32_t v = trow[t], f = srow[t], fneg = p - f, nl = k - t - 1;
             const bool upd = gi != t && f != 0;
-            for (uint32_t sl = gsub; sl <= k; sl += 8) {
+            for (uint32_t sl = gsub; sl <= k; sl += GT) {
                 const bool own = sl == k;
                 const uint32_t col = sl < nl ? t + 1 + sl : (!own ? k + (sl - nl) : (gi <= t ? gi : k + gi));
                 const uint32_t x = (col == k + t && gi != t) ? 0u : srow[col];
@@ -264,26 +282,26 @@ __device__ void pivot_solve(const RJob& job, const RArgs& a, const Ar& ar, uint3
     __syncthreads();                                  // every wave holds W: the region may be overwritten
     uint32_t* B = pan;
     const uint32_t ncb = (nb + 31) / 32;
-    for (uint32_t cb = wave; cb < ncb; cb += RT / 64) {
-        const uint32_t j = cb * 32 + lr;
+    uint32_t poff[16];                                // entry (s_P[t], c) for this lane's k-bytes
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t t2 = 16 * lg + i;
+        poff[i] = t2 < k ? s_P[t2] * job.ld4 + 4 * c : kDeadRow;
+    }
+    for (uint32_t cb = wave; cb < ncb; cb += NT / 64) {
+        const uint32_t j = cb * 32 + lr, j4 = j < nb ? 4 * j : kDeadCol;
         v4i fb[1][L];
-        split16<L>([&](int i) {
-            const uint32_t t2 = 16 * lg + i;
-            return (j < nb && t2 < k) ? job.A[(int64_t)s_P[t2] * job.lda + c + j] : 0u;
-        }, p, a.half, fb[0]);
+        split16<L>([&](int i) { return bload(sbuf, poff[i] + j4); }, p, a.half, fb[0]);
         uint32_t x[16];
         limb_small_product<L, 1>(fa, fb, sc, x);       // (rows at or past k: W's are zero, so is x)
-        if (j >= nb) continue;
-        uint32_t word[4][L];                          // limb bytes of rows g*8 + lg*4 .. +3, per plane
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const uint32_t t = (e / 4) * 8 + lg * 4 + (e % 4);
-            if (t < k) {
-                job.U[(size_t)(r + t) * job.n + c + j] = x[e];
-                if (!planes) B[t * nb + j] = x[e];
-            }
+            bstore(ubuf, (t < k ? 4 * ((r + t) * job.n + c) : kDeadRow) + j4, x[e]);
+            if (!planes && t < k && j < nb) B[t * nb + j] = x[e];
         }
-        if (planes) {
+        if (planes && j < nb) {
+            uint32_t word[4][L];                      // limb bytes of rows g*8 + lg*4 .. +3, per plane
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const uint32_t x4[4] = {x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3]};
@@ -301,14 +319,13 @@ __device__ void pivot_solve(const RJob& job, const RArgs& a, const Ar& ar, uint3
     __syncthreads();
 }
 
-template <class Ar, int L>
+template <class Ar, int L, int NT>
 __device__ void rref_one(const RJob& job, const Ar& ar, const RArgs& a, uint32_t* sm) {
-    __shared__ uint32_t s_cand[2][RT / 64];
+    __shared__ uint32_t s_cand[2][NT / 64];
     __shared__ uint32_t s_P[RW], s_q[RW], s_inv[RW];
-    __shared__ uint32_t s_keep[RT / 64];
+    __shared__ uint32_t s_keep[NT / 64];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t m = job.m, n = job.n, p = ar.p;
-    const int64_t lda = job.lda;
     uint32_t* pan = sm;
     uint32_t* list = sm + a.region;
     uint8_t* chosen = (uint8_t*)(list + a.mmax);
@@ -318,36 +335,38 @@ __device__ void rref_one(const RJob& job, const Ar& ar, const RArgs& a, uint32_t
     }
     uint32_t w = job.panel ? min((uint32_t)RW, job.panel) : (uint32_t)RW;
     while (w > 1 && ((uint64_t)m * (w | 1) > a.region || (uint64_t)w * n > a.region)) w >>= 1;
-    for (uint32_t i = tid; i < m; i += RT) list[i] = i;
+    for (uint32_t i = tid; i < m; i += NT) list[i] = i;
+    if (job.S != job.A)                                       // (the kernel addresses S by 32-bit byte offsets)
+        for (uint32_t i = wave; i < m; i += NT / 64)
+            for (uint32_t j = lane; j < n; j += 64) job.S[(size_t)i * n + j] = job.A[(int64_t)i * job.lda + j];
+    const rsrc_t sbuf = buffer_of(job.S, bytes_s(job));
     __syncthreads();
 
     uint32_t mu = m, r = 0;
     for (uint32_t c = 0; c < n && mu > 0; c += w) {
         const uint32_t wc = min(w, n - c), ws = wc | 1u, nb = n - c;
         // (a) panel of the unused rows, pivot search by the smallest-row rule
-        for (uint32_t i0 = 0; i0 < mu * wc; i0 += 8 * RT) {      // eight loads per thread in flight
+        for (uint32_t i0 = 0; i0 < mu * wc; i0 += 8 * NT) {      // eight loads per thread in flight
             uint32_t v[8], at[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const uint32_t idx = i0 + e * RT + tid;
-                if (idx < mu * wc) {
-                    const uint32_t u = wc == RW ? idx / RW : idx / wc, q = idx - u * wc;
-                    v[e] = job.A[(int64_t)list[u] * lda + c + q];
-                    at[e] = u * ws + q;
-                }
+                const uint32_t idx = i0 + e * NT + tid;
+                const uint32_t ic = min(idx, mu * wc - 1), u = wc == RW ? ic / RW : ic / wc, q = ic - u * wc;
+                v[e] = bload(sbuf, list[u] * job.ld4 + 4 * (c + q));
+                at[e] = u * ws + q;
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                if (i0 + e * RT + tid < mu * wc) pan[at[e]] = v[e];
+                if (i0 + e * NT + tid < mu * wc) pan[at[e]] = v[e];
         }
-        for (uint32_t u = tid; u < mu; u += RT) chosen[u] = 0;
+        for (uint32_t u = tid; u < mu; u += NT) chosen[u] = 0;
         __syncthreads();
         uint32_t k = 0;
         for (uint32_t q = 0; q < wc; ++q) {
-            // the wave's smallest candidate row: rounds of 256 rows in order, the lowest hit lane of
+            // the wave's smallest candidate row: rounds of NT rows in order, the lowest hit lane of
             // the first round with a hit (a wave-uniform loop)
             uint32_t best = 0xffffffffu;
-            for (uint32_t u0 = 0; u0 < mu; u0 += RT) {
+            for (uint32_t u0 = 0; u0 < mu; u0 += NT) {
                 const uint32_t u = u0 + tid;
                 const uint64_t bal = __ballot(u < mu && !chosen[u] && pan[u * ws + q] != 0);
                 if (bal) {
@@ -357,11 +376,14 @@ __device__ void rref_one(const RJob& job, const Ar& ar, const RArgs& a, uint32_t
             }
             if (lane == 0) s_cand[q & 1][wave] = best;
             __syncthreads();
-            const uint32_t bu = min(min(s_cand[q & 1][0], s_cand[q & 1][1]), min(s_cand[q & 1][2], s_cand[q & 1][3]));
+            uint32_t bu = s_cand[q & 1][0];
+#pragma unroll
+            for (int v = 1; v < NT / 64; ++v) bu = min(bu, s_cand[q & 1][v]);
+            bu = scalar(bu);
             if (bu == 0xffffffffu) continue;
             const uint32_t* prow = pan + bu * ws;
             const uint32_t v = prow[q];
-            for (uint32_t u = tid; u < mu; u += RT) {
+            for (uint32_t u = tid; u < mu; u += NT) {
                 if (u == bu) { chosen[u] = 1; continue; }
                 if (chosen[u]) continue;
                 uint32_t* row = pan + u * ws;
@@ -373,6 +395,7 @@ __device__ void rref_one(const RJob& job, const Ar& ar, const RArgs& a, uint32_t
             if (tid == 0) { s_P[k] = list[bu]; s_q[k] = q; }
             ++k;
         }
+        if (tid >= k && tid < RW) s_q[tid] = kDeadCol / 4;        // (times 4: a dead column's offset)
         __syncthreads();
         if (k == 0) continue;
 
@@ -383,11 +406,11 @@ __device__ void rref_one(const RJob& job, const Ar& ar, const RArgs& a, uint32_t
         // X's limb planes (L x nb x 32 bytes) replace X in LDS when they fit (then the trailing
         // pass reads its B fragments directly); X itself goes straight to U rows r .. r+k-1
         const bool planes = (uint64_t)8 * L * nb <= a.region;
-        pivot_solve<L>(job, a, ar, pan, k, c, nb, r, planes, s_P, s_q, s_inv);
+        pivot_solve<L, NT>(job, a, ar, pan, k, c, nb, r, planes, s_P, s_q, s_inv);
 
         // (d) trailing update of the other unused rows, S[i, j] -= sum_t S[i, J_t] X[t, j], and the
         // reduction of the stored pivot rows 0 .. r-1 against this panel's pivots (MFMA)
-        trailing_mfma<L>(job, a, B, planes, nb, wc, k, c, mu, list, chosen, s_q, r);
+        trailing_mfma<L, NT>(job, a, B, planes, nb, wc, k, c, mu, list, chosen, s_q, r);
         // (e) this panel's pivot rows are X, already in U rows r .. r+k-1 from column c on (the
         // final copy writes their zeros left of c); pivots, pivot rows
         if (tid < k) {
@@ -395,12 +418,12 @@ __device__ void rref_one(const RJob& job, const Ar& ar, const RArgs& a, uint32_t
             job.pivot_rows[r + tid] = s_P[tid];
         }
         __syncthreads();
-        // stable compaction of the unused list (chosen rows leave), 256 positions per round: a
+        // stable compaction of the unused list (chosen rows leave), NT positions per round: a
         // ballot per wave gives each kept row its place (writes only ever move left, past rows
         // this round has already read)
         {
             uint32_t base = 0;
-            for (uint32_t u0 = 0; u0 < mu; u0 += RT) {
+            for (uint32_t u0 = 0; u0 < mu; u0 += NT) {
                 const uint32_t u = u0 + tid;
                 const bool keep = u < mu && !chosen[u];
                 const uint32_t val = keep ? list[u] : 0u;
@@ -409,7 +432,7 @@ __device__ void rref_one(const RJob& job, const Ar& ar, const RArgs& a, uint32_t
                 __syncthreads();
                 uint32_t off = base, tot = 0;
 #pragma unroll
-                for (uint32_t w = 0; w < RT / 64; ++w) {
+                for (uint32_t w = 0; w < NT / 64; ++w) {
                     off += w < wave ? s_keep[w] : 0u;
                     tot += s_keep[w];
                 }
@@ -427,8 +450,8 @@ __device__ void rref_one(const RJob& job, const Ar& ar, const RArgs& a, uint32_t
     __syncthreads();
 
     // the RREF over the job's matrix: rank rows of U, then zero rows
-    for (uint32_t i = wave; i < m; i += RT / 64) {          // a wave per row, four words per lane in flight
-        uint32_t* Ai = job.A + (int64_t)i * lda;
+    for (uint32_t i = wave; i < m; i += NT / 64) {          // a wave per row, four words per lane in flight
+        uint32_t* Ai = job.A + (int64_t)i * job.lda;
         const uint32_t* Ui = job.U + (size_t)i * n;
         const uint32_t c0 = i < r ? list[m - 1 - i] : n;     // zeros left of the row's panel
         for (uint32_t j0 = lane; j0 < n; j0 += 256) {
@@ -444,17 +467,18 @@ __device__ void rref_one(const RJob& job, const Ar& ar, const RArgs& a, uint32_t
     __syncthreads();
 }
 
-template <class Ar, int L>
-__global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2, 8))) void rref_batch_kernel(RArgs a, Ar ar) {
+template <class Ar, int L, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 8))) void rref_batch_kernel(RArgs a, Ar ar) {
     extern __shared__ __attribute__((aligned(16))) uint32_t sm[];
     __shared__ uint32_t s_job;
     for (;;) {
         if (threadIdx.x == 0) s_job = atomicAdd(a.next, 1u);
         __syncthreads();
-        const uint32_t jj = s_job;
+        const uint32_t jj = scalar(s_job);   // the job is scalar data
         __syncthreads();
         if (jj >= a.njobs) break;
-        rref_one<Ar, L>(a.jobs[a.order[jj]], ar, a, sm);
+        const RJob job = a.jobs[scalar(a.order[jj])];
+        rref_one<Ar, L, NT>(job, ar, a, sm);
     }
 }
 
@@ -473,11 +497,32 @@ struct RBatch {
     uint32_t region = 0, mmax = 0, nmax = 0;
     size_t lds = 0;
     uint32_t grid = 0;
+    uint32_t nt = 256;                  // threads per workgroup (256 or 512)
     uint32_t per_cu = 1;                // workgroups per CU the LDS size was chosen for (1 or 2)
     uint32_t planes_out = 0;            // jobs whose first panel keeps X's limb planes outside LDS
 };
 
 constexpr size_t kLdsCap = 156 * 1024;
+
+uint32_t limbs_of(uint32_t p) { return p <= 255u ? 1 : (p <= 65279u ? 2 : (p <= 16711423u ? 3 : 4)); }
+
+template <class Ar, int L>
+const void* batch_kernel_nt(uint32_t nt) {
+    return nt == 256 ? (const void*)rref_batch_kernel<Ar, L, 256> : (const void*)rref_batch_kernel<Ar, L, 512>;
+}
+template <class Ar>
+const void* batch_kernel_l(uint32_t limbs, uint32_t nt) {
+    switch (limbs) {
+        case 1: return batch_kernel_nt<Ar, 1>(nt);
+        case 2: return batch_kernel_nt<Ar, 2>(nt);
+        case 3: return batch_kernel_nt<Ar, 3>(nt);
+        default: return batch_kernel_nt<Ar, 4>(nt);
+    }
+}
+// The kernel of a modulus (its arithmetic and its limb count, the MFMA fragments' size) and a workgroup size.
+const void* batch_kernel(uint32_t p, uint32_t nt) {
+    return (p & 1u) ? batch_kernel_l<ArMont>(limbs_of(p), nt) : batch_kernel_l<ArBarrett>(limbs_of(p), nt);
+}
 
 }  // namespace
 
@@ -519,7 +564,11 @@ int rref_batch_create_impl(const hx_modctx& ctx, const hx_rref_job* jobs, uint32
             HX_CHECK(j.m <= 4096, "rref job: m > 4096 (use hx_rref_u32)");
             HX_CHECK(j.rank != nullptr, "rref job: rank is NULL");
             HX_CHECK(j.panel == 0 || j.panel == 8 || j.panel == 16 || j.panel == 32, "rref job: panel must be 0, 8, 16 or 32");
-            hj[i] = RJob{j.m, j.n, j.A, j.lda, j.pivots, j.pivot_rows, j.rank, nullptr, j.panel};
+            const bool copy = j.m > 1 && ((uint64_t)j.lda > kMaxBytes / 4 ||
+                                          (uint64_t)(j.m - 1) * (uint64_t)j.lda + j.n > kMaxBytes / 4);
+            hj[i] = RJob{j.m, j.n, j.A, j.lda, j.pivots, j.pivot_rows, j.rank, nullptr,
+                         copy ? nullptr : j.A, (uint32_t)(4 * (copy ? (int64_t)j.n : j.lda)), j.panel};
+            if (copy) ucount += (size_t)j.m * j.n;
             ucount += (size_t)std::min(j.m, j.n) * j.n;
             mmax = std::max(mmax, j.m);
             nmax = std::max(nmax, j.n);
@@ -555,8 +604,7 @@ int rref_batch_create_impl(const hx_modctx& ctx, const hx_rref_job* jobs, uint32
         b->lds = (size_t)b->region * 4 + fixed;
         {
             // the kernel's own test (X's limb planes in LDS iff 8 L nb <= region, nb = n - c) at c = 0
-            const uint32_t pp = ctx.p;
-            const uint32_t L = pp <= 255u ? 1 : (pp <= 65279u ? 2 : (pp <= 16711423u ? 3 : 4));
+            const uint32_t L = limbs_of(ctx.p);
             for (const RJob& jj : hj)
                 if (jj.m && jj.n && (uint64_t)8 * L * jj.n > b->region) ++b->planes_out;
         }
@@ -565,6 +613,10 @@ int rref_batch_create_impl(const hx_modctx& ctx, const hx_rref_job* jobs, uint32
         for (uint32_t i = 0; i < njobs; ++i) {
             hj[i].U = b->d_U + off;
             off += (size_t)std::min(hj[i].m, hj[i].n) * hj[i].n;
+            if (hj[i].S == nullptr && hj[i].m) {
+                hj[i].S = b->d_U + off;
+                off += (size_t)hj[i].m * hj[i].n;
+            }
         }
         std::vector<uint32_t> order(njobs);
         std::iota(order.begin(), order.end(), 0u);
@@ -584,17 +636,17 @@ int rref_batch_create_impl(const hx_modctx& ctx, const hx_rref_job* jobs, uint32
         int cus = 256;
         hipDeviceProp_t prop;
         if (hipGetDeviceProperties(&prop, 0) == hipSuccess) cus = prop.multiProcessorCount;
+        // 512 threads a job where single jobs decide: every job has a compute unit of its own, or the work is
+        // below 96 of the largest job.  Otherwise two jobs of 256 threads share a compute unit (registers: two
+        // waves a SIMD), which is the better throughput (ms on 256 / 512 threads, work in largest jobs in
+        // brackets; jobs of 16..512: 4096 [148] 2.20 / 3.34, 2048 [81] 2.05 / 1.70, 512 [23] 2.04 / 1.56; of 16..128:
+        // 4096 [354] 0.77 / 1.32, 512 [50] 0.30 / 0.27; 512 x 512: 512 jobs 3.12 / 3.83, 256 jobs 2.46 / 1.92, one
+        // 2.29 / 1.74).
+        b->nt = !two_per_cu && (njobs <= (uint32_t)cus || wsum <= 96.0 * wmax) ? 512 : 256;
+        const void* kern = batch_kernel(ctx.p, b->nt);
+        (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsCap);
         const uint32_t per_cu = std::max<uint32_t>(1, (uint32_t)(160 * 1024 / std::max<size_t>(b->lds, 1)));
         b->grid = std::max<uint32_t>(1, std::min<uint32_t>(njobs, (uint32_t)cus * std::min<uint32_t>(per_cu, 4)));
-        static bool attr_done = false;
-        if (!attr_done) {
-            for (const void* f : {(const void*)rref_batch_kernel<ArMont, 1>, (const void*)rref_batch_kernel<ArMont, 2>,
-                                  (const void*)rref_batch_kernel<ArMont, 3>, (const void*)rref_batch_kernel<ArMont, 4>,
-                                  (const void*)rref_batch_kernel<ArBarrett, 1>, (const void*)rref_batch_kernel<ArBarrett, 2>,
-                                  (const void*)rref_batch_kernel<ArBarrett, 3>, (const void*)rref_batch_kernel<ArBarrett, 4>})
-                (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsCap);
-            attr_done = true;
-        }
     } catch (...) {
         rref_batch_destroy_impl(b);
         throw;
@@ -620,22 +672,14 @@ int rref_batch_run_impl(void* vb, hipStream_t s) {
     a.M = devmod(b->ctx);
     a.inv = 1.0 / (double)b->ctx.p;
     a.half = (b->ctx.p - 1) / 2;
-    const uint32_t pp = b->ctx.p;                       // limbs from p itself (balanced digits)
-    a.L = pp <= 255u ? 1 : (pp <= 65279u ? 2 : (pp <= 16711423u ? 3 : 4));
-    // one kernel per limb count (the MFMA fragments' size is a compile-time constant)
-    auto launch = [&](auto ar) {
-        using Ar = decltype(ar);
-        switch (a.L) {
-            case 1: rref_batch_kernel<Ar, 1><<<b->grid, RT, b->lds, s>>>(a, ar); break;
-            case 2: rref_batch_kernel<Ar, 2><<<b->grid, RT, b->lds, s>>>(a, ar); break;
-            case 3: rref_batch_kernel<Ar, 3><<<b->grid, RT, b->lds, s>>>(a, ar); break;
-            default: rref_batch_kernel<Ar, 4><<<b->grid, RT, b->lds, s>>>(a, ar); break;
-        }
-    };
+    ArMont mont = {};
+    ArBarrett barrett = {};
     if (b->ctx.p & 1u)
-        launch(make_mont(b->ctx.p));
+        mont = make_mont(b->ctx.p);
     else
-        launch(make_barrett(b->ctx.p));
+        barrett = make_barrett(b->ctx.p);
+    void* args[] = {&a, (b->ctx.p & 1u) ? (void*)&mont : (void*)&barrett};
+    HX_HIP(hipLaunchKernel(batch_kernel(b->ctx.p, b->nt), dim3(b->grid), dim3(b->nt), args, b->lds, s));
     after_launch("rref_batch_kernel");
     return HX_OK;
 }

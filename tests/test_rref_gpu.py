@@ -102,3 +102,47 @@ def test_rref_batch_graph_replay(hx_gpu, O):
             for A, M, res in zip(inputs, work, b.results()):
                 _check(O, p, A, res, E.from_device(M), f"replay {rep} {A.shape}")
         _lib.check(_lib.lib().hx_graph_destroy(g))
+
+
+@pytest.mark.parametrize("p", [2, 251, 65521, 1000003, 2147483647])
+@pytest.mark.parametrize("mode", ["few", "many"])
+def test_rref_batch_workgroups(hx_gpu, O, p, mode):
+    """Jobs of 512 threads (few jobs) and of 256 (two on a compute unit) at the edges of panels and of the row
+    rounds, as windows of wider matrices; the entries around each window stay."""
+    from hacs_amd import engine as E
+    from hacs_amd import _lib
+    ctx = E.ModCtx(p)
+    rng = np.random.default_rng(p + 1)
+    shapes = [(1, 33), (31, 32), (32, 31), (33, 65), (64, 64), (255, 40), (257, 96), (511, 33), (513, 64), (40, 520)]
+    inputs = [make(rng, m, n, p, KINDS[i % len(KINDS)], rank=max(1, min(m, n) * 2 // 3)) for i, (m, n) in enumerate(shapes)]
+    hulls = []
+    for A in inputs:
+        H = np.full((A.shape[0] + 2, A.shape[1] + 5), 0xDEADBEEF, np.uint32)
+        H[1:-1, 3:-2] = A
+        hulls.append(E.to_device(H))
+    b = E.RrefBatch(ctx, [H[1:-1, 3:-2] for H in hulls],
+                    mode=_lib.HX_RREF_BATCH_AUTO if mode == "few" else _lib.HX_RREF_BATCH_TWO_PER_CU)
+    b.run()
+    b.status()
+    torch.cuda.synchronize()
+    for A, H, res in zip(inputs, hulls, b.results()):
+        out = E.from_device(H)
+        _check(O, p, A, res, out[1:-1, 3:-2], f"p={p} {mode} {A.shape}")
+        out[1:-1, 3:-2] = 0xDEADBEEF
+        assert (out == 0xDEADBEEF).all(), f"p={p} {mode} {A.shape}: entries around the window"
+
+
+def test_rref_batch_far_rows(hx_gpu, O):
+    """Rows farther apart than 32-bit byte offsets reach: the job is eliminated in a copy."""
+    from hacs_amd import engine as E
+    p, ld = 1000003, (1 << 29) + 4
+    rng = np.random.default_rng(3)
+    A = make(rng, 3, 40, p, "planted", rank=2)
+    flat = torch.empty(2 * ld + 40, dtype=torch.int32, device="cuda")
+    M = flat.as_strided((3, 40), (ld, 1))
+    M.copy_(E.to_device(A))
+    b = E.RrefBatch(E.ModCtx(p), [M])
+    b.run()
+    b.status()
+    torch.cuda.synchronize()
+    _check(O, p, A, b.results()[0], E.from_device(M.contiguous()), "far rows")
