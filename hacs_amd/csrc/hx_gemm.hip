@@ -1427,9 +1427,9 @@ __global__ __launch_bounds__(256) void crt_kernel(CrtArgs a) {
 // pipelined against the MFMAs (limb3_kernel), 4 = limb3's pipeline on eight waves
 // (limb4_kernel), 5 = the 96 x 128 tile on twelve waves (limb5_kernel); 0 = the default.
 constexpr int kLimbDefault = 4;
-// (internal) limb kernel 4 on 64 x 64 tiles, the default's choice where the 64 x 128 tiles are fewer than the units
-// (64 x 128 / 64 x 64, us a call: 1024^3 mod 65521 36 / 31, mod 2147483629 51 / 45; 512^2 x 8192 193 / 120; 2048^3, 512
-// wide tiles, 146 / 147)
+// (internal) limb kernel 4 on 64 x 64 tiles, the default's choice where those still find a compute unit each, up to
+// 128 tiles of 64 x 128 (64 x 128 / 64 x 64, us a call: 128 tiles, 1024^3 mod 65521 34 / 29, mod 2147483629 48 / 42;
+// 32 tiles, 512^2 x 8192 193 / 120; 130 tiles, 795 x 1202 x 645 40 / 45; 252 tiles, 1103 x 1788 x 139 25 / 32)
 constexpr int kLimb4Narrow = 40;
 inline int limb_version(int tile) { return tile >= 1 && tile <= 5 ? tile : kLimbDefault; }
 // tile 6 of the limb variant: the residue route (res_gemm_kernel) in place of the limb kernels
@@ -1633,7 +1633,7 @@ void gemm_limb(const hx_modctx& ctx, const GemmArgs& g0, hipStream_t s, void* ws
         la.M = devmod(ctx);
         const bool last = k0 + kc >= g.k;
         int ver = limb_version(tile);
-        if (tile == 0 && la.ntm * la.ntn < 256) ver = kLimb4Narrow;
+        if (tile == 0 && la.ntm * la.ntn <= 128) ver = kLimb4Narrow;
         if (ev0 && k0 == 0) HX_HIP(hipEventRecord(ev0, s));
         switch (L) {
             case 1: launch_limb<1>(la, s, ver); break;
@@ -1675,29 +1675,37 @@ size_t residue_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t nmod
 }
 
 // Whether the automatic choice splits a thin deep product over K on the plain kernel: its limb tiles cannot fill
-// the GPU (256 x 256 x 65536: plain split 64 ways 0.87 ms, limb route 1.50 ms, plain unsplit 11.7 ms).
+// the GPU (256 x 256 x 65536: plain split 64 ways 0.87 ms, limb route 1.50 ms, plain unsplit 11.7 ms).  To
+// k = 8192 the matrix units win all the same (us, split plain / limb or residue route, mod 1000003: 100 x 100 x 1200
+// 77 / 25, 300 x 300 x 1800 107 / 33, 256 x 256 x 4096 112 / 44, 64 x 64 x 8192 162 / 57).
 bool auto_splits(uint32_t m, uint32_t n, uint32_t k) {
     const uint64_t limb_tiles = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
-    return limb_tiles < 32 && plain_suggest_splits(m, n, k) > 1;
+    return k > 8192 && limb_tiles < 32 && plain_suggest_splits(m, n, k) > 1;
 }
 
 // The moduli count of the residue route when this product takes it, else 0.  It needs host-side sizes,
 // 1 <= k <= RES_KMAX and enough moduli; tile kResidueTile asks for it wherever it applies.  The limb variant's
 // default (tile 0) takes it where it runs at most L^2 - 4 int8 products (four-limb moduli: 10 or 11 for 16) and
 // m, n, k >= 4096.  The automatic variant takes it at every m, n once k is deep enough to pay for the splits
-// and the CRT, whose cost does not grow with k: k >= 1536, and k >= 768 for four limbs where the limb kernel's
-// 64 x 128 tiles fill the units, as its 64 x 64 tiles are the better ones below (us, limb kernel 4 / residue
-// route; mod 2147483629: 768^3 33 / 40, 1024^3 45 / 48, 1677 x 1419 x 2049 133 / 114, 512^2 x 8192 120 / 80, 2048^3
-// 147 / 145, 4096^3 990 / 760, 8192^3 7400 / 5200, 8192^2 x 512 600 / 680, x 1024 1131 / 953; mod 65521: 2048^3
-// 96 / 96, 4096^3 596 / 473, 512^2 x 8192 85 / 65, 8192^2 x 512 421 / 480; mod 1000003: 2048^3 107 / 109, 4096^3
-// 675 / 550).  Two-limb moduli stay on the limb kernels (mod 61001: 2048^2 x 1024 49 / 66, 8192^2 x 1024 411 / 670).
+// and the CRT, whose cost does not grow with k, for three and four limbs: from 256 tiles of 64 x 128 on from
+// k = 1536 / 768 (us, limb kernel 4 / residue route; mod 2147483629: 1500^2 x 1600 110 / 86, 1677 x 1419 x 2049
+// 133 / 114, 2048^3 147 / 145, 4096^3 990 / 760, 8192^3 7400 / 5200, 8192^2 x 512 600 / 680, x 1024 1131 / 953; mod
+// 65521: 1500^2 x 1600 77 / 62, 2048^3 96 / 96, 4096^3 596 / 473, 8192^2 x 512 421 / 480), and up to 64 tiles from
+// k = 2560 / 1536, where its ten products fill units that the limb kernel leaves idle (mod 2147483629: 512^2 x
+// 1600 46 / 41, x 5000 86 / 62; mod 65521: 512^2 x 1600 34 / 36, x 3000 47 / 43).  Between them the limb kernels have
+// one tile for each unit and the residue route the tiles' remainders of ten products (mod 2147483629: 1024^2 x
+// 2000 58 / 67, x 5000 104 / 119, 7033 x 34 x 3000 85 / 126, 1280^2 x 3000 98 / 103).  Two-limb moduli stay on the limb
+// kernels (mod 61001: 2048^2 x 1024 49 / 66, 8192^2 x 1024 411 / 670).
 uint32_t residue_choice(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, bool device_sizes, int tile,
                         bool automatic) {
     if (device_sizes || (tile != 0 && tile != kResidueTile)) return 0;
     const uint32_t N = residue_moduli(ctx.p, k);
     if (N == 0 || tile == kResidueTile) return N;
     const uint64_t limb_tiles = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
-    if (automatic && ctx.limbs >= 3 && k >= (ctx.limbs == 4 && limb_tiles >= 256 ? 768u : 1536u)) return N;
+    if (automatic && ctx.limbs >= 3) {
+        if (limb_tiles >= 256 && k >= (ctx.limbs == 4 ? 768u : 1536u)) return N;
+        if (limb_tiles <= 64 && k >= (ctx.limbs == 4 ? 1536u : 2560u)) return N;
+    }
     const bool large = m >= 4096 && n >= 4096 && k >= 4096;
     return large && ctx.limbs > 0 && N + 4 <= ctx.limbs * ctx.limbs ? N : 0;
 }

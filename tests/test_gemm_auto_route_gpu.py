@@ -21,8 +21,10 @@ def _draw(p, m, n, seed, form):
 
 
 @pytest.mark.parametrize("p,n,k,route", [(2147483629, 2048, 767, 4), (2147483629, 2048, 768, 6), (4278124259, 1500, 1000, 6),
-                                         (2147483629, 700, 1535, 4), (2147483629, 700, 1536, 6),
-                                         (65521, 2048, 1535, 4), (65521, 700, 1536, 6), (61001, 700, 2000, 4)])
+                                         (65521, 2048, 1535, 4), (65521, 1500, 1536, 6), (61001, 700, 2000, 4),
+                                         (2147483629, 500, 1535, 4), (2147483629, 500, 1536, 6), (65521, 500, 2559, 4),
+                                         (65521, 500, 2560, 6), (2147483629, 1024, 5000, 4), (65521, 256, 2000, 4),
+                                         (65521, 256, 8192, 6), (65521, 256, 8193, 0)])
 def test_auto_route_rule(p, n, k, route):
     from hacs_amd import engine as E
     assert E.gemm_route(E.ModCtx(p), n, n, k, E.HX_GEMM_AUTO) == route
@@ -31,7 +33,7 @@ def test_auto_route_rule(p, n, k, route):
 @pytest.mark.parametrize("p", [251, 61001, 65521, 2147483629, 4278124259])
 @pytest.mark.parametrize("m,n,k", [(200, 300, 129), (64, 64, 1000), (65, 129, 1023), (1000, 700, 500)])
 def test_narrow_limb_tiles(hx_gpu, p, m, n, k):
-    """Limb kernel 4 on 64 x 64 tiles (the default below 256 wide tiles) against the wide ones (tile 4)."""
+    """Limb kernel 4 on 64 x 64 tiles (the default up to 128 wide tiles) against the wide ones (tile 4)."""
     from hacs_amd import engine as E
     ctx = E.ModCtx(p)
     A, B = _draw(p, m, k, 1, "row"), _draw(p, k, n, 2, "row")
@@ -44,7 +46,7 @@ def test_narrow_limb_tiles(hx_gpu, p, m, n, k):
 
 @pytest.mark.parametrize("fa,fb,fc", [("row", "row", "row"), ("col", "col", "col"), ("window", "row", "window"),
                                       ("row", "window", "row"), ("step", "col", "step"), ("col", "step", "row")])
-@pytest.mark.parametrize("p,m,n,k", [(2147483629, 515, 700, 1540), (65521, 640, 513, 1537), (1000003, 1025, 257, 1600),
+@pytest.mark.parametrize("p,m,n,k", [(2147483629, 515, 700, 1540), (65521, 640, 513, 2561), (1000003, 1025, 257, 2600),
                                      (2147483647, 1793, 2049, 833)])      # the last: 256 x 256 tiles
 def test_auto_route_equals_plain(hx_gpu, p, m, n, k, fa, fb, fc):
     from hacs_amd import engine as E
