@@ -22,7 +22,7 @@
 //    The operands are split into limb planes once per call (limb_prep_kernel, HBM-bound:
 //    4 bytes in, L bytes out per element), so the MFMA loop streams int8 planes only.
 //
-// No floating point anywhere; no atomics on results.
+// Every result is exact (floating point only finds quotients, with proven bounds); no atomics on results.
 #include "hx_gemm.h"
 #include "hx_limbs.h"
 #include "hx_residue.h"

@@ -25,16 +25,16 @@
 //        S'[i, :] = S[R_i, W:] - S[R_i, J] X[:, W:]
 //     as k <= 32 products on the INT8 matrix cores (upd32_kernel: A's limbs split on the fly, X's
 //     from its limb planes) with a row gather on A and C_in, a column gather on A, and output into
-//     the other S buffer (compaction for free).  Lookahead: the next panel's W columns are computed first on
-//     the caller's stream, the rest on a second stream, overlapping the next panel's tournament
-//     (which reads only those W columns); the next panel's step 2 waits for it.  P, J and the
-//     update's sizes are double-buffered by panel parity for the overlap.
+//     the other S buffer (compaction for free).  The next panel's W columns are computed
+//     in a launch of their own; the rest of the update shares a launch with the next panel's pivot
+//     search, which reads only those W columns (rrp_step_kernel).  P, J and the update's sizes are
+//     double-buffered by panel parity for the overlap.
 //  4. Gauss-Jordan: the pivot rows stored so far (U rows 0 .. r-1) are reduced against the panel's
-//     pivots, U[0:r, c:n] -= U[0:r, c + J] X, on the second stream after the rest of the update
-//     (their panel columns gathered first, since the product overwrites them); X is exactly the
-//     identity at J, so those entries become zero.  When the last panel is done the U rows are the
-//     RREF's rows.  The X copy is double-buffered by panel parity, so the next panel's X does not
-//     overwrite the one this product reads.
+//     pivots, U[0:r, c:n] -= U[0:r, c + J] X, in that same launch (their panel columns gathered before,
+//     by X's launch, since the product overwrites them); X is exactly the identity at J, so those
+//     entries become zero.  When the last panel is done the U rows are the RREF's rows.
+//     The X copy is double-buffered by panel parity, so the next panel's X does not overwrite the
+//     one this product reads.
 //  All sizes (m_a, k, r) live in device memory; the host only knows upper bounds, so a panel is a
 //  fixed sequence of launches.
 #include <algorithm>
