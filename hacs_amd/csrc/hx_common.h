@@ -8,6 +8,8 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <memory>
+#include <mutex>
 #include <string>
 
 #include "../../include/hacs_mi355x.h"
@@ -106,11 +108,28 @@ void rref_stacked(uint32_t m, uint64_t* A, size_t row_words, uint32_t cap, uint3
 void arena_free(void* p);
 // Whether s is being captured into a graph (then nothing may be allocated or freed for it).
 bool stream_capturing(hipStream_t s);
-// Library-owned scratch of at least `bytes`, private to stream s and one purpose (below); grows
-// (after waiting for s) but never shrinks; nullptr when it would have to grow inside a capture.
+// Library-owned scratch of at least `bytes`, one buffer per device, stream and purpose; it grows (after waiting
+// for s) but never shrinks.  The lease holds the buffer's lock: a caller keeps it from before the first launch
+// that uses the buffer until after the last, so the launches of two host threads on one stream do not mix (split,
+// split, product, product) and no buffer is replaced under a call that still launches on it.  ptr is nullptr, and
+// nothing is held, when the buffer would have to grow inside a capture.  Leases of one purpose do not nest.
 enum ScratchPurpose { SCRATCH_LIMB = 0, SCRATCH_MLP = 1, SCRATCH_RREF = 2, SCRATCH_SPLIT = 3, SCRATCH_PACKED = 4,
                       SCRATCH_U64 = 5 };
-void* stream_scratch(hipStream_t s, int purpose, size_t bytes);
+struct ScratchSlot {
+    std::mutex mu;               // held by the lease
+    void* ptr = nullptr;
+    size_t bytes = 0;
+};
+struct ScratchLease {
+    std::shared_ptr<ScratchSlot> slot;
+    std::unique_lock<std::mutex> held;
+    void* ptr = nullptr;
+};
+ScratchLease stream_scratch(hipStream_t s, int purpose, size_t bytes);
+// Whether a call that can also run without scratch may take it on s: not inside a capture (a graph would keep
+// the address of a buffer that a later call may replace), and not on hipStreamPerThread (one handle for a stream
+// of every host thread).
+bool stream_scratch_safe(hipStream_t s);
 void stream_scratch_release(hipStream_t s);
 // A rows x width-byte block between pageable host memory and the device (either direction, pitches in
 // bytes) through the runtime's pinned staging chunks, ordered on st; returns once it has landed.

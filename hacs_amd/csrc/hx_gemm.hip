@@ -1866,6 +1866,7 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
     // against 97 us)
     if (automatic && variant == HX_GEMM_PLAIN && ctx.limbs > 0 && !split && splits <= 1 && g.k > 256 && g.m_dev == nullptr && g.k_dev == nullptr)
         variant = HX_GEMM_LIMB;
+    ScratchLease planes, partials;   // the library's own workspaces, held until the product is launched
     uint32_t rn = 0;            // moduli of the residue route, 0 = the limb kernels
     if (variant == HX_GEMM_LIMB && g.m != 0 && g.n != 0)
         rn = residue_choice(ctx, g.m, g.n, g.k, g.m_dev != nullptr || g.k_dev != nullptr, tile, automatic);
@@ -1875,14 +1876,13 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
         const bool asked = tile == kResidueTile;
         const size_t need = residue_workspace_bytes(g.m, g.n, g.k, rn);
         if (ws == nullptr) {
-            void* own = nullptr;
             try {
-                own = stream_scratch(s, SCRATCH_LIMB, need);
+                planes = stream_scratch(s, SCRATCH_LIMB, need);
             } catch (const Error& e) {
                 if (asked || e.code != HX_E_NOMEM) throw;
             }
-            if (own != nullptr) {
-                ws = own;
+            if (planes.ptr != nullptr) {
+                ws = planes.ptr;
                 ws_bytes = need;
             } else if (asked) {
                 throw Error{HX_E_CAPTURE, "the residue route needs a caller workspace inside a stream capture "
@@ -1900,7 +1900,8 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
             // library-owned planes private to this stream (never shared with another stream); inside a
             // capture they can only be used when they are already large enough
             const size_t need = limb_workspace_bytes(ctx, g.m, g.n, g.k);
-            ws = stream_scratch(s, SCRATCH_LIMB, need);
+            planes = stream_scratch(s, SCRATCH_LIMB, need);
+            ws = planes.ptr;
             ws_bytes = ws ? need : 0;
             if (ws == nullptr && !automatic)
                 throw Error{HX_E_CAPTURE, "the limb route needs a caller workspace inside a stream capture "
@@ -1922,7 +1923,8 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
             const size_t need = plain_split_workspace_bytes(g.m, g.n, sp);
             if (split_ws == nullptr) {
                 // library-owned partials private to this stream; inside a capture only when already large enough
-                split_ws = stream_scratch(s, SCRATCH_SPLIT, need);
+                partials = stream_scratch(s, SCRATCH_SPLIT, need);
+                split_ws = partials.ptr;
                 split_ws_bytes = split_ws ? need : 0;
                 if (split_ws == nullptr && !auto_split)
                     throw Error{HX_E_CAPTURE, "split-K needs a caller workspace inside a stream capture "

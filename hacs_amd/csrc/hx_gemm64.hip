@@ -327,7 +327,7 @@ constexpr size_t RES64_WS = (size_t)4 << 30;      // bytes of planes held at a t
 
 // C op= A B by the residue route; false, with nothing launched, where it does not apply.
 bool gemm64_residue(const hx_modctx64& ctx, const Gemm64Args& g, hipStream_t s) {
-    if (g.k == 0 || stream_capturing(s)) return false;
+    if (g.k == 0 || !stream_scratch_safe(s)) return false;
     auto up = [](uint64_t x, uint64_t a) { return (x + a - 1) / a * a; };
     const uint64_t p = ctx.p;
     const uint32_t kc = std::min<uint32_t>(g.k, RES_KMAX / 64 * 64), N = moduli64(p, kc);
@@ -337,13 +337,14 @@ bool gemm64_residue(const hx_modctx64& ctx, const Gemm64Args& g, hipStream_t s) 
     uint64_t mb = up(g.m, side), nb = up(g.n, side);
     auto bytes = [&] { return N * (mb * Kp0 + nb * Kp0 + mb * nb); };
     while (bytes() > RES64_WS && (mb > side || nb > side)) (mb >= nb ? mb : nb) = up((mb >= nb ? mb : nb) / 2, side);
-    char* ws;
+    ScratchLease planes;                         // held until every block is launched
     try {
-        ws = (char*)stream_scratch(s, SCRATCH_U64, bytes());
+        planes = stream_scratch(s, SCRATCH_U64, bytes());
     } catch (const Error& e) {
         if (e.code != HX_E_NOMEM) throw;
         return false;
     }
+    char* const ws = (char*)planes.ptr;
     if (ws == nullptr) return false;
 
     Split64 sp{};

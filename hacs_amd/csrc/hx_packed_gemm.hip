@@ -305,7 +305,7 @@ inline uint64_t up(uint64_t x, uint64_t a) { return (x + a - 1) / a * a; }
 template <int P>
 bool packed_gemm(uint32_t m, uint32_t n, uint32_t k, const uint64_t* A, uint32_t lda, const uint64_t* B, uint32_t ldb,
                  uint64_t* C, uint32_t ldc, bool accumulate, hipStream_t s) {
-    if (m == 0 || n == 0 || k == 0 || stream_capturing(s)) return false;
+    if (m == 0 || n == 0 || k == 0 || !stream_scratch_safe(s)) return false;
     // the 128 x 128 tile where 256 x 256 tiles would leave compute units idle
     const bool small = up(m, 256) / 256 * (up(n, 256) / 256) < 256;
     const uint64_t tile = small ? 128 : 256, Mp = up(m, tile), Np = up(n, tile);
@@ -313,13 +313,14 @@ bool packed_gemm(uint32_t m, uint32_t n, uint32_t k, const uint64_t* A, uint32_t
     const uint64_t fit = PG_WS / (Mp + Np) * 2 / 128 * 128;                     // k whose planes fit PG_WS
     if (fit == 0) return false;
     const uint32_t chunk = (uint32_t)std::min<uint64_t>({up(k, 128), fit, PG_KMAX});
-    uint8_t* ws;
+    ScratchLease planes;                         // held until every chunk is launched
     try {
-        ws = (uint8_t*)stream_scratch(s, SCRATCH_PACKED, (Mp + Np) * (chunk / 2));
+        planes = stream_scratch(s, SCRATCH_PACKED, (Mp + Np) * (chunk / 2));
     } catch (const Error& e) {
         if (e.code != HX_E_NOMEM) throw;
         return false;
     }
+    uint8_t* const ws = (uint8_t*)planes.ptr;
     if (ws == nullptr) return false;
     const uint32_t nw = (n + 63) / 64;
     for (uint64_t k0 = 0; k0 < k; k0 += chunk) {

@@ -8,6 +8,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -79,14 +81,15 @@ const Avail& avail() {
 
 // ---- device arena (the caching allocator of Cuda/CudaCtx.h:104-168, designed afresh) ----------
 // Blocks are rounded up to a granule (512 B below 1 MiB, 2 MiB above) and cached on free in
-// exact-size free lists; a request first takes a cached block of its rounded size.  A failed
+// exact-size free lists of their device; a request first takes a cached block of its rounded size.  A failed
 // hipMalloc is answered by a trim (every cached block returned to the driver) and one retry.
 // Nothing here is legal inside a stream capture (hipMalloc / hipFree are not): callers allocate
 // before a capture begins.
 struct Arena {
     std::mutex mu;
-    std::unordered_map<size_t, std::vector<void*>> free_lists;   // rounded size -> cached blocks
-    std::unordered_map<void*, size_t> live;                      // block -> rounded size
+    using Kind = std::pair<int, size_t>;                         // device, rounded size
+    std::map<Kind, std::vector<void*>> free_lists;               // cached blocks
+    std::unordered_map<void*, Kind> live;                        // block -> its kind
     hx_arena_stats st{};
 };
 Arena& arena() {
@@ -104,8 +107,8 @@ size_t arena_trim_locked(Arena& a) {
     for (auto& kv : a.free_lists) {
         for (void* p : kv.second) {
             (void)hipFree(p);
-            freed += kv.first;
-            a.st.reserved_bytes -= kv.first;
+            freed += kv.first.second;
+            a.st.reserved_bytes -= kv.first.second;
             ++a.st.driver_frees;
         }
         kv.second.clear();
@@ -115,23 +118,29 @@ size_t arena_trim_locked(Arena& a) {
 }
 
 // ---- per-stream library scratch --------------------------------------------------------------
-// One buffer per (stream, purpose): work queued on a stream only ever uses that stream's buffer,
-// so calls on different streams never share bytes.  A buffer grows by first waiting for the work
-// already queued on its stream (the only stream that reads it), then returning it to the arena.
+// One buffer per (device, stream, purpose): work queued on a stream only ever uses that stream's buffer,
+// so calls on different streams never share bytes (the null stream is one handle on every device).  A
+// buffer grows by first waiting for the work already queued on its stream (the only stream that reads
+// it), then returning it to the arena.
 struct ScratchKey {
+    int dev;
     hipStream_t s;
     int purpose;
-    bool operator==(const ScratchKey& o) const { return s == o.s && purpose == o.purpose; }
+    bool operator==(const ScratchKey& o) const { return dev == o.dev && s == o.s && purpose == o.purpose; }
 };
 struct ScratchKeyHash {
-    size_t operator()(const ScratchKey& k) const { return std::hash<void*>()((void*)k.s) * 31 + (size_t)k.purpose; }
-};
-struct ScratchSlot {
-    void* ptr = nullptr;
-    size_t bytes = 0;
+    size_t operator()(const ScratchKey& k) const {
+        return (std::hash<void*>()((void*)k.s) * 31 + (size_t)k.purpose) * 31 + (size_t)k.dev;
+    }
 };
 std::mutex g_scratch_mu;
-std::unordered_map<ScratchKey, ScratchSlot, ScratchKeyHash> g_scratch;
+std::unordered_map<ScratchKey, std::shared_ptr<ScratchSlot>, ScratchKeyHash> g_scratch;
+
+int current_device() {
+    int dev = 0;
+    HX_HIP(hipGetDevice(&dev));
+    return dev;
+}
 
 // ---- pinned staging for pageable transfers (the CopyPool role, Cuda/CudaCtx.cpp:158-230) -------------
 // Two pinned chunks of 16 MiB, allocated on first use: a transfer moves through them alternately, so
@@ -234,9 +243,10 @@ void* arena_alloc(size_t bytes) {
     if (bytes == 0) return nullptr;
     Arena& a = arena();
     const size_t r = arena_round(bytes);
+    const Arena::Kind kind{current_device(), r};
     std::lock_guard<std::mutex> lk(a.mu);
     void* p = nullptr;
-    auto it = a.free_lists.find(r);
+    auto it = a.free_lists.find(kind);
     if (it != a.free_lists.end() && !it->second.empty()) {
         p = it->second.back();
         it->second.pop_back();
@@ -255,7 +265,7 @@ void* arena_alloc(size_t bytes) {
         a.st.reserved_bytes += r;
         a.st.peak_reserved_bytes = std::max(a.st.peak_reserved_bytes, a.st.reserved_bytes);
     }
-    a.live[p] = r;
+    a.live[p] = kind;
     a.st.live_bytes += r;
     a.st.peak_live_bytes = std::max(a.st.peak_live_bytes, a.st.live_bytes);
     return p;
@@ -267,10 +277,10 @@ void arena_free(void* p) {
     std::lock_guard<std::mutex> lk(a.mu);
     auto it = a.live.find(p);
     if (it == a.live.end()) throw Error{HX_E_ARGUMENT, "pointer was not allocated by this library (or freed twice)"};
-    const size_t r = it->second;
+    const Arena::Kind kind = it->second;
     a.live.erase(it);
-    a.st.live_bytes -= r;
-    a.free_lists[r].push_back(p);
+    a.st.live_bytes -= kind.second;
+    a.free_lists[kind].push_back(p);
 }
 
 bool stream_capturing(hipStream_t s) {
@@ -282,32 +292,53 @@ bool stream_capturing(hipStream_t s) {
     return cs != hipStreamCaptureStatusNone;
 }
 
-void* stream_scratch(hipStream_t s, int purpose, size_t bytes) {
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    ScratchSlot& sl = g_scratch[ScratchKey{s, purpose}];
-    if (sl.bytes >= bytes) return sl.ptr;
-    if (stream_capturing(s)) return nullptr;          // no allocation inside a capture
-    if (sl.ptr) {
-        HX_HIP(hipStreamSynchronize(s));               // the queued work that reads the old buffer is done
-        arena_free(sl.ptr);
-        sl.ptr = nullptr;
-        sl.bytes = 0;
+bool stream_scratch_safe(hipStream_t s) { return s != hipStreamPerThread && !stream_capturing(s); }
+
+ScratchLease stream_scratch(hipStream_t s, int purpose, size_t bytes) {
+    ScratchLease l;
+    {
+        const ScratchKey key{current_device(), s, purpose};
+        std::lock_guard<std::mutex> lk(g_scratch_mu);
+        std::shared_ptr<ScratchSlot>& sl = g_scratch[key];
+        if (!sl) sl = std::make_shared<ScratchSlot>();
+        l.slot = sl;
     }
-    const size_t want = bytes + bytes / 4 + 4096;
-    sl.ptr = arena_alloc(want);
-    sl.bytes = want;
-    return sl.ptr;
+    ScratchSlot& sl = *l.slot;
+    l.held = std::unique_lock<std::mutex>(sl.mu);
+    if (sl.bytes < bytes) {
+        if (stream_capturing(s)) return ScratchLease{};   // no allocation inside a capture
+        if (sl.ptr) {
+            HX_HIP(hipStreamSynchronize(s));               // the queued work that reads the old buffer is done
+            arena_free(sl.ptr);
+            sl.ptr = nullptr;
+            sl.bytes = 0;
+        }
+        const size_t want = bytes + bytes / 4 + 4096;
+        sl.ptr = arena_alloc(want);
+        sl.bytes = want;
+    }
+    l.ptr = sl.ptr;
+    return l;
 }
 
 void stream_scratch_release(hipStream_t s) {
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    for (auto it = g_scratch.begin(); it != g_scratch.end();) {
-        if (it->first.s == s) {
-            arena_free(it->second.ptr);
-            it = g_scratch.erase(it);
-        } else {
-            ++it;
+    std::vector<std::shared_ptr<ScratchSlot>> gone;
+    {
+        std::lock_guard<std::mutex> lk(g_scratch_mu);
+        for (auto it = g_scratch.begin(); it != g_scratch.end();) {
+            if (it->first.s == s) {
+                gone.push_back(it->second);
+                it = g_scratch.erase(it);
+            } else {
+                ++it;
+            }
         }
+    }
+    for (const std::shared_ptr<ScratchSlot>& sl : gone) {
+        std::lock_guard<std::mutex> lk(sl->mu);
+        arena_free(sl->ptr);
+        sl->ptr = nullptr;
+        sl->bytes = 0;
     }
 }
 
