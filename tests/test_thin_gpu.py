@@ -35,7 +35,7 @@ def _check(E, ctx, A, B, C, what):
 
 @pytest.mark.parametrize("p", P)
 @pytest.mark.parametrize("m,n,k", [(32, 32, 1), (33, 127, 31), (31, 129, 32), (100, 200, 33), (1, 4096, 64), (4096, 1, 63),
-                                   (65, 128, 65), (70, 90, 129), (40, 50, 500), (2050, 2111, 40)])
+                                   (65, 128, 65), (70, 90, 129), (40, 50, 500), (2050, 2111, 40), (140001, 20, 31)])
 def test_thin_shapes(hx_gpu, p, m, n, k):
     from hacs_amd import engine as E
     ctx = E.ModCtx(p)
