@@ -1674,10 +1674,11 @@ size_t residue_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t nmod
     return (size_t)nmod * (Mp * Kp + Np * Kp + Mp * Np);
 }
 
-// Whether the automatic choice splits a thin deep product over K on the plain kernel: its limb tiles cannot fill
-// the GPU (256 x 256 x 65536: plain split 64 ways 0.87 ms, limb route 1.50 ms, plain unsplit 11.7 ms).  To
-// k = 8192 the matrix units win all the same (us, split plain / limb or residue route, mod 1000003: 100 x 100 x 1200
-// 77 / 25, 300 x 300 x 1800 107 / 33, 256 x 256 x 4096 112 / 44, 64 x 64 x 8192 162 / 57).
+// Whether the automatic choice splits a thin deep product over K on the plain kernel: its few limb tiles run the
+// whole of K in series (mod 2147483629, us, split plain / limb or residue route: 2 x 2 x 900000 2590 / 10350, 4 x 4 x
+// 200000 594 / 2330, 16 x 16 x 15000 74 / 86).  To k = 8192 the matrix units win all the same (mod 1000003: 100 x 100 x
+// 1200 77 / 25, 300 x 300 x 1800 107 / 33, 256 x 256 x 4096 112 / 44, 64 x 64 x 8192 162 / 57), and for sides past 32
+// deeper still (mod 2147483629: 32 x 32 x 9000 85 / 65, 256 x 256 x 16384 450 / 100 on the residue route).
 bool auto_splits(uint32_t m, uint32_t n, uint32_t k) {
     const uint64_t limb_tiles = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
     return k > 8192 && limb_tiles < 32 && plain_suggest_splits(m, n, k) > 1;
@@ -1846,15 +1847,40 @@ int gemm_auto_variant(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k) 
     return work >= 4.0e6 ? HX_GEMM_LIMB : HX_GEMM_PLAIN;
 }
 
+// The kernel of a product: 0 = the plain one, 1 .. 5 = that limb kernel, kResidueTile with its moduli, kThinRoute.
+struct GemmRoute {
+    int kernel;
+    uint32_t moduli;
+};
+constexpr int kThinRoute = 7;
+
+// The whole choice, for the dispatch and the public queries alike.  lists: rows or columns are gathered; splits as
+// in gemm_dispatch.
+GemmRoute gemm_route(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile, bool host_sizes,
+                     bool lists, uint32_t splits) {
+    const bool automatic = variant == HX_GEMM_AUTO;
+    if (automatic) {
+        if (host_sizes && !lists && splits <= 1 && thin_applies(ctx, m, n, k)) return {kThinRoute, 0};
+        variant = gemm_auto_variant(ctx, m, n, k);
+        if (host_sizes) {
+            if (splits != 1 && auto_splits(m, n, k)) return {0, 0};
+            // small but deep: the limb kernels' few tiles still beat the plain kernel's serial depth (32 x 32 x
+            // 512: 22 us against 97; 1 x 1 x 1000: 22 / 189)
+            if (splits <= 1 && ctx.limbs > 0 && k > 256) variant = HX_GEMM_LIMB;
+        }
+    }
+    if (variant != HX_GEMM_LIMB || ctx.limbs == 0) return {0, 0};
+    const uint32_t rn = residue_choice(ctx, m, n, k, !host_sizes, tile, automatic);
+    return rn != 0 ? GemmRoute{kResidueTile, rn} : GemmRoute{limb_version(tile), 0};
+}
+
 void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int variant, void* ws, size_t ws_bytes,
                    int tile, hipEvent_t ev0, hipEvent_t ev1, uint32_t splits, void* split_ws, size_t split_ws_bytes) {
     const bool automatic = variant == HX_GEMM_AUTO;
-    if (automatic) variant = gemm_auto_variant(ctx, g.m, g.n, g.k);
-    const bool split = automatic && variant == HX_GEMM_LIMB && splits != 1 && g.m_dev == nullptr && g.k_dev == nullptr &&
-                       auto_splits(g.m, g.n, g.k);
-    if (split) variant = HX_GEMM_PLAIN;
-    if (automatic && splits <= 1 && g.m_dev == nullptr && g.k_dev == nullptr && g.a_rows == nullptr &&
-        g.a_cols == nullptr && g.c_rows == nullptr && thin_applies(ctx, g.m, g.n, g.k)) {
+    const bool host_sizes = g.m_dev == nullptr && g.k_dev == nullptr;
+    const bool lists = g.a_rows != nullptr || g.a_cols != nullptr || g.c_rows != nullptr;
+    const GemmRoute rt = gemm_route(ctx, g.m, g.n, g.k, variant, tile, host_sizes, lists, splits);
+    if (rt.kernel == kThinRoute) {
         if (ev0) HX_HIP(hipEventRecord(ev0, s));
         gemm_thin(ctx, g, s);
         if (ev1) HX_HIP(hipEventRecord(ev1, s));
@@ -1862,14 +1888,9 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
         stat_add(ST_LIMB, 1);
         return;
     }
-    // small but deep: the limb kernels' few tiles still beat the plain kernel's serial depth (32 x 32 x 512: 28
-    // against 97 us)
-    if (automatic && variant == HX_GEMM_PLAIN && ctx.limbs > 0 && !split && splits <= 1 && g.k > 256 && g.m_dev == nullptr && g.k_dev == nullptr)
-        variant = HX_GEMM_LIMB;
     ScratchLease planes, partials;   // the library's own workspaces, held until the product is launched
-    uint32_t rn = 0;            // moduli of the residue route, 0 = the limb kernels
-    if (variant == HX_GEMM_LIMB && g.m != 0 && g.n != 0)
-        rn = residue_choice(ctx, g.m, g.n, g.k, g.m_dev != nullptr || g.k_dev != nullptr, tile, automatic);
+    variant = rt.kernel == 0 ? HX_GEMM_PLAIN : HX_GEMM_LIMB;
+    uint32_t rn = g.m != 0 && g.n != 0 ? rt.moduli : 0;      // moduli of the residue route, 0 = the limb kernels
     if (rn != 0) {
         // the default route falls back to the limb kernels when its planes do not fit (a caller workspace
         // sized for the limb planes, the library's own that cannot grow inside a capture, device memory)
@@ -2241,11 +2262,9 @@ extern "C" {
 HX_API size_t hx_gemm_workspace_bytes_tile(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant,
                                            int tile) {
     if (ctx == nullptr) return 0;
-    const bool automatic = variant == HX_GEMM_AUTO;
-    if (automatic) variant = gemm_auto_variant(*ctx, m, n, k);
-    if (variant != HX_GEMM_LIMB) return 0;
-    const uint32_t rn = residue_choice(*ctx, m, n, k, false, tile, automatic);
-    return rn ? residue_workspace_bytes(m, n, k, rn) : limb_workspace_bytes(*ctx, m, n, k);
+    const GemmRoute rt = gemm_route(*ctx, m, n, k, variant, tile, true, false, 0);
+    if (rt.kernel == 0 || rt.kernel == kThinRoute) return 0;
+    return rt.moduli ? residue_workspace_bytes(m, n, k, rt.moduli) : limb_workspace_bytes(*ctx, m, n, k);
 }
 
 HX_API size_t hx_gemm_workspace_bytes(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant) {
@@ -2255,17 +2274,7 @@ HX_API size_t hx_gemm_workspace_bytes(const hx_modctx* ctx, uint32_t m, uint32_t
 HX_API uint32_t hx_gemm_residue_moduli(uint32_t p, uint32_t k) { return p >= 2 ? residue_moduli(p, k) : 0; }
 
 HX_API int hx_gemm_route(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile) {
-    if (ctx == nullptr) return -1;
-    const bool automatic = variant == HX_GEMM_AUTO;
-    if (automatic) {
-        if (thin_applies(*ctx, m, n, k)) return 7;
-        variant = gemm_auto_variant(*ctx, m, n, k);
-        if (variant == HX_GEMM_LIMB && auto_splits(m, n, k)) return 0;
-        if (ctx->limbs > 0 && k > 256) variant = HX_GEMM_LIMB;
-    }
-    if (variant != HX_GEMM_LIMB || ctx->limbs == 0) return 0;
-    if (residue_choice(*ctx, m, n, k, false, tile, automatic) != 0) return kResidueTile;
-    return limb_version(tile);
+    return ctx == nullptr ? -1 : gemm_route(*ctx, m, n, k, variant, tile, true, false, 0).kernel;
 }
 
 HX_API int hx_gemm_u32(const hx_modctx* ctx, hx_view A, hx_view B, hx_view C, int op, hx_stream s,

@@ -1,0 +1,35 @@
+"""The automatic choice of the product's kernel, by its public queries (host arithmetic, no device)."""
+import pytest
+
+from hacs_amd import engine as E
+
+P = {1: 251, 2: 61001, 3: 65521, 4: 2147483629}          # a modulus of each limb count
+
+
+@pytest.mark.parametrize("limbs", [1, 2, 3, 4])
+def test_deep_products_of_few_tiles_split(limbs):
+    """Past k = 8192 the few tiles of a narrow product would run all of K in series: it splits over K on the
+    plain kernel on both sides of 4e6 multiply-adds, and past the residue route's depth."""
+    c = E.ModCtx(P[limbs])
+    for m, n, k in [(16, 16, 15000), (16, 16, 16000), (8, 8, 60000), (4, 4, 200000), (1, 1, 8193), (256, 256, 16384),
+                    (200, 100, 140000)]:
+        assert E.gemm_route(c, m, n, k, E.HX_GEMM_AUTO) == 0, (m, n, k)
+    for m, n, k in [(16, 16, 8192), (1, 1, 300), (8, 8, 257), (64, 64, 8192)]:
+        assert E.gemm_route(c, m, n, k, E.HX_GEMM_AUTO) in (4, 6), (m, n, k)
+
+
+@pytest.mark.parametrize("limbs", [1, 2, 3, 4])
+def test_workspace_follows_the_route(limbs):
+    """hx_gemm_workspace_bytes(AUTO) is zero exactly where the reported kernel needs no planes, and else serves
+    that kernel."""
+    c = E.ModCtx(P[limbs])
+    for m, n, k in [(8, 8, 8), (40, 40, 500), (40, 40, 257), (40, 40, 256), (300, 300, 64), (300, 300, 65),
+                    (16, 16, 15000), (1024, 1024, 1024), (2048, 2048, 2048), (256, 256, 16384), (4096, 34, 2000)]:
+        route = E.gemm_route(c, m, n, k, E.HX_GEMM_AUTO)
+        got = E.gemm_workspace_bytes(c, m, n, k, E.HX_GEMM_AUTO)
+        if route in (0, 7):
+            assert got == 0, (m, n, k)
+        elif route == 6:
+            assert got == E.gemm_workspace_bytes(c, m, n, k, E.HX_GEMM_LIMB, tile=6), (m, n, k)
+        else:
+            assert got == E.gemm_workspace_bytes(c, m, n, k, E.HX_GEMM_LIMB, tile=4) > 0, (m, n, k)

@@ -61,3 +61,17 @@ def test_auto_route_equals_plain(hx_gpu, p, m, n, k, fa, fb, fc):
     E.gemm_nt(ctx, A, _draw(p, k, n, 2, fb).t(), C)
     E.gemm(ctx, A, B, D, variant=E.HX_GEMM_PLAIN, splits=1)
     assert torch.equal(C, D)
+
+
+@pytest.mark.parametrize("p", [251, 61001, 65521, 2147483629])
+@pytest.mark.parametrize("m,n,k", [(16, 16, 15000), (16, 16, 16000), (8, 8, 60000), (4, 4, 140000), (16, 16, 8192), (3, 5, 300)])
+def test_auto_deep_products_of_few_tiles(hx_gpu, p, m, n, k):
+    """Both sides of the depth where few tiles are split over K, and of 4e6 multiply-adds."""
+    from hacs_amd import engine as E
+    ctx = E.ModCtx(p)
+    A, B = _draw(p, m, k, 1, "row"), _draw(p, k, n, 2, "row")
+    for op in (E.GemmOp.Set, E.GemmOp.Sub):
+        C, D = _draw(p, m, n, 3, "row"), _draw(p, m, n, 3, "row")
+        E.gemm(ctx, A, B, C, op)
+        E.gemm(ctx, A, B, D, op, variant=E.HX_GEMM_PLAIN, splits=1)
+        assert torch.equal(C, D), op
