@@ -1679,9 +1679,10 @@ size_t residue_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t nmod
 // 200000 594 / 2330, 16 x 16 x 15000 74 / 86).  To k = 8192 the matrix units win all the same (mod 1000003: 100 x 100 x
 // 1200 77 / 25, 300 x 300 x 1800 107 / 33, 256 x 256 x 4096 112 / 44, 64 x 64 x 8192 162 / 57), and for sides past 32
 // deeper still (mod 2147483629: 32 x 32 x 9000 85 / 65, 256 x 256 x 16384 450 / 100 on the residue route).
-bool auto_splits(uint32_t m, uint32_t n, uint32_t k) {
+// any_depth: the planes of the shallower ones are not to be had, or the caller asks for the split.
+bool auto_splits(uint32_t m, uint32_t n, uint32_t k, bool any_depth) {
     const uint64_t limb_tiles = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
-    return k > 8192 && limb_tiles < 32 && plain_suggest_splits(m, n, k) > 1;
+    return (any_depth || k > 8192) && limb_tiles < 32 && plain_suggest_splits(m, n, k) > 1;
 }
 
 // The moduli count of the residue route when this product takes it, else 0.  It needs host-side sizes,
@@ -1855,22 +1856,24 @@ struct GemmRoute {
 constexpr int kThinRoute = 7;
 
 // The whole choice, for the dispatch and the public queries alike.  lists: rows or columns are gathered; splits as
-// in gemm_dispatch.
+// in gemm_dispatch.  planes_ok: a caller workspace, or the library's scratch outside a capture.  Without it an
+// automatic product takes no route that adds planes: a graph would keep the address of a buffer that a later,
+// larger call on the stream replaces.
 GemmRoute gemm_route(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile, bool host_sizes,
-                     bool lists, uint32_t splits) {
+                     bool lists, uint32_t splits, bool planes_ok) {
     const bool automatic = variant == HX_GEMM_AUTO;
     if (automatic) {
         if (host_sizes && !lists && splits <= 1 && thin_applies(ctx, m, n, k)) return {kThinRoute, 0};
         variant = gemm_auto_variant(ctx, m, n, k);
         if (host_sizes) {
-            if (splits != 1 && auto_splits(m, n, k)) return {0, 0};
+            if (splits != 1 && auto_splits(m, n, k, !planes_ok)) return {0, 0};
             // small but deep: the limb kernels' few tiles still beat the plain kernel's serial depth (32 x 32 x
             // 512: 22 us against 97; 1 x 1 x 1000: 22 / 189)
-            if (splits <= 1 && ctx.limbs > 0 && k > 256) variant = HX_GEMM_LIMB;
+            if (planes_ok && splits <= 1 && ctx.limbs > 0 && k > 256) variant = HX_GEMM_LIMB;
         }
     }
     if (variant != HX_GEMM_LIMB || ctx.limbs == 0) return {0, 0};
-    const uint32_t rn = residue_choice(ctx, m, n, k, !host_sizes, tile, automatic);
+    const uint32_t rn = residue_choice(ctx, m, n, k, !host_sizes, tile, automatic && planes_ok);
     return rn != 0 ? GemmRoute{kResidueTile, rn} : GemmRoute{limb_version(tile), 0};
 }
 
@@ -1879,7 +1882,8 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
     const bool automatic = variant == HX_GEMM_AUTO;
     const bool host_sizes = g.m_dev == nullptr && g.k_dev == nullptr;
     const bool lists = g.a_rows != nullptr || g.a_cols != nullptr || g.c_rows != nullptr;
-    const GemmRoute rt = gemm_route(ctx, g.m, g.n, g.k, variant, tile, host_sizes, lists, splits);
+    const bool planes_ok = !automatic || ws != nullptr || stream_scratch_safe(s);
+    const GemmRoute rt = gemm_route(ctx, g.m, g.n, g.k, variant, tile, host_sizes, lists, splits, planes_ok);
     if (rt.kernel == kThinRoute) {
         if (ev0) HX_HIP(hipEventRecord(ev0, s));
         gemm_thin(ctx, g, s);
@@ -2262,7 +2266,7 @@ extern "C" {
 HX_API size_t hx_gemm_workspace_bytes_tile(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant,
                                            int tile) {
     if (ctx == nullptr) return 0;
-    const GemmRoute rt = gemm_route(*ctx, m, n, k, variant, tile, true, false, 0);
+    const GemmRoute rt = gemm_route(*ctx, m, n, k, variant, tile, true, false, 0, true);
     if (rt.kernel == 0 || rt.kernel == kThinRoute) return 0;
     return rt.moduli ? residue_workspace_bytes(m, n, k, rt.moduli) : limb_workspace_bytes(*ctx, m, n, k);
 }
@@ -2274,7 +2278,7 @@ HX_API size_t hx_gemm_workspace_bytes(const hx_modctx* ctx, uint32_t m, uint32_t
 HX_API uint32_t hx_gemm_residue_moduli(uint32_t p, uint32_t k) { return p >= 2 ? residue_moduli(p, k) : 0; }
 
 HX_API int hx_gemm_route(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile) {
-    return ctx == nullptr ? -1 : gemm_route(*ctx, m, n, k, variant, tile, true, false, 0).kernel;
+    return ctx == nullptr ? -1 : gemm_route(*ctx, m, n, k, variant, tile, true, false, 0, true).kernel;
 }
 
 HX_API int hx_gemm_u32(const hx_modctx* ctx, hx_view A, hx_view B, hx_view C, int op, hx_stream s,

@@ -94,7 +94,10 @@ typedef struct hx_gemm_opts {   /* GemmOpts, CudaKernels.h:64-79 */
                                64-deep K chunk, hx_gemm_limb_k_chunk) runs K in chunks, same bytes; smaller: AUTO
                                runs the plain kernel, LIMB fails (HX_E_ARGUMENT).  NULL = library-owned planes
                                private to the stream (grown outside a capture only: inside one, AUTO falls back
-                               to the plain kernel when they are too small and LIMB fails with HX_E_CAPTURE) */
+                               to the plain kernel when they are too small, and does not use them at all for
+                               products below 4e6 multiply-adds or of fewer than 32 tiles of 64 x 128 and
+                               k >= 1024, nor for residue planes below m, n, k = 4096; LIMB fails with
+                               HX_E_CAPTURE when they are too small) */
     size_t workspace_bytes;
     hx_event main_begin;    /* optional timing events recorded on the stream right before / after the */
     hx_event main_end;      /* main product kernel (instrumentation only; NULL = none) */
