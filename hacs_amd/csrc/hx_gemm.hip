@@ -1866,7 +1866,7 @@ GemmRoute gemm_route(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, i
         if (host_sizes && !lists && splits <= 1 && thin_applies(ctx, m, n, k)) return {kThinRoute, 0};
         variant = gemm_auto_variant(ctx, m, n, k);
         if (host_sizes) {
-            if (splits != 1 && auto_splits(m, n, k, !planes_ok)) return {0, 0};
+            if (splits != 1 && auto_splits(m, n, k, !planes_ok || splits > 1)) return {0, 0};
             // small but deep: the limb kernels' few tiles still beat the plain kernel's serial depth (32 x 32 x
             // 512: 22 us against 97; 1 x 1 x 1000: 22 / 189)
             if (planes_ok && splits <= 1 && ctx.limbs > 0 && k > 256) variant = HX_GEMM_LIMB;

@@ -153,3 +153,23 @@ def test_split_k_inside_graph_capture(hx_gpu, O):
             s.synchronize()
             assert np.array_equal(E.from_device(other), want)
         _lib.check(L.hx_graph_destroy(g))
+
+
+@pytest.mark.parametrize("shape,splits", [((100, 70, 3333), 5), ((300, 300, 2000), 3), ((64, 64, 8192), 16), ((40, 40, 900), 4)])
+def test_split_k_count_under_the_automatic_variant(hx_gpu, O, shape, splits):
+    """An explicit count under AUTO runs the split plain kernel in the caller's workspace wherever few limb
+    tiles would leave the GPU idle."""
+    from hacs_amd import engine as E
+    p = 2147483629
+    ctx = E.ModCtx(p)
+    m, n, k = shape
+    rng = np.random.default_rng(m + n + k)
+    A, B = _rand(rng, p, (m, k)), _rand(rng, p, (k, n))
+    ws = torch.empty(E.split_workspace_bytes(m, n, k, splits), dtype=torch.uint8, device="cuda")
+    dC = torch.zeros((m, n), dtype=torch.int32, device="cuda")
+    before = _stats()
+    E.gemm(ctx, E.to_device(A), E.to_device(B), dC, E.GemmOp.Set, splits=splits, split_workspace=ws)
+    torch.cuda.synchronize()
+    after = _stats()
+    assert after.splitk_launches == before.splitk_launches + 1 and after.limb_launches == before.limb_launches
+    assert np.array_equal(E.from_device(dC), O.gemm_fast(p, A, B))
