@@ -1675,14 +1675,17 @@ size_t residue_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t nmod
 }
 
 // Whether the automatic choice splits a thin deep product over K on the plain kernel: its few limb tiles run the
-// whole of K in series (mod 2147483629, us, split plain / limb or residue route: 2 x 2 x 900000 2590 / 10350, 4 x 4 x
-// 200000 594 / 2330, 16 x 16 x 15000 74 / 86).  To k = 8192 the matrix units win all the same (mod 1000003: 100 x 100 x
-// 1200 77 / 25, 300 x 300 x 1800 107 / 33, 256 x 256 x 4096 112 / 44, 64 x 64 x 8192 162 / 57), and for sides past 32
-// deeper still (mod 2147483629: 32 x 32 x 9000 85 / 65, 256 x 256 x 16384 450 / 100 on the residue route).
-// any_depth: the planes of the shallower ones are not to be had, or the caller asks for the split.
-bool auto_splits(uint32_t m, uint32_t n, uint32_t k, bool any_depth) {
+// whole of K in series.  Below 4e6 multiply-adds past k = 12288, except for one limb, whose tiles keep up (us, split
+// plain / limb or residue route: 1 x 1 x 9000 69 / 63 mod 2147483629 and 69 / 54 mod 61001, 16 x 16 x 15000 74 / 86 and
+// 78 / 89, 4 x 4 x 200000 594 / 2330 and 593 / 970; 8 x 8 x 60000 mod 251 203 / 193).  Larger products past k = 8192: to there
+// the matrix units win (mod 1000003: 100 x 100 x 1200 77 / 25, 300 x 300 x 1800 107 / 33, 256 x 256 x 4096 112 / 44, 64 x 64 x
+// 8192 162 / 57), and for sides past 32 deeper still (mod 2147483629: 32 x 32 x 9000 85 / 65, 256 x 256 x 16384 450 / 100 on the
+// residue route).  any_depth: the planes of the shallower ones are not to be had, or the caller asks for the split.
+bool auto_splits(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, bool any_depth) {
     const uint64_t limb_tiles = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
-    return (any_depth || k > 8192) && limb_tiles < 32 && plain_suggest_splits(m, n, k) > 1;
+    const bool small = gemm_auto_variant(ctx, m, n, k) == HX_GEMM_PLAIN;
+    const bool deep = small ? k > 12288 && ctx.limbs != 1 : k > 8192;
+    return (any_depth || deep) && limb_tiles < 32 && plain_suggest_splits(m, n, k) > 1;
 }
 
 // The moduli count of the residue route when this product takes it, else 0.  It needs host-side sizes,
@@ -1866,7 +1869,7 @@ GemmRoute gemm_route(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, i
         if (host_sizes && !lists && splits <= 1 && thin_applies(ctx, m, n, k)) return {kThinRoute, 0};
         variant = gemm_auto_variant(ctx, m, n, k);
         if (host_sizes) {
-            if (splits != 1 && auto_splits(m, n, k, !planes_ok || splits > 1)) return {0, 0};
+            if (splits != 1 && auto_splits(ctx, m, n, k, !planes_ok || splits > 1)) return {0, 0};
             // small but deep: the limb kernels' few tiles still beat the plain kernel's serial depth (32 x 32 x
             // 512: 22 us against 97; 1 x 1 x 1000: 22 / 189)
             if (planes_ok && splits <= 1 && ctx.limbs > 0 && k > 256) variant = HX_GEMM_LIMB;

@@ -8,13 +8,15 @@ P = {1: 251, 2: 61001, 3: 65521, 4: 2147483629}          # a modulus of each lim
 
 @pytest.mark.parametrize("limbs", [1, 2, 3, 4])
 def test_deep_products_of_few_tiles_split(limbs):
-    """Past k = 8192 the few tiles of a narrow product would run all of K in series: it splits over K on the
-    plain kernel on both sides of 4e6 multiply-adds, and past the residue route's depth."""
+    """The few tiles of a deep narrow product would run all of K in series: it splits over K on the plain kernel
+    past k = 8192 from 4e6 multiply-adds on, below past k = 12288 (not with one limb), past the residue route's
+    depth too."""
     c = E.ModCtx(P[limbs])
-    for m, n, k in [(16, 16, 15000), (16, 16, 16000), (8, 8, 60000), (4, 4, 200000), (1, 1, 8193), (256, 256, 16384),
-                    (200, 100, 140000)]:
+    for m, n, k in [(16, 16, 16000), (256, 256, 16384), (200, 100, 140000), (32, 32, 8193)]:
         assert E.gemm_route(c, m, n, k, E.HX_GEMM_AUTO) == 0, (m, n, k)
-    for m, n, k in [(16, 16, 8192), (1, 1, 300), (8, 8, 257), (64, 64, 8192)]:
+    for m, n, k in [(16, 16, 15000), (8, 8, 60000), (4, 4, 200000), (1, 1, 12289)]:
+        assert E.gemm_route(c, m, n, k, E.HX_GEMM_AUTO) == (4 if limbs == 1 else 0), (m, n, k)
+    for m, n, k in [(16, 16, 8192), (1, 1, 12288), (1, 1, 300), (8, 8, 257), (64, 64, 8192)]:
         assert E.gemm_route(c, m, n, k, E.HX_GEMM_AUTO) in (4, 6), (m, n, k)
 
 
