@@ -1688,15 +1688,44 @@ bool auto_splits(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, bool 
     return (any_depth || deep) && limb_tiles < 32 && plain_suggest_splits(m, n, k) > 1;
 }
 
+// 256 x 256 tiles once they fill the 256 compute units twice (3072^3, ten moduli: 1440 tiles, 370 us against 418
+// with 128 x 128; 4096^3 770 / 913); below, the smaller tiles cost at most as much (2048^3, 640 tiles: 145 / 147).
+uint32_t residue_side(uint32_t m, uint32_t n, uint32_t N) {
+    const uint64_t tiles = (uint64_t)((m + RTM - 1) / RTM) * ((n + RTN - 1) / RTN) * N;
+    return tiles >= 512 ? RTM : RTM / 2;
+}
+
+// Whether the residue route is the faster one for a product of 256 and more tiles of 64 x 128, by both routes' times
+// in microseconds: rounds and tiles of the matrix units, passes over the operands, outputs.  Fitted to 731 products
+// (sides 34 to 20000, depths 768 to 16384, 17 to 31 bits; mean error 4 %): the route saves multiply-adds but writes and
+// reads N planes where the limb kernel has L, and pads to larger tiles, which a long narrow operand pays for most
+// (mod 2147483629, us limb / residue: 34 x 40000 x 2000 313 / 530, 129 x 20000 x 2000 213 / 294, 20000 x 34 x 3000 306 / 380,
+// 300 x 7000 x 4096 254 / 305, 384 x 20000 x 2048 342 / 409; 512 x 4200 x 2048 136 / 109, 20000 x 256 x 4096 530 / 490).  From
+// sides of 1100 on it always does at these depths, or costs a few per cent.
+bool residue_pays(uint32_t limbs, uint32_t N, uint32_t m, uint32_t n, uint32_t k) {
+    const uint32_t narrow = std::min(m, n);
+    if (narrow >= 1100) return true;
+    auto cd = [](uint64_t a, uint64_t b) { return (double)((a + b - 1) / b); };
+    const double K = 1e-3 * k, M = 1e-3 * m, Nn = 1e-3 * n;
+    const uint64_t lt = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
+    const double limb = 14.7 + K * limbs * limbs * (1.23 * cd(lt, 256) + 0.46 / 256 * (double)lt) +
+                        K * (1.96 * M + 2.1 * Nn) + 1.64 * M * Nn;
+    const uint32_t side = residue_side(m, n, N);
+    const uint64_t rt = (uint64_t)N * ((m + side - 1) / side) * ((n + side - 1) / side);
+    const double round = side == RTM ? 5.84 : 2.52, tile = (side == RTM ? 6.85 : 1.49) / 256;
+    const double res = 17.5 + K * (round * cd(rt, 256) + tile * (double)rt) + K * N * (0.35 * M + 0.424 * Nn) + 0.678 * N * M * Nn;
+    return res < (narrow < 256 ? 0.88 : 0.97) * limb;        // (in doubt the limb kernel)
+}
+
 // The moduli count of the residue route when this product takes it, else 0.  It needs host-side sizes,
 // 1 <= k <= RES_KMAX and enough moduli; tile kResidueTile asks for it wherever it applies.  The limb variant's
 // default (tile 0) takes it where it runs at most L^2 - 4 int8 products (four-limb moduli: 10 or 11 for 16) and
-// m, n, k >= 4096.  The automatic variant takes it at every m, n once k is deep enough to pay for the splits
-// and the CRT, whose cost does not grow with k, for three and four limbs: from 256 tiles of 64 x 128 on from
+// m, n, k >= 4096.  The automatic variant takes it once k is deep enough to pay for the splits and the CRT, whose
+// cost does not grow with k, for three and four limbs: from 256 tiles of 64 x 128 on, where residue_pays, from
 // k = 1536 / 768 (us, limb kernel 4 / residue route; mod 2147483629: 1500^2 x 1600 110 / 86, 1677 x 1419 x 2049
 // 133 / 114, 2048^3 147 / 145, 4096^3 990 / 760, 8192^3 7400 / 5200, 8192^2 x 512 600 / 680, x 1024 1131 / 953; mod
-// 65521: 1500^2 x 1600 77 / 62, 2048^3 96 / 96, 4096^3 596 / 473, 8192^2 x 512 421 / 480), and up to 64 tiles from
-// k = 2560 / 1536, where its ten products fill units that the limb kernel leaves idle (mod 2147483629: 512^2 x
+// 65521: 1500^2 x 1600 77 / 62, 2048^3 96 / 96, 4096^3 596 / 473, 8192^2 x 512 421 / 480), and up to 64 tiles of sides up to
+// m + n = 2560 (mod 2147483629: 100 x 2000 x 3000 62 / 54, 64 x 4096 x 3000 68 / 82, 34 x 8192 x 3000 80 / 174) from k = 2560 / 1536, where its ten products fill units that the limb kernel leaves idle (mod 2147483629: 512^2 x
 // 1600 46 / 41, x 5000 86 / 62; mod 65521: 512^2 x 1600 34 / 36, x 3000 47 / 43).  Between them the limb kernels have
 // one tile for each unit and the residue route the tiles' remainders of ten products (mod 2147483629: 1024^2 x
 // 2000 58 / 67, x 5000 104 / 119, 7033 x 34 x 3000 85 / 126, 1280^2 x 3000 98 / 103).  Two-limb moduli stay on the limb
@@ -1708,18 +1737,11 @@ uint32_t residue_choice(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k
     if (N == 0 || tile == kResidueTile) return N;
     const uint64_t limb_tiles = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
     if (automatic && ctx.limbs >= 3) {
-        if (limb_tiles >= 256 && k >= (ctx.limbs == 4 ? 768u : 1536u)) return N;
-        if (limb_tiles <= 64 && k >= (ctx.limbs == 4 ? 1536u : 2560u)) return N;
+        if (limb_tiles >= 256 && k >= (ctx.limbs == 4 ? 768u : 1536u) && residue_pays(ctx.limbs, N, m, n, k)) return N;
+        if (limb_tiles <= 64 && k >= (ctx.limbs == 4 ? 1536u : 2560u) && (uint64_t)m + n <= 2560) return N;
     }
     const bool large = m >= 4096 && n >= 4096 && k >= 4096;
     return large && ctx.limbs > 0 && N + 4 <= ctx.limbs * ctx.limbs ? N : 0;
-}
-
-// 256 x 256 tiles once they fill the 256 compute units twice (3072^3, ten moduli: 1440 tiles, 370 us against 418
-// with 128 x 128; 4096^3 770 / 913); below, the smaller tiles cost at most as much (2048^3, 640 tiles: 145 / 147).
-uint32_t residue_side(uint32_t m, uint32_t n, uint32_t N) {
-    const uint64_t tiles = (uint64_t)((m + RTM - 1) / RTM) * ((n + RTN - 1) / RTN) * N;
-    return tiles >= 512 ? RTM : RTM / 2;
 }
 
 void residue_product(const ResArgs& a, uint32_t N, uint32_t side, hipStream_t s) {

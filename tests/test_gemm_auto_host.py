@@ -35,3 +35,17 @@ def test_workspace_follows_the_route(limbs):
             assert got == E.gemm_workspace_bytes(c, m, n, k, E.HX_GEMM_LIMB, tile=6), (m, n, k)
         else:
             assert got == E.gemm_workspace_bytes(c, m, n, k, E.HX_GEMM_LIMB, tile=4) > 0, (m, n, k)
+
+
+@pytest.mark.parametrize("p,m,n,k,route", [
+    # long narrow products: the residue planes' passes and padding cost more than the multiply-adds they save
+    (2147483629, 34, 8192, 2000, 4), (2147483629, 8192, 34, 3000, 4), (2147483629, 20000, 34, 3000, 4),
+    (2147483629, 34, 40000, 3000, 4), (2147483629, 1, 8192, 3000, 4), (2147483629, 64, 4096, 5000, 4),
+    (2147483629, 129, 20000, 1600, 4), (65521, 129, 20000, 1600, 4), (65521, 34, 40000, 3000, 4),
+    (2147483629, 300, 7000, 4096, 4), (2147483629, 384, 20000, 2048, 4),
+    # and where they do not
+    (2147483629, 100, 2000, 3000, 6), (2147483629, 1000, 34, 5000, 6), (2147483629, 512, 4200, 2048, 6),
+    (2147483629, 1677, 1419, 2049, 6), (2147483629, 700, 3000, 2560, 6), (16777213, 20000, 200, 8192, 6),
+    (65521, 8192, 8192, 4096, 6), (2147483629, 8192, 8192, 1024, 6)])
+def test_residue_route_by_shape(p, m, n, k, route):
+    assert E.gemm_route(E.ModCtx(p), m, n, k, E.HX_GEMM_AUTO) == route
