@@ -1668,10 +1668,24 @@ uint32_t residue_moduli(uint32_t p, uint32_t k) {
     return 0;
 }
 
-size_t residue_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, uint32_t nmod) {
-    const size_t Mp = round_up(std::max<uint32_t>(m, 1), RTM), Np = round_up(std::max<uint32_t>(n, 1), RTN);
-    const size_t Kp = round_up(std::max<uint32_t>(k, 1), 64);
-    return (size_t)nmod * (Mp * Kp + Np * Kp + Mp * Np);
+// The planes held at a time: C runs in blocks of mb x nb (multiples of 256) whose planes fit RES_WS, each a residue
+// product of its own.  At 8 GiB, 3 % of the card, 16384^3 is still one block (ten moduli); unbounded, 32768 x 32768 x 1024
+// would hold 10.3 GB on the stream for good.  whole: one block whatever its size (tile kResidueTile).
+constexpr uint64_t RES_WS = (uint64_t)8 << 30;
+struct ResPlan {
+    uint64_t mb, nb, bytes;
+};
+ResPlan residue_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t nmod, bool whole) {
+    auto up = [](uint64_t x, uint64_t a) { return (std::max<uint64_t>(x, 1) + a - 1) / a * a; };
+    const uint64_t Kp = up(k, 64);
+    ResPlan r{up(m, RTM), up(n, RTN), 0};
+    auto bytes = [&] { return nmod * (r.mb * Kp + r.nb * Kp + r.mb * r.nb); };
+    while (!whole && bytes() > RES_WS && (r.mb > RTM || r.nb > RTN)) {
+        uint64_t& longer = r.mb >= r.nb ? r.mb : r.nb;
+        longer = up(longer / 2, RTM);
+    }
+    r.bytes = bytes();
+    return r;
 }
 
 // Whether the automatic choice splits a thin deep product over K on the plain kernel: its few limb tiles run the
@@ -1752,15 +1766,10 @@ void residue_product(const ResArgs& a, uint32_t N, uint32_t side, hipStream_t s)
 }
 
 // C op= A B mod p by the residue route with N moduli: residue planes of A and B (res_prep_kernel),
-// one int8 product per modulus (res_gemm_kernel, grid.y = modulus), CRT into C (crt_kernel).
+// one int8 product per modulus (res_gemm_kernel, grid.y = modulus), CRT into C (crt_kernel).  One block of C:
 // ws holds N (Mp Kp + Np Kp + Mp Np) bytes (Mp, Np: m, n rounded up to 256; Kp: k to 64).
-void gemm_residue(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32_t N, void* ws, size_t ws_bytes,
-                  hipEvent_t ev0, hipEvent_t ev1) {
-    if (g.m == 0 || g.n == 0) return;
-    HX_CHECK(N >= 1 && N <= (uint32_t)RES_MAXN && g.m_dev == nullptr && g.k_dev == nullptr && g.k >= 1,
-             "residue route: no plan for this product");
-    HX_CHECK(ws != nullptr && ws_bytes >= residue_workspace_bytes(g.m, g.n, g.k, N),
-             "residue route: workspace too small");
+void residue_block(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32_t N, void* ws, hipEvent_t ev0,
+                   hipEvent_t ev1) {
     const uint32_t p = ctx.p;
     const uint32_t side = residue_side(g.m, g.n, N);
     const uint32_t Mp = round_up(g.m, side), Np = round_up(g.n, side), Kp = round_up(g.k, 64);
@@ -1863,6 +1872,31 @@ void gemm_residue(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32
     after_launch("crt_kernel");
 }
 
+// The product in the plan's blocks; ev0 and ev1 around the first block's and the last block's residue_product.
+void gemm_residue(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32_t N, const ResPlan& r, void* ws,
+                  size_t ws_bytes, hipEvent_t ev0, hipEvent_t ev1) {
+    if (g.m == 0 || g.n == 0) return;
+    HX_CHECK(N >= 1 && N <= (uint32_t)RES_MAXN && g.m_dev == nullptr && g.k_dev == nullptr && g.k >= 1,
+             "residue route: no plan for this product");
+    HX_CHECK(ws != nullptr && ws_bytes >= r.bytes, "residue route: workspace too small");
+    for (uint64_t i0 = 0; i0 < g.m; i0 += r.mb)
+        for (uint64_t j0 = 0; j0 < g.n; j0 += r.nb) {
+            const int64_t i = (int64_t)i0, j = (int64_t)j0;
+            GemmArgs b = g;
+            b.m = (uint32_t)std::min<uint64_t>(r.mb, g.m - i0);
+            b.n = (uint32_t)std::min<uint64_t>(r.nb, g.n - j0);
+            if (g.a_rows) b.a_rows = g.a_rows + i;
+            else b.A = g.A + i * g.ars;
+            b.B = g.B + j * g.bcs;
+            b.Cin = g.Cin + j * g.cics;
+            if (g.c_rows) b.c_rows = g.c_rows + i;
+            else b.Cin += i * g.cirs;
+            b.Cout = g.Cout + i * g.cors + j * g.cocs;
+            residue_block(ctx, b, s, N, ws, i0 + j0 == 0 ? ev0 : nullptr,
+                          i0 + r.mb >= g.m && j0 + r.nb >= g.n ? ev1 : nullptr);
+        }
+}
+
 // The automatic choice: the limb route once the product is big enough to pay for the two
 // operand splits, and deep enough (k >= 64, one full LDS stage) for the MFMA work to outweigh the
 // recombination epilogue; thinner products (the k = 32 Schur updates of the eliminations) run
@@ -1920,11 +1954,13 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
     ScratchLease planes, partials;   // the library's own workspaces, held until the product is launched
     variant = rt.kernel == 0 ? HX_GEMM_PLAIN : HX_GEMM_LIMB;
     uint32_t rn = g.m != 0 && g.n != 0 ? rt.moduli : 0;      // moduli of the residue route, 0 = the limb kernels
+    ResPlan rplan{};
     if (rn != 0) {
         // the default route falls back to the limb kernels when its planes do not fit (a caller workspace
         // sized for the limb planes, the library's own that cannot grow inside a capture, device memory)
         const bool asked = tile == kResidueTile;
-        const size_t need = residue_workspace_bytes(g.m, g.n, g.k, rn);
+        rplan = residue_plan(g.m, g.n, g.k, rn, asked);
+        const size_t need = rplan.bytes;
         if (ws == nullptr) {
             try {
                 planes = stream_scratch(s, SCRATCH_LIMB, need);
@@ -1987,7 +2023,7 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
         }
     }
     if (rn != 0)
-        gemm_residue(ctx, g, s, rn, ws, ws_bytes, ev0, ev1);
+        gemm_residue(ctx, g, s, rn, rplan, ws, ws_bytes, ev0, ev1);
     else if (variant == HX_GEMM_LIMB)
         gemm_limb(ctx, g, s, ws, ws_bytes, tile, ev0, ev1);
     else
@@ -2293,7 +2329,7 @@ HX_API size_t hx_gemm_workspace_bytes_tile(const hx_modctx* ctx, uint32_t m, uin
     if (ctx == nullptr) return 0;
     const GemmRoute rt = gemm_route(*ctx, m, n, k, variant, tile, true, false, 0, true);
     if (rt.kernel == 0 || rt.kernel == kThinRoute) return 0;
-    return rt.moduli ? residue_workspace_bytes(m, n, k, rt.moduli) : limb_workspace_bytes(*ctx, m, n, k);
+    return rt.moduli ? residue_plan(m, n, k, rt.moduli, tile == kResidueTile).bytes : limb_workspace_bytes(*ctx, m, n, k);
 }
 
 HX_API size_t hx_gemm_workspace_bytes(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant) {

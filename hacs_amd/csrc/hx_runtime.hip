@@ -313,7 +313,7 @@ ScratchLease stream_scratch(hipStream_t s, int purpose, size_t bytes) {
             sl.ptr = nullptr;
             sl.bytes = 0;
         }
-        const size_t want = bytes + bytes / 4 + 4096;
+        const size_t want = bytes + std::min<size_t>(bytes / 4, (size_t)256 << 20) + 4096;
         sl.ptr = arena_alloc(want);
         sl.bytes = want;
     }

@@ -85,7 +85,8 @@ typedef struct hx_gemm_opts {   /* GemmOpts, CudaKernels.h:64-79 */
                                twelve waves, 6 = the residue route: N <= 12 int8 products modulo small
                                coprime moduli and a CRT recombination (N = 10 for p < 2^32, k <= 8192;
                                host-side sizes and k <= 133144 only, else the limb kernels; its workspace
-                               is hx_gemm_workspace_bytes_tile's, all of it: K is not chunked).  0 takes
+                               is hx_gemm_workspace_bytes_tile's, all of it: K is not chunked, nor C here;
+                               where 0 takes the route C runs in blocks of at most 8 GiB of planes).  0 takes
                                the residue route for large four-limb products (under HX_GEMM_AUTO for
                                every deep three- and four-limb product) when its workspace fits
                                (hx_gemm_route), else kernel 4 */

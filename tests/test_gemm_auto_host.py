@@ -49,3 +49,17 @@ def test_workspace_follows_the_route(limbs):
     (65521, 8192, 8192, 4096, 6), (2147483629, 8192, 8192, 1024, 6)])
 def test_residue_route_by_shape(p, m, n, k, route):
     assert E.gemm_route(E.ModCtx(p), m, n, k, E.HX_GEMM_AUTO) == route
+
+
+def test_residue_planes_are_bounded():
+    """The default and the automatic choice run C in blocks of at most 8 GiB of residue planes; a tile the caller
+    asks for keeps its one-piece formula."""
+    c = E.ModCtx(P[4])
+    for m, n, k in [(32768, 32768, 1024), (60000, 60000, 5000), (2000000, 2000, 800), (1100, 3000000, 1536), (100000, 100000, 133000)]:
+        for variant in (E.HX_GEMM_AUTO, E.HX_GEMM_LIMB):
+            if E.gemm_route(c, m, n, k, variant) == 6:
+                assert 0 < E.gemm_workspace_bytes(c, m, n, k, variant) <= 8 << 30, (m, n, k)
+        assert E.gemm_route(c, m, n, k, E.HX_GEMM_AUTO) == 6
+    assert E.gemm_workspace_bytes(c, 16384, 16384, 16384, E.HX_GEMM_AUTO) == 10 * 3 * 16384 * 16384
+    N = E.residue_moduli(c.p, 1024)
+    assert E.gemm_workspace_bytes(c, 32768, 32768, 1024, E.HX_GEMM_LIMB, tile=6) == N * (2 * 32768 * 1024 + 32768 * 32768)

@@ -75,3 +75,24 @@ def test_auto_deep_products_of_few_tiles(hx_gpu, p, m, n, k):
         E.gemm(ctx, A, B, C, op)
         E.gemm(ctx, A, B, D, op, variant=E.HX_GEMM_PLAIN, splits=1)
         assert torch.equal(C, D), op
+
+
+def test_residue_blocks_of_c(hx_gpu):
+    """Planes past 8 GiB: C in blocks (ragged at both edges), the stream's scratch bounded, the limb kernel's bytes."""
+    from hacs_amd import engine as E
+    p, m, n, k = 2147483629, 31001, 29999, 801
+    ctx = E.ModCtx(p)
+    assert E.gemm_route(ctx, m, n, k, E.HX_GEMM_AUTO) == 6
+    assert E.residue_moduli(p, k) * (m * n + (m + n) * k) > 8 << 30
+    A, B = _draw(p, m, k, 1, "col"), _draw(p, k, n, 2, "row")
+    s = torch.cuda.Stream()
+    g = torch.Generator(device="cuda").manual_seed(3)
+    C = torch.randint(0, p, (m, n), generator=g, device="cuda", dtype=torch.int32)
+    D = C.clone()
+    torch.cuda.synchronize()
+    live = E.arena_stats()["live_bytes"]
+    E.gemm(ctx, A, B, C, E.GemmOp.Sub, stream=s.cuda_stream)
+    assert E.arena_stats()["live_bytes"] - live <= (8 << 30) + (260 << 20)
+    s.synchronize()
+    E.gemm(ctx, A, B, D, E.GemmOp.Sub, variant=E.HX_GEMM_LIMB, tile=4)
+    assert torch.equal(C, D)
