@@ -310,6 +310,8 @@ bool packed_gemm(uint32_t m, uint32_t n, uint32_t k, const uint64_t* A, uint32_t
     const bool small = up(m, 256) / 256 * (up(n, 256) / 256) < 256;
     const uint64_t tile = small ? 128 : 256, Mp = up(m, tile), Np = up(n, tile);
     if (Mp > 0xffffffffu || Np > 0xffffffffu) return false;
+    // pg_kernel's grid: a launch holds fewer than 2^32 threads (C of 69 GB and more runs on the tables)
+    if ((Mp / tile) * (Np / tile) * 512 >= (uint64_t)1 << 32) return false;
     const uint64_t fit = PG_WS / (Mp + Np) * 2 / 128 * 128;                     // k whose planes fit PG_WS
     if (fit == 0) return false;
     const uint32_t chunk = (uint32_t)std::min<uint64_t>({up(k, 128), fit, PG_KMAX});

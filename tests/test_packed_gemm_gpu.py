@@ -76,3 +76,16 @@ def test_packed_gemm_captured(hx_gpu, p):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(C, _words(p, _product(p, a, b)))
+
+
+def test_packed_gemm_past_the_grid_limit(hx_gpu):
+    """An F_2 product of 2^23 tiles of 256 x 256 (69 GB of C): one launch cannot hold its threads, the table
+    kernel runs it."""
+    from hacs_amd import engine as E
+    m, n, k = 1 << 20, 1 << 19, 50
+    a, b = _entries(2, m, k, 1), _entries(2, k, n, 2)
+    A, B = _words(2, a), _words(2, b)
+    C = torch.zeros((m, n // 64), dtype=torch.int64, device="cuda")
+    E.f2_gemm(A, B, C, k, n)
+    for i0 in (0, 300000, m - 128):
+        assert torch.equal(C[i0:i0 + 128], _words(2, _product(2, a[i0:i0 + 128], b)))
