@@ -17,8 +17,9 @@
 // eight 32-cycle MFMAs and wave).  8192^3 over F_3: 0.263 ms for the call (the expansion of both operands
 // included, 4.2 P multiply-adds/s) against 5.51 ms on subset-sum tables in LDS; 4096^3 51 us against 2.76 ms
 // (F_2: 44 us against 0.98 ms); 64^3 15.5 us against 24 us, 4096 x 4096 x 128 over F_2 14 us against 33 us:
-// it is the faster one at every size measured, so the tables remain only for captures, where this route's
-// planes (library scratch that a later call may move) must not be recorded in a graph.
+// it is the faster one at every size measured but long F_2 operands of one word of k, so the tables remain for those
+// and for captures, where this route's planes (library scratch that a later call may move) must not be recorded
+// in a graph.
 #include "hx_packed_gemm.h"
 
 #include <algorithm>
@@ -310,6 +311,10 @@ bool packed_gemm(uint32_t m, uint32_t n, uint32_t k, const uint64_t* A, uint32_t
     const bool small = up(m, 256) / 256 * (up(n, 256) / 256) < 256;
     const uint64_t tile = small ? 128 : 256, Mp = up(m, tile), Np = up(n, tile);
     if (Mp > 0xffffffffu || Np > 0xffffffffu) return false;
+    // One word of A over F_2 and long operands: the tables take one pass, the planes pad k to 128 (us, tables / here:
+    // 1000000 x 64 x 64 69 / 84, 1000 x 300000 x 64 93 / 105; 100000 x 64 x 64 18 / 17, 20000^2 x 64 128 / 121, 1000000 x 64 x 200
+    // 257 / 107; over F_3 201 / 135 for the first).
+    if (P == 2 && k <= 64 && Mp + Np > 200000) return false;
     // pg_kernel's grid: a launch holds fewer than 2^32 threads (C of 69 GB and more runs on the tables)
     if ((Mp / tile) * (Np / tile) * 512 >= (uint64_t)1 << 32) return false;
     const uint64_t fit = PG_WS / (Mp + Np) * 2 / 128 * 128;                     // k whose planes fit PG_WS

@@ -37,7 +37,8 @@ def _product(p, a, b):
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (127, 65, 127), (128, 128, 128), (129, 129, 129), (130, 700, 385),
                                    (257, 383, 641), (200, 64, 1000),
                                    (4096, 4096, 200), (4100, 3841, 897),      # 256 x 256 tiles
-                                   (100, 64, 4194304 + 77)])                  # more than one K chunk
+                                   (100, 64, 4194304 + 77),                   # more than one K chunk
+                                   (199800, 70, 64), (199900, 70, 64), (60, 210000, 33)])   # one word of k, long operands
 def test_packed_gemm_edges(hx_gpu, p, m, n, k):
     from hacs_amd import engine as E
     mul = E.f2_gemm if p == 2 else E.f3_gemm
@@ -82,7 +83,7 @@ def test_packed_gemm_past_the_grid_limit(hx_gpu):
     """An F_2 product of 2^23 tiles of 256 x 256 (69 GB of C): one launch cannot hold its threads, the table
     kernel runs it."""
     from hacs_amd import engine as E
-    m, n, k = 1 << 20, 1 << 19, 50
+    m, n, k = 1 << 20, 1 << 19, 70
     a, b = _entries(2, m, k, 1), _entries(2, k, n, 2)
     A, B = _words(2, a), _words(2, b)
     C = torch.zeros((m, n // 64), dtype=torch.int64, device="cuda")
