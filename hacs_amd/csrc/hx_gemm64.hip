@@ -2,7 +2,7 @@
 // u64 GEMM of Cuda/cuda_kernels.cu:104-164; the CPU path of record is kernels::gemm<uint64_t>,
 // ModArithmetic/Kernels.h:184).  Two routes with the same bytes:
 //
-//  * The residue route (gemm64_residue; k >= 40, outside a stream capture): the operands modulo up to 19
+//  * The residue route (gemm64_residue; k >= 96, or k >= 40 with small planes; outside a stream capture): the operands modulo up to 19
 //    pairwise coprime bytes, one int8 MFMA product per modulus (res_gemm_kernel, hx_gemm.hip), and the CRT
 //    back to 64 bits.  2048^3 mod 2^61 - 1: 17 products, 0.256 ms = 3.4e13 multiply-adds/s for the whole
 //    call, against 4.19 ms (2.05e12) on the plain kernel; 512^3 0.049 against 0.364 ms.  Bound by the int8
@@ -322,7 +322,10 @@ uint32_t moduli64(uint64_t p, uint32_t k) {
 // Shallower products stay on the plain kernel: the splits and the CRT cost the same at any k, the plain kernel's
 // time grows with k (mod 2^61 - 1, us plain / residue: 2048 x 2048 x 16 59 / 109, x 64 180 / 122; 32^3 27 / 33,
 // 64^3 56 / 32; 512^3 364 / 49, 2048^3 4190 / 256).
-constexpr uint32_t RES64_MIN_K = 40;
+constexpr uint32_t RES64_MIN_K = 40, RES64_ANY_K = 96;
+// Between them only where the planes are small beside the plain kernel's rounds of 256 tiles (bytes <= 350000 k a
+// round; mod 2^61 - 1, us plain / residue, k = 40 and 64: 34 x 4096 39 / 40 and 51 / 41 at 13 MB; 1000 x 1000 45 / 50 and
+// 54 / 50 at 20 MB; 1 x 8192 37 / 51 and 47 / 52 at 25 MB; 10 x 20000 56 / 91 and 72 / 91 at 66 MB, x 128 141 / 100).
 constexpr size_t RES64_WS = (size_t)4 << 30;      // bytes of planes held at a time; C runs in blocks that fit
 
 // C op= A B by the residue route; false, with nothing launched, where it does not apply.
@@ -336,6 +339,8 @@ bool gemm64_residue(const hx_modctx64& ctx, const Gemm64Args& g, hipStream_t s) 
     const uint64_t Kp0 = up(kc, 64);
     uint64_t mb = up(g.m, side), nb = up(g.n, side);
     auto bytes = [&] { return N * (mb * Kp0 + nb * Kp0 + mb * nb); };
+    const uint64_t tiles = (uint64_t)((g.m + G64_TILE - 1) / G64_TILE) * ((g.n + G64_TILE - 1) / G64_TILE);
+    if (g.k < RES64_ANY_K && (double)bytes() > 350e3 * g.k * std::max(1.0, (double)tiles / 256)) return false;
     while (bytes() > RES64_WS && (mb > side || nb > side)) (mb >= nb ? mb : nb) = up((mb >= nb ? mb : nb) / 2, side);
     ScratchLease planes;                         // held until every block is launched
     try {

@@ -317,8 +317,8 @@ typedef struct hx_modctx64 {    /* ModCtx<uint64_t>'s device-relevant constants 
 } hx_modctx64;
 HX_API int hx_modctx64_init(uint64_t p, hx_modctx64 *out);
 /* C op= A * B mod p; views of 8-byte words (strides in elements), operands canonical (< p); k < 2^32.
- * Exact: int8 matrix products modulo up to 19 coprime bytes and the CRT (k >= 40, outside a capture; uses the
- * stream's own scratch), else 160-bit sums, one reduction per output. */
+ * Exact: int8 matrix products modulo up to 19 coprime bytes and the CRT (k >= 96, or k >= 40 where its planes are
+ * small; outside a capture; uses the stream's own scratch), else 160-bit sums, one reduction per output. */
 HX_API int hx_gemm_u64(const hx_modctx64 *ctx, hx_view A, hx_view B, hx_view C, int op, hx_stream s);
 
 /* ---- batched GEMM of uneven shapes (generalises GemmBatch<Elt>, CudaKernels.h:135-185, whose

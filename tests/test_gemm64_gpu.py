@@ -69,7 +69,8 @@ def test_gemm_u64_worst_case_carries(hx_gpu, O, p):
 
 @pytest.mark.parametrize("p", [2305843009213693951, 18446744073709551557, (1 << 64) - 2, 4294967311])
 @pytest.mark.parametrize("shape", [(128, 128, 64), (129, 127, 65), (255, 300, 129), (1, 700, 1000), (700, 1, 1000),
-                                   (1400, 1500, 70)])                              # the last: 256 x 256 tiles
+                                   (1400, 1500, 70),                               # 256 x 256 tiles
+                                   (10, 20001, 64), (10, 20001, 96), (34, 4097, 64), (1001, 999, 40)])   # either side of the rule below k = 96
 def test_gemm_u64_residue_route(hx_gpu, O, p, shape):
     """The matrix-core route at the edges of its tiles, row- and column-major operands, every op."""
     from hacs_amd import engine as E
