@@ -1,6 +1,7 @@
 """Products of small depth and small products (hx_thin.hip, the automatic choice) against the plain kernel: the
 edges of its 32-row blocks, 128-column workgroups and 32 / 64-deep k-steps, every limb count, the largest
-balanced entries (so the anti-diagonals reach their bounds), orders, strides and ops."""
+balanced entries, the largest digits (test_thin_largest_digits: the anti-diagonals at their bounds), orders, strides
+and ops."""
 import pytest
 import torch
 
@@ -39,6 +40,7 @@ def _check(E, ctx, A, B, C, what):
 def test_thin_shapes(hx_gpu, p, m, n, k):
     from hacs_amd import engine as E
     ctx = E.ModCtx(p)
+    assert (E.gemm_route(ctx, m, n, k, E.HX_GEMM_AUTO) == 7) == (k <= 256)       # (past it: the limb kernel)
     for extreme in (False, True):
         A, B = _draw(p, m, k, 1, extreme=extreme), _draw(p, k, n, 2, extreme=extreme)
         if extreme:
@@ -52,4 +54,43 @@ def test_thin_shapes(hx_gpu, p, m, n, k):
 @pytest.mark.parametrize("p,m,n,k", [(2147483629, 150, 301, 30), (65521, 301, 150, 64), (1000003, 61, 75, 200)])
 def test_thin_forms(hx_gpu, p, m, n, k, fa, fb, fc):
     from hacs_amd import engine as E
+    assert E.gemm_route(E.ModCtx(p), m, n, k, E.HX_GEMM_AUTO) == 7
     _check(E, E.ModCtx(p), _draw(p, m, k, 1, fa), _draw(p, k, n, 2, fb), lambda: _draw(p, m, n, 3, fc), (fa, fb, fc))
+
+
+def _digits(v, p):
+    """The balanced base-256 digits of the residue v."""
+    v, out = v - p if v > (p - 1) // 2 else v, []
+    for _ in range(4):
+        d = (v + 128) % 256 - 128
+        out.append(d)
+        v = (v - d) // 256
+    assert v == 0
+    return out
+
+
+@pytest.mark.parametrize("k", [31, 32, 63, 64, 200])
+@pytest.mark.parametrize("p,pos,neg", [
+    (2147483647, 0x3F7F7F7F, 0x3F808080),        # digits 127, 127, 127, 63 and -128, -128, -128, -63
+    (2147483629, 0x3F7F7F7F, 0x3F808080),
+    (16777259, 0x7F7F7F, 0x7E8080),              # four limbs at their smallest modulus
+    (16711423, 0x7F7F7F, 0x7E8080), (65279, 0x7F7F, 0x7E80), (251, 125, 125)])
+def test_thin_largest_digits(hx_gpu, p, pos, neg, k):
+    """Every digit at the end of its range, all products of one anti-diagonal with one sign: the sums and the
+    pairs of sums of the kernel (and of the eliminations' updates, the same reduction) at their bounds."""
+    from hacs_amd import engine as E
+    ctx, m, n = E.ModCtx(p), 40, 70
+    assert E.gemm_route(ctx, m, n, k, E.HX_GEMM_AUTO) == 7
+    vals = (pos, p - neg)
+    if p > 251:                              # (the digits that the modulus leaves free)
+        assert set(_digits(vals[0], p)[:ctx.c.limbs - 1]) == {127}
+        assert set(_digits(vals[1], p)[:min(2, ctx.c.limbs - 1)]) == {-128}
+    for x in vals:
+        for y in vals:
+            A = torch.full((m, k), x, dtype=torch.int64, device="cuda").to(torch.int32)
+            B = torch.full((k, n), y, dtype=torch.int64, device="cuda").to(torch.int32)
+            C = torch.zeros((m, n), dtype=torch.int32, device="cuda")
+            E.gemm(ctx, A, B, C)
+            assert (C == k * x * y % p).all(), (x, y)
+            E.gemm(ctx, A, B, C, E.GemmOp.Sub)
+            assert (C == 0).all(), (x, y)
