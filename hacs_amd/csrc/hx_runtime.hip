@@ -138,7 +138,10 @@ std::unordered_map<ScratchKey, std::shared_ptr<ScratchSlot>, ScratchKeyHash> g_s
 
 int current_device() {
     int dev = 0;
-    HX_HIP(hipGetDevice(&dev));
+    if (hipGetDevice(&dev) != hipSuccess) {      // no device: the allocation below reports it
+        (void)hipGetLastError();
+        dev = 0;
+    }
     return dev;
 }
 
