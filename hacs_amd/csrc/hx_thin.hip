@@ -193,10 +193,11 @@ void gemm_thin(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s) {
     t.ntn = (g.n + TH_N - 1) / TH_N;
     const uint32_t rblocks = (g.m + 31) / 32;
     // as many row blocks per workgroup (one split of B) as leave two workgroups per compute unit
-    // (4095 x 4033 x 32: 8 blocks 34 us, 4 blocks 37, 2 blocks 43, 1 block 52).  Reading C at k <= 32, where the loads of C
-    // decide, only waves with columns count: 100000 x 16 x 32 40 us with one block, 49 with six (plain kernel 38);
-    // x 100 the same 54; at k = 64 or without the read the longer walk is at least as fast (mod 65521 18 us / 20).
-    const uint64_t waves = g.op != HX_OP_SET && g.k <= 32 ? (g.n + 31) / 32 : 4 * (uint64_t)t.ntn;
+    // (4095 x 4033 x 32: 8 blocks 34 us, 4 blocks 37, 2 blocks 43, 1 block 52; 7 blocks, 608 workgroups, 20 us more where C
+    // is read).  Of one workgroup across, reading C at k <= 32 where the loads of C decide, only the waves with
+    // columns count: 100000 x 16 x 32 40 us with one block, 49 with six (plain kernel 38); at k = 64 or without the
+    // read the longer walk is at least as fast (mod 65521 18 us / 20).
+    const uint64_t waves = t.ntn == 1 && g.op != HX_OP_SET && g.k <= 32 ? (g.n + 31) / 32 : 4 * (uint64_t)t.ntn;
     t.nb = g.k > 64 ? 1 : (uint32_t)std::clamp<uint64_t>(rblocks * waves / 2048, 1, 8);
     const uint32_t blocks = t.ntn * ((rblocks + t.nb - 1) / t.nb);
     switch (ctx.limbs) {
