@@ -1915,14 +1915,17 @@ struct GemmRoute {
 constexpr int kThinRoute = 7;
 
 // The whole choice, for the dispatch and the public queries alike.  lists: rows or columns are gathered; splits as
-// in gemm_dispatch.  planes_ok: a caller workspace, or the library's scratch outside a capture.  Without it an
+// in gemm_dispatch.  ask_planes: a caller workspace, or the library's scratch outside a capture.  Without it an
 // automatic product takes no route that adds planes: a graph would keep the address of a buffer that a later,
 // larger call on the stream replaces.
+template <class F>
 GemmRoute gemm_route(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile, bool host_sizes,
-                     bool lists, uint32_t splits, bool planes_ok) {
+                     bool lists, uint32_t splits, F&& ask_planes) {
     const bool automatic = variant == HX_GEMM_AUTO;
+    bool planes_ok = true;
     if (automatic) {
         if (host_sizes && !lists && splits <= 1 && thin_applies(ctx, m, n, k)) return {kThinRoute, 0};
+        planes_ok = ask_planes();
         variant = gemm_auto_variant(ctx, m, n, k);
         if (host_sizes) {
             if (splits != 1 && auto_splits(ctx, m, n, k, !planes_ok || splits > 1)) return {0, 0};
@@ -1941,8 +1944,8 @@ void gemm_dispatch(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, int v
     const bool automatic = variant == HX_GEMM_AUTO;
     const bool host_sizes = g.m_dev == nullptr && g.k_dev == nullptr;
     const bool lists = g.a_rows != nullptr || g.a_cols != nullptr || g.c_rows != nullptr;
-    const bool planes_ok = !automatic || ws != nullptr || stream_scratch_safe(s);
-    const GemmRoute rt = gemm_route(ctx, g.m, g.n, g.k, variant, tile, host_sizes, lists, splits, planes_ok);
+    const GemmRoute rt = gemm_route(ctx, g.m, g.n, g.k, variant, tile, host_sizes, lists, splits,
+                                    [&] { return ws != nullptr || stream_scratch_safe(s); });
     if (rt.kernel == kThinRoute) {
         if (ev0) HX_HIP(hipEventRecord(ev0, s));
         gemm_thin(ctx, g, s);
@@ -2327,7 +2330,7 @@ extern "C" {
 HX_API size_t hx_gemm_workspace_bytes_tile(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant,
                                            int tile) {
     if (ctx == nullptr) return 0;
-    const GemmRoute rt = gemm_route(*ctx, m, n, k, variant, tile, true, false, 0, true);
+    const GemmRoute rt = gemm_route(*ctx, m, n, k, variant, tile, true, false, 0, [] { return true; });
     if (rt.kernel == 0 || rt.kernel == kThinRoute) return 0;
     return rt.moduli ? residue_plan(m, n, k, rt.moduli, tile == kResidueTile).bytes : limb_workspace_bytes(*ctx, m, n, k);
 }
@@ -2339,7 +2342,7 @@ HX_API size_t hx_gemm_workspace_bytes(const hx_modctx* ctx, uint32_t m, uint32_t
 HX_API uint32_t hx_gemm_residue_moduli(uint32_t p, uint32_t k) { return p >= 2 ? residue_moduli(p, k) : 0; }
 
 HX_API int hx_gemm_route(const hx_modctx* ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile) {
-    return ctx == nullptr ? -1 : gemm_route(*ctx, m, n, k, variant, tile, true, false, 0, true).kernel;
+    return ctx == nullptr ? -1 : gemm_route(*ctx, m, n, k, variant, tile, true, false, 0, [] { return true; }).kernel;
 }
 
 HX_API int hx_gemm_u32(const hx_modctx* ctx, hx_view A, hx_view B, hx_view C, int op, hx_stream s,
