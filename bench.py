@@ -580,7 +580,7 @@ def lu_c2(E, reps=3, cpu=True):
     g = C.c_void_p()
     with torch.cuda.stream(s):
         h = s.cuda_stream
-        E.rref_device(ctx, A, R2, d_out, ws, stream=h)          # eager once (creates the side streams)
+        E.rref_device(ctx, A, R2, d_out, ws, stream=h)          # eager once
         s.synchronize()
         _lib.check(L.hx_graph_begin(h))
         E.rref_device(ctx, A, R2, d_out, ws, stream=h)

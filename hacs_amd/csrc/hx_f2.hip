@@ -552,10 +552,6 @@ __global__ void f2_init_kernel(uint8_t* done, uint32_t m, F2State* st) {
 
 using namespace hx;
 
-extern "C" {
-
-}  // extern "C"
-
 namespace {
 size_t f2_ws_bytes(uint32_t m, uint32_t n, uint32_t ldw) {
     const size_t mn = std::min(m, n);

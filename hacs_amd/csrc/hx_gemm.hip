@@ -1899,8 +1899,7 @@ void gemm_residue(const hx_modctx& ctx, const GemmArgs& g, hipStream_t s, uint32
 
 // The automatic choice: the limb route once the product is big enough to pay for the two
 // operand splits, and deep enough (k >= 64, one full LDS stage) for the MFMA work to outweigh the
-// recombination epilogue; thinner products (the k = 32 Schur updates of the eliminations) run
-// faster on the plain kernel.
+// recombination epilogue.  gemm_route refines it (thin products, small deep ones, the residue route).
 int gemm_auto_variant(const hx_modctx& ctx, uint32_t m, uint32_t n, uint32_t k) {
     if (ctx.limbs == 0 || k < 64) return HX_GEMM_PLAIN;
     const double work = (double)m * n * k;

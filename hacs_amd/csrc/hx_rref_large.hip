@@ -14,7 +14,7 @@
 //     levels (by the last workgroup to finish): groups of 16 candidate lists, the rule re-run on
 //     their raw rows (two threads per row); the last level writes the panel's pivot rows P (pivot
 //     order), columns J and count k.  Before all that, every workgroup runs the rule on the first
-//     64 rows alone, which settles most panels without the tournament (see rrp_pivot_kernel).
+//     64 rows alone, which settles most panels without the tournament (see pivot_block).
 //  2. X = S[P, J]^{-1} S[P, :]: every workgroup owns a slab of 16 columns and performs the same
 //     row reduction on [S[P, J] | S[P, slab]] (division-free Gauss-Jordan, one barrier per pivot,
 //     then one inverse per pivot) -- or, when the search over the first rows settled the panel,
@@ -40,8 +40,6 @@
 #include <algorithm>
 #include <chrono>
 #include <cstdio>
-#include <mutex>
-#include <unordered_map>
 #include <vector>
 
 #include "hx_elim.h"
@@ -775,8 +773,8 @@ __global__ __launch_bounds__(PXT) void panel_x_kernel(const uint32_t* S, int64_t
     }
 }
 
-// The trailing update of a panel may still run (second stream) while the next panel's
-// tournament rewrites k / m_new: it reads its own copy.
+// Past the last panel: its pivots join the rank.  (Every other panel's are added by the next pivot search; the
+// products beside that search read the sizes of their own panel from the snap_ copies.)
 __global__ void advance_kernel(LState* st) {
     if (threadIdx.x == 0) {
         st->r += st->k;

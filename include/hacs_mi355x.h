@@ -243,10 +243,13 @@ HX_API size_t hx_gemm_workspace_bytes_tile(const hx_modctx *ctx, uint32_t m, uin
 HX_API uint32_t hx_gemm_residue_moduli(uint32_t p, uint32_t k);
 /* The kernel a product with host-side sizes runs for (variant, tile), given a large enough workspace: 0 = the
  * plain kernel, 1 .. 5 = that limb kernel, 6 = the residue route, 7 = the thin kernel (limbs split on the fly, AUTO
- * only: k <= 64, and k <= 256 for small products); -1 for a NULL ctx.  LIMB's default (tile 0) takes the residue
- * route where it needs at most limbs^2 - 4 int8 products and m, n, k >= 4096, else limb kernel 4; AUTO takes it
- * for three and four limbs at depths of 1536 and more (768 for large four-limb products; not between 64 and 256 tiles
- * of 64 x 128, where the limb kernel is the faster one).  No counterpart in the reference. */
+ * only: p < 2^31 with limbs, m n >= 256 and k <= 64, or k <= 256 below 4e6 multiply-adds); -1 for a NULL ctx.  LIMB's
+ * default (tile 0) takes the residue route where it needs at most limbs^2 - 4 int8 products and m, n, k >= 4096, else
+ * limb kernel 4.  AUTO also takes it for moduli of four (three) limbs from 256 tiles of 64 x 128 and k = 768 (1536) on
+ * where its measured costs are the lower ones (long narrow products stay on the limb kernel), and up to 64
+ * tiles from k = 1536 (2560) on with m + n <= 2560; AUTO splits products of fewer than 32 tiles over K on the plain
+ * kernel past k = 8192 (12288 below 4e6 multiply-adds, there not with one limb).  Inside a stream capture without
+ * opts->workspace AUTO keeps to kernels without new library planes.  No counterpart in the reference. */
 HX_API int hx_gemm_route(const hx_modctx *ctx, uint32_t m, uint32_t n, uint32_t k, int variant, int tile);
 /* The K chunk a limb workspace of workspace_bytes runs (imma_k_chunk, CudaKernels.h:100-110): min(k, the
  * int32-exact chunk) when its planes fit, else the largest multiple of 64 that fits; 0 when not even a

@@ -117,7 +117,7 @@ def test_rref_device_entry_captured_and_replayed(hx_gpu, O):
     L = _lib.lib()
     with torch.cuda.stream(s):
         h = s.cuda_stream
-        E.rref_device(ctx, dA, R, out, ws, stream=h)          # eager once (creates the side stream)
+        E.rref_device(ctx, dA, R, out, ws, stream=h)          # eager once
         s.synchronize()
         res = E.rref_device_result(out, m, n)
         assert res.rank == want[0]
