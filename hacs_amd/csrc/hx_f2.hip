@@ -27,8 +27,8 @@
 //    previous panel, the rest tables, candidates and the store; then 4 us f2_copy_kernel.
 //  * f2_finish: the pivot rows in pivot order to the top, zero rows below (the non-pivot rows are
 //    zero after the last panel: every row is reduced against every pivot).
-//  * The product runs on the matrix cores (hx_packed_gemm.hip).  Inside a stream capture, or when that
-//    route's planes do not fit: f2_gemm_kernel, the same tables over B's rows, 64 at a time, accumulating
+//  * The product runs on the matrix cores (hx_packed_gemm.hip).  Where that route does not
+//    apply (hx_packed_gemm.h): f2_gemm_kernel, the same tables over B's rows, 64 at a time, accumulating
 //    the output words in registers (one lookup per byte of A's word).
 #include <algorithm>
 #include <cstring>

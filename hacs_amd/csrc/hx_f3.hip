@@ -21,8 +21,8 @@
 //    lookups: per group of 4 slots an LDS table of the 81 combinations of those rows with coefficients
 //    in F_3 (for the workgroup's 4 words, both planes), one lookup per group.
 //  * f3_gather / f3_place: the pivot rows in pivot order to the top, zero rows below.
-//  * The product runs on the matrix cores (hx_packed_gemm.hip).  Inside a stream capture, or when that
-//    route's planes do not fit: f3_gemm_kernel, the same tables over B's rows, 64 at a time (one word pair
+//  * The product runs on the matrix cores (hx_packed_gemm.hip).  Where that route does not
+//    apply (hx_packed_gemm.h): f3_gemm_kernel, the same tables over B's rows, 64 at a time (one word pair
 //    of A).
 //
 // F_3 arithmetic on 64 entries at once (x = (x1, x2) one-hot, z = x + y): z1 is set where (x, y) is
