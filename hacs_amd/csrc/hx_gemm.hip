@@ -1715,10 +1715,10 @@ uint32_t residue_side(uint32_t m, uint32_t n, uint32_t N) {
 // reads N planes where the limb kernel has L, and pads to larger tiles, which a long narrow operand pays for most
 // (mod 2147483629, us limb / residue: 34 x 40000 x 2000 313 / 530, 129 x 20000 x 2000 213 / 294, 20000 x 34 x 3000 306 / 380,
 // 300 x 7000 x 4096 254 / 305, 384 x 20000 x 2048 342 / 409; 512 x 4200 x 2048 136 / 109, 20000 x 256 x 4096 530 / 490).  From
-// sides of 1100 on it always does at these depths, or costs a few per cent.
+// sides of 1450 on it does at these depths, or costs a few per cent.
 bool residue_pays(uint32_t limbs, uint32_t N, uint32_t m, uint32_t n, uint32_t k) {
     const uint32_t narrow = std::min(m, n);
-    if (narrow >= 1100) return true;
+    if (narrow >= 1450) return true;
     auto cd = [](uint64_t a, uint64_t b) { return (double)((a + b - 1) / b); };
     const double K = 1e-3 * k, M = 1e-3 * m, Nn = 1e-3 * n;
     const uint64_t lt = (uint64_t)((m + LM - 1) / LM) * ((n + LN - 1) / LN);
@@ -1728,7 +1728,7 @@ bool residue_pays(uint32_t limbs, uint32_t N, uint32_t m, uint32_t n, uint32_t k
     const uint64_t rt = (uint64_t)N * ((m + side - 1) / side) * ((n + side - 1) / side);
     const double round = side == RTM ? 5.84 : 2.52, tile = (side == RTM ? 6.85 : 1.49) / 256;
     const double res = 17.5 + K * (round * cd(rt, 256) + tile * (double)rt) + K * N * (0.35 * M + 0.424 * Nn) + 0.678 * N * M * Nn;
-    return res < (narrow < 256 ? 0.88 : 0.97) * limb;        // (in doubt the limb kernel)
+    return res < (narrow < 256 ? 0.88 : 1.0) * limb;         // (the narrowest: in doubt the limb kernel)
 }
 
 // The moduli count of the residue route when this product takes it, else 0.  It needs host-side sizes,
