@@ -96,3 +96,5 @@ def test_residue_blocks_of_c(hx_gpu):
     s.synchronize()
     E.gemm(ctx, A, B, D, E.GemmOp.Sub, variant=E.HX_GEMM_LIMB, tile=4)
     assert torch.equal(C, D)
+    del A, B, C, D
+    torch.cuda.empty_cache()

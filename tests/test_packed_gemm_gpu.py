@@ -90,3 +90,5 @@ def test_packed_gemm_past_the_grid_limit(hx_gpu):
     E.f2_gemm(A, B, C, k, n)
     for i0 in (0, 300000, m - 128):
         assert torch.equal(C[i0:i0 + 128], _words(2, _product(2, a[i0:i0 + 128], b)))
+    del a, b, A, B, C
+    torch.cuda.empty_cache()
